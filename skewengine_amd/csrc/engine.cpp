@@ -66,6 +66,7 @@ struct DevPlanBuf {
         v.fl = fl.p;
         v.maxL = ip.maxL;
         v.maxH = ip.maxH;
+        v.maxI = ip.maxI;
         return v;
     }
 };
@@ -496,7 +497,6 @@ struct Core {
                 break;
             case SKE_KERNEL_RADON:
                 if (local) {
-                    SKE_TRY(launch("fill", [&] { return launch_fill_f64(W.p, (size_t)ip.so_total, stream); }));
                     SKE_TRY(launch("op_lrt", [&] {
                         return launch_lrt(v, in4.p, nullptr, W.p, arena.p, ctab.p, gtab.p, stream);
                     }));
@@ -829,7 +829,6 @@ int sector_kernel(ske_engine* e) {
     case SKE_KERNEL_RADON: {
         if (c.radon_local) {
             SKE_TRY(e->W1.ensure(2 * (size_t)e->N + e->dim_l));
-            SKE_TRY(c.launch("fill", [&] { return launch_fill_f64(e->W1.p, (size_t)sp.H * sp.dim_i, c.stream); }));
             SKE_TRY(c.launch("op_lrt", [&] {
                 return launch_lrt(v, c.in4.p, e->S.p, e->W1.p, e->SO.p, c.ctab.p, c.gtab.p, c.stream);
             }));

@@ -316,100 +316,208 @@ hipError_t launch_radn_smear(const DevPlan& p, const float* q, float* SO, hipStr
 //   Y = FFT64(y)/8,  out = |Y_{m-1}|^2 at the first m in [5, 32) with
 //   |Y_m|^2 > |Y_{m-1}|^2 (0 if none; getParameter :96-108).
 // Here in two passes:
-//   lrt_rowsum: one workgroup per skewed row; the row is staged in LDS and
-//     every column's 65-wide window sum is formed in double in the
-//     reference's order (ascending l), for all dim_i columns -> W.
-//   op_lrt: one wave per skewed row, lanes over its cells.  Each cell reads
-//     its 64 window sums down column j of W (coalesced across the lanes),
-//     and evaluates the 26 needed real parts of X and then |Y_m|^2 for
-//     m = 4, 5, ... directly as cosine/sine sums (FP64), stopping at the
-//     first rise.  The direct sums differ from the reference's radix-2 FFT
-//     only by FP64 rounding.
+//   lrt_rowsum: one wave per skewed row forms every column's 65-wide window
+//     sum in double -> W, all rows and columns of the sector.
+//   op_lrt: a workgroup stages the 95 rows of window sums that a tile of 64
+//     columns x 32 rows reaches in LDS; each cell then takes its 64 window
+//     sums from there and evaluates the 26 needed real parts of X and
+//     |Y_m|^2 for m = 4, 5, ... as cosine/sine sums (FP64), stopping at the
+//     first rise.  The sums differ from the reference's radix-2 FFT only by
+//     FP64 rounding.
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(128) void k_lrt_rowsum(const SecDesc* __restrict__ secs, const RowWork* __restrict__ work,
-                                                    const float* __restrict__ in4, const int* __restrict__ target,
-                                                    const float* __restrict__ weight, const uint32_t* __restrict__ fl,
-                                                    const float* __restrict__ Sbuf, double* __restrict__ W) {
-    extern __shared__ float lds[];
-    float* row = lds + kPad;
-    const RowWork w = work[blockIdx.x];
-    const SecDesc sd = secs[w.sec];
-    const uint32_t v = fl[sd.rows + w.row];
-    const int f = fl_first(v);
-    const int L = fl_last(v) - f;
-    if (L <= 0) return;
-    stage_row(row, sd, w.row, f, L, in4, target, weight, Sbuf);
-    __syncthreads();
-    double* out = W + sd.so + (size_t)w.row * sd.dim_i;
-    for (int j = threadIdx.x; j < sd.dim_i; j += blockDim.x) {
-        const int lo = max(j - 32, f) - f, hi = min(j + 32, f + L - 1) - f;
-        double acc = 0.0;
-        for (int l = lo; l <= hi; ++l) acc += (double)row[l];
-        out[j] = acc;
+// Blocks of a launch over all sectors of a plan: blockIdx.x the block within
+// the sector, the sector split over y and z (a grid's y and z end at 65535).
+constexpr int kSecY = 32768;
+inline dim3 sector_grid(unsigned per_sector, int nsec) {
+    return dim3(per_sector, (unsigned)(nsec < kSecY ? nsec : kSecY), (unsigned)((nsec + kSecY - 1) / kSecY));
+}
+__device__ __forceinline__ int sector_index() { return (int)(blockIdx.z * kSecY + blockIdx.y); }
+
+// Inclusive sums over the 64 lanes, from lane 0 up (kUp) or from lane 63
+// down: four DPP steps inside the rows of 16 lanes, then the totals of the
+// rows before (after) this lane's, read as scalars.  Additions only, so a run
+// of zeros stays exactly zero.
+template <int kCtrl>
+__device__ __forceinline__ double dpp_add(double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kCtrl, 0xf, 0xf, false);
+    return x + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <bool kUp>
+__device__ __forceinline__ double wave_scan(double x, int lane) {
+    constexpr int kShift = kUp ? 0x110 : 0x100;  // row_shr / row_shl
+    x = dpp_add<kShift + 1>(x);
+    x = dpp_add<kShift + 2>(x);
+    x = dpp_add<kShift + 4>(x);
+    x = dpp_add<kShift + 8>(x);
+    const int row = kUp ? lane >> 4 : 3 - (lane >> 4);  // rows already passed
+    const double t0 = lane_value(x, kUp ? 15 : 48), t1 = lane_value(x, kUp ? 31 : 32),
+                 t2 = lane_value(x, kUp ? 47 : 16);
+    const double t01 = t0 + t1, t012 = t01 + t2;
+    return x + (row == 0 ? 0.0 : row == 1 ? t0 : row == 2 ? t01 : t012);
+}
+
+// Window sums W(r, j) = sum_{l=j-32}^{j+32} S(r, l) [first <= l < last].  With
+// the row cut in blocks of 64 cells, the window of column 64 t - 32 + s is the
+// tail of block t - 1 from its cell s and the head of block t up to its cell
+// s, so two scans of a block's 64 cells serve 64 windows.  65 additions a cell and a
+// zero fill before: 482 + 66 us for the 180 sectors of a 512^2 slice; now 206
+// us, of which the 543 MB it writes take 112.  Every column of every row of the
+// sector is written, rows without cells as zeros.
+__global__ __launch_bounds__(256) void k_lrt_rowsum(const SecDesc* __restrict__ secs, int nsec,
+                                                    const float* __restrict__ in4,
+                                                    const int* __restrict__ target, const float* __restrict__ weight,
+                                                    const uint32_t* __restrict__ fl, const float* __restrict__ Sbuf,
+                                                    double* __restrict__ W) {
+    const int si = sector_index();
+    if (si >= nsec) return;
+    const SecDesc& sd = secs[si];
+    const int r = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (r >= sd.H) return;  // wave-uniform
+    const int lane = threadIdx.x & 63;
+    const uint32_t v = fl[sd.rows + r];
+    const int f = fl_first(v), l = fl_last(v);
+    const int dim_i = sd.dim_i, dim_o = sd.dim_o;
+    const float* src = in4 + sd.img + (size_t)sd.type * sd.N;
+    const int* tt = target + sd.tab;
+    const float* ww = weight + sd.tab;
+    double* out = W + sd.so + (size_t)r * dim_i;
+    auto cell = [&](int j) -> float {
+        if (j < f || j >= l) return 0.0f;
+        return Sbuf ? Sbuf[(size_t)r * dim_i + j] : skew_cell_sel(src, tt[j], ww[j], r, j, dim_i, dim_o);
+    };
+    double tail = 0.0;
+    float next = cell(lane);
+    for (int c = 0; c - 32 < dim_i; c += 64) {
+        const double x = (double)next;
+        next = cell(c + 64 + lane);
+        const bool some = c < l && c + 64 > f;  // uniform
+        const double head = some ? wave_scan<true>(x, lane) : 0.0;
+        const int j = c - 32 + lane;
+        if (j >= 0 && j < dim_i) out[j] = tail + head;
+        tail = some ? wave_scan<false>(x, lane) : 0.0;
     }
 }
 
-// tab: the sine ramp sin(f/24.6 * pi/2) for f <= 25 at [160,186), the two
-// DFT matrices at kLrtC and kLrtY (ske_types.h); gauss: 64 weights per folded
-// angle (newAngle).
-__global__ __launch_bounds__(64) void k_op_lrt(const SecDesc* __restrict__ secs, const RowWork* __restrict__ work,
-                                               const uint32_t* __restrict__ fl, const double* __restrict__ W,
-                                               const double* __restrict__ tab, const double* __restrict__ gauss,
-                                               float* __restrict__ arena) {
-    const RowWork w = work[blockIdx.x];
-    const SecDesc sd = secs[w.sec];
-    const int i = w.row;
-    const uint32_t v = fl[sd.rows + i];
-    const int f = fl_first(v), l = fl_last(v);
-    const double* g = gauss + 64 * sd.newAngle;
+// The transform.  x_kk (times 1/8) is folded before the first cosine sum:
+// cos(pi q kk/32) is even about kk = 32 and even or odd about 16 and 8 with
+// the parity of q and q/2, so the 64 samples fall into nine groups ("orbits"
+// k = 0..8 of kk -> 64 - kk, 32 - kk, 16 - kk) of which q = 0, 4, .. needs 9,
+// q = 2, 6, .. 8 and odd q 16 values: 319 products instead of 64 x 26.  The
+// coefficients (with the sine ramp and both factors 1/8, exact powers of two,
+// already in them) come in wave-uniform rows: scalar loads.
+// A cell whose 26 values are all zero (no image in its windows) is 0 by the
+// peak rule and leaves the search for the first rise at once; otherwise 97% of
+// cells stop at m <= 9.
+// Bound by FP64 VALU issue: 64 columns x 32 rows a workgroup, a wave per row
+// at a time, five window-sum reads of 8 B per cell from memory and 64 from LDS
+// (conflict-free).  512^2, 180 sectors: 5.28 -> 1.42 ms.
+constexpr int kLrtRows = 32, kLrtWin = kLrtRows + 63;
+__global__ __launch_bounds__(512) void k_op_lrt(const SecDesc* __restrict__ secs, int nsec, int coltiles,
+                                                const uint32_t* __restrict__ fl, const double* __restrict__ W,
+                                                const double* __restrict__ tab, const double* __restrict__ gauss,
+                                                float* __restrict__ arena) {
+    __shared__ double win[kLrtWin * 64];
+    const int si = sector_index();
+    if (si >= nsec) return;  // uniform
+    const SecDesc& sd = secs[si];
+    const int H = sd.H, dim_i = sd.dim_i;
+    const int rt = (int)blockIdx.x / coltiles;
+    const int i0 = rt * kLrtRows, j0 = ((int)blockIdx.x - rt * coltiles) * 64;
+    if (i0 >= H || j0 >= dim_i) return;  // uniform
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    {   // leave when no row of the tile has a cell in these columns (every wave finds the same)
+        bool some = false;
+        if (lane < kLrtRows && i0 + lane < H) {
+            const uint32_t v = fl[sd.rows + i0 + lane];
+            some = fl_first(v) < j0 + 64 && fl_last(v) > j0 && fl_first(v) < fl_last(v);
+        }
+        if (__builtin_amdgcn_ballot_w64(some) == 0) return;
+    }
     const double* Wb = W + sd.so;
-    const int k0 = max(0, 32 - i), k1 = min(64, sd.H - i + 32);  // kk with 0 <= i-32+kk < H
-    for (int j = f + (int)threadIdx.x; j < l; j += 64) {
-        double re1[26];
+    const int j = j0 + lane;
+    for (int y = wave; y < kLrtWin; y += 8) {
+        const int k = i0 - 32 + y;
+        win[y * 64 + lane] = (k >= 0 && k < H && j < dim_i) ? Wb[(size_t)k * dim_i + j] : 0.0;
+    }
+    __syncthreads();
+    const double* g = gauss + 64 * sd.newAngle;
+    for (int y = wave; y < kLrtRows; y += 8) {
+        const int i = i0 + y;
+        if (i >= H) break;  // uniform
+        const uint32_t v = fl[sd.rows + i];
+        const bool in = j >= fl_first(v) && j < fl_last(v);
+        if (__builtin_amdgcn_ballot_w64(in) == 0) continue;
+        const double* w = win + y * 64 + lane;  // sample kk at w[64 kk]
+        double re[26];  // q = 0, 4, .., 24; q = 2, 6, .., 22; q = 1, 3, .., 25
+        {
+            const double u0 = g[0] * w[0], u32 = g[32] * w[64 * 32], u16 = g[16] * (w[64 * 16] + w[64 * 48]);
+            const double v0 = u0 + u32, e = v0 + u16, o = v0 - u16, d = u0 - u32;
+            const double* C = tab + kLrtC;
 #pragma unroll
-        for (int q = 0; q < 26; ++q) re1[q] = 0.0;
-        int kk = k0;
-        // four window sums in flight per pass; re1 still accumulates in kk order
-        for (; kk + 4 <= k1; kk += 4) {
-            double xs[4];
+            for (int q = 0; q < 7; ++q) re[q] = e * C[q];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) xs[u] = Wb[(size_t)(i - 32 + kk + u) * sd.dim_i + j];
+            for (int q = 0; q < 6; ++q) re[7 + q] = o * C[7 + q];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double x = xs[u] * g[kk + u];
-                const double* C = tab + kLrtC + 32 * (kk + u);  // wave-uniform row: scalar loads
-#pragma unroll
-                for (int q = 0; q < 26; ++q) re1[q] = __builtin_fma(x, C[q], re1[q]);
-            }
+            for (int q = 0; q < 13; ++q) re[13 + q] = d * C[13 + q];
         }
-        for (; kk < k1; ++kk) {
-            const double x = Wb[(size_t)(i - 32 + kk) * sd.dim_i + j] * g[kk];
-            const double* C = tab + kLrtC + 32 * kk;
+        {
+            const double u8 = g[8] * (w[64 * 8] + w[64 * 56]), u24 = g[24] * (w[64 * 24] + w[64 * 40]);
+            const double e = u8 + u24, d = u8 - u24;
+            const double* C = tab + kLrtC + 40 * 8;
 #pragma unroll
-            for (int q = 0; q < 26; ++q) re1[q] = __builtin_fma(x, C[q], re1[q]);
+            for (int q = 0; q < 7; ++q) re[q] = __builtin_fma(e, C[q], re[q]);
+#pragma unroll
+            for (int q = 0; q < 13; ++q) re[13 + q] = __builtin_fma(d, C[13 + q], re[13 + q]);
         }
+#pragma unroll 1
+        for (int k = 1; k < 8; ++k) {
+            const double* wp = w + 64 * k;
+            const double* wm = w - 64 * k;
+            const double ua = g[k] * (wp[0] + wm[64 * 64]), ub = g[16 - k] * (wm[64 * 16] + wp[64 * 48]);
+            const double uc = g[16 + k] * (wp[64 * 16] + wm[64 * 48]), ud = g[32 - k] * (wm[64 * 32] + wp[64 * 32]);
+            const double va = ua + ud, vb = ub + uc;
+            const double e = va + vb, o = va - vb, da = ua - ud, db = ub - uc;
+            const double* C = tab + kLrtC + 40 * k;
 #pragma unroll
-        for (int q = 0; q < 26; ++q) re1[q] *= 0.125 * tab[160 + q];
+            for (int q = 0; q < 7; ++q) re[q] = __builtin_fma(e, C[q], re[q]);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) re[7 + q] = __builtin_fma(o, C[7 + q], re[7 + q]);
+#pragma unroll
+            for (int q = 0; q < 13; ++q)
+                re[13 + q] = __builtin_fma(db, C[26 + q], __builtin_fma(da, C[13 + q], re[13 + q]));
+        }
+        uint32_t some = 0;
+#pragma unroll
+        for (int q = 0; q < 26; ++q) some |= (uint32_t)(__builtin_bit_cast(uint64_t, re[q]) >> 32);
+        bool search = in && (some << 1) != 0;
         double prev = 0.0, val = 0.0;
-        for (int m = 4; m < 32; ++m) {
-            double yr = 0.0, yi = 0.0;
-            const double* Y = tab + kLrtY + 64 * m;
+        for (int m = 4; m < 32 && __builtin_amdgcn_ballot_w64(search) != 0; ++m) {
+            const double* Y = tab + kLrtY + 64 * m;  // the 26 cosines, then the sines, in the order of re
+            double yr[2] = {0.0, 0.0}, yi[2] = {0.0, 0.0};
 #pragma unroll
             for (int q = 0; q < 26; ++q) {
-                yr = __builtin_fma(re1[q], Y[2 * q], yr);
-                yi = __builtin_fma(re1[q], Y[2 * q + 1], yi);
+                yr[q & 1] = __builtin_fma(re[q], Y[2 * q], yr[q & 1]);
+                yi[q & 1] = __builtin_fma(re[q], Y[2 * q + 1], yi[q & 1]);
             }
-            yr *= 0.125;
-            yi *= 0.125;
-            const double cur = yr * yr + yi * yi;
-            if (m > 4 && cur > prev) {
+            const double r = yr[0] + yr[1], s = yi[0] + yi[1];
+            const double cur = r * r + s * s;
+            if (m > 4 && search && cur > prev) {
                 val = prev;
-                break;
+                search = false;
             }
             prev = cur;
         }
-        arena[sd.so + (size_t)i * sd.dim_i + j] = (float)val;
+        if (in) arena[sd.so + (size_t)i * dim_i + j] = (float)val;
     }
 }
 
@@ -469,11 +577,12 @@ hipError_t launch_lrt_samples(const DevPlan& p, const SampleReq* req, int nreq, 
 
 hipError_t launch_lrt(const DevPlan& p, const float* in4, const float* Sbuf, double* W, float* arena,
                       const double* tab, const double* gauss, hipStream_t s) {
-    if (p.nwork == 0) return hipSuccess;
-    const size_t lds = sizeof(float) * (size_t)(p.maxL + 2 * kPad);
-    hipLaunchKernelGGL(k_lrt_rowsum, dim3(p.nwork), dim3(128), lds, s, p.secs, p.work, in4, p.target, p.weight, p.fl,
-                       Sbuf, W);
-    hipLaunchKernelGGL(k_op_lrt, dim3(p.nwork), dim3(64), 0, s, p.secs, p.work, p.fl, W, tab, gauss, arena);
+    if (p.nsec == 0 || p.maxH <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_lrt_rowsum, sector_grid((unsigned)(p.maxH + 3) / 4, p.nsec), dim3(256), 0, s, p.secs, p.nsec,
+                       in4, p.target, p.weight, p.fl, Sbuf, W);
+    const unsigned ct = (unsigned)(p.maxI + 63) / 64, rt = (unsigned)(p.maxH + kLrtRows - 1) / kLrtRows;
+    hipLaunchKernelGGL(k_op_lrt, sector_grid(ct * rt, p.nsec), dim3(512), 0, s, p.secs, p.nsec, (int)ct, p.fl, W, tab,
+                       gauss, arena);
     return hipGetLastError();
 }
 

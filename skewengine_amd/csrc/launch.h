@@ -18,6 +18,7 @@ struct DevPlan {
     const uint32_t* fl = nullptr;  // first | last << 16 per row
     int maxL = 0;                   // longest valid row (LDS sizing)
     int maxH = 0;                   // tallest skewed block (rows per sector)
+    int maxI = 0;                   // longest skewed row (columns per sector)
 };
 
 enum DeskewSource { kDeskewDense = 0, kDeskewArena = 1, kDeskewRadon = 2 };
@@ -66,8 +67,8 @@ hipError_t launch_radn_filter(const DevPlan& p, const double* P, float* q, const
                               const int* tw_off, int maxH2, hipStream_t s);
 
 // Local Radon transform (LRT=true): window sums of every skewed row into W
-// (doubles at the arena offsets of the rows, zero-filled beforehand by the
-// caller), then the per-cell transform into the arena.  tab as for the
+// (doubles at the arena offsets of the rows, every column of every row of the
+// planned sectors), then the per-cell transform into the arena.  tab as for the
 // blur operator plus the sine ramp at [160,186); gauss: 64 weights per
 // folded angle 0..90.
 hipError_t launch_lrt(const DevPlan& p, const float* in4, const float* Sbuf, double* W, float* arena,

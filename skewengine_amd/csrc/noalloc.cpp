@@ -259,6 +259,7 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
         v.fl = reinterpret_cast<const uint32_t*>(base + ch.fl);
         v.maxL = ch.ip.maxL;
         v.maxH = ch.ip.maxH;
+        v.maxI = ch.ip.maxI;
         switch (kernel_id) {
         case SKE_KERNEL_SDEM: {
             // the engine's default launch shape (two waves for short rows)
@@ -274,7 +275,6 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
             break;
         case SKE_KERNEL_RADON:
             if (local) {
-                SKE_HIP(launch_fill_f64(W, (size_t)ch.ip.so_total, stream));
                 SKE_HIP(launch_lrt(v, in4, nullptr, W, arena, ctab, gtab, stream));
             } else {
                 SKE_HIP(launch_radn_rowsum(v, in4, nullptr, P, stream));

@@ -141,6 +141,7 @@ void plan_append(int dimx, int dimy, int s0, int s1, long long img, ImagePlan& i
             }
         }
         ip.maxH = std::max(ip.maxH, sp.H);
+        ip.maxI = std::max(ip.maxI, sp.dim_i);
         so += (long long)sp.H * sp.dim_i;
         q += sp.H;
         if (!seen[sp.type]) {
@@ -204,7 +205,7 @@ void fft_twiddles(int mmax, std::vector<double>& tw, std::vector<int>& off) {
 }
 
 void cepstrum_table(std::vector<double>& tab) {
-    static_assert(kLrtC >= kLogTab + 2 * 256 + 2, "table layout");
+    static_assert(kLrtC >= kLogTab + 2 * 256 + 2 && kLrtC % 2 == 0 && kLrtY % 2 == 0, "table layout");
     tab.assign(kCtabSize, 0.0);
     for (int t = 0; t < 64; t++) {
         tab[2 * t] = cos(2.0 * M_PI * t / 64.0);
@@ -224,15 +225,22 @@ void cepstrum_table(std::vector<double>& tab) {
     const long double ln2 = logl(2.0L);
     tab[kLogTab + 512] = (double)ln2;
     tab[kLogTab + 513] = (double)(ln2 - (long double)(double)ln2);
-    // the local Radon's two DFT matrices, rows contiguous (copies of the
-    // cos/sin entries above; frequencies q >= 26 stay 0)
-    for (int kk = 0; kk < 64; kk++)
-        for (int q = 0; q < 26; q++) tab[kLrtC + 32 * kk + q] = tab[2 * ((q * kk) & 63)];
+    // the local Radon's two DFT matrices (ske_types.h), from the cos/sin entries above; the frequencies in
+    // the order of the folded sums
+    int qs[26];
+    for (int i = 0; i < 7; i++) qs[i] = 4 * i;
+    for (int i = 0; i < 6; i++) qs[7 + i] = 4 * i + 2;
+    for (int i = 0; i < 13; i++) qs[13 + i] = 2 * i + 1;
+    for (int k = 0; k <= 8; k++) {
+        double* C = tab.data() + kLrtC + 40 * k;
+        for (int i = 0; i < 26; i++) C[i] = tab[2 * ((qs[i] * k) & 63)] * tab[160 + qs[i]] / 64;
+        for (int i = 0; i < 13; i++) C[26 + i] = tab[2 * ((qs[13 + i] * (16 - k)) & 63)] * tab[160 + qs[13 + i]] / 64;
+    }
     for (int m = 0; m < 32; m++)
-        for (int q = 0; q < 26; q++) {
-            const int t = (q * m) & 63;
-            tab[kLrtY + 64 * m + 2 * q] = tab[2 * t];
-            tab[kLrtY + 64 * m + 2 * q + 1] = tab[2 * t + 1];
+        for (int i = 0; i < 26; i++) {
+            const int t = (qs[i] * m) & 63;
+            tab[kLrtY + 64 * m + 2 * i] = tab[2 * t];
+            tab[kLrtY + 64 * m + 2 * i + 1] = tab[2 * t + 1];
         }
     // the cepstrum's 64-sample window DFT (bins k < 32), rows contiguous
     for (int m = 0; m < 64; m++)

@@ -37,6 +37,7 @@ struct ImagePlan {
     std::vector<RowWork> work;  // rows with at least one valid cell
     int maxL = 0;
     int maxH = 0;
+    int maxI = 0;               // longest skewed row (dim_i)
     long long so_total = 0;     // arena floats (sum of H*dim_i)
     long long q_total = 0;      // sum of H
     int range[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // per-type [begin, end) into secs

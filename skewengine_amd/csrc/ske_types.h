@@ -11,8 +11,12 @@ namespace ske {
 constexpr int kMaxDim = 16000;
 constexpr int kPad = 64;        // LDS guard band on each side of a staged row
 constexpr int kLogTab = 192;    // offset of the log table in the cepstrum constants (planner.cpp)
-constexpr int kLrtC = 720;      // local Radon first DFT: cos(2 pi (q kk mod 64)/64) at [kLrtC + 32 kk + q]
-constexpr int kLrtY = kLrtC + 2048;  // second DFT: cos, sin of 2 pi (q m mod 64)/64 at [kLrtY + 64 m + 2 q (+1)]
+// local Radon first DFT, folded: for the orbit k = 0..8 of the samples (kernels_radn.hip) 40 doubles at [kLrtC + 40 k]:
+// cos(pi q k/32) for q = 0, 4, .., 24, for q = 2, 6, .., 22, for q = 1, 3, .., 25, then cos(pi q (16 - k)/32) for
+// q = 1, 3, .., 25, each times sin(q/24.6 pi/2) / 64
+constexpr int kLrtC = 720;
+// second DFT: cos, sin of 2 pi (q m mod 64)/64 at [kLrtY + 64 m + 2 i (+1)], q the i-th of 0, 4, .., 24, 2, 6, .., 22, 1, 3, .., 25
+constexpr int kLrtY = kLrtC + 360;
 constexpr int kBlurD = kLrtY + 2048;  // cepstrum window DFT: cos, sin of 2 pi (k m mod 64)/64 at [kBlurD + 64 m + 2 k (+1)]
 constexpr int kCtabSize = kBlurD + 4096;
 constexpr int kNumSectors = 180; // maxSector, src/global.cpp:69
