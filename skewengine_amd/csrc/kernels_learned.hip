@@ -654,138 +654,251 @@ __global__ __launch_bounds__(64 * FwdSplit<C>::kWaves, C == 16 ? 5 : 2) void k_c
 // layer input they flow into
 // ---------------------------------------------------------------------------
 
-// dA3[q][ci] = sum_t W4[t][ci] * dout[q - off(t)], times (a3 > 0).
+// The two single-channel layers' backward kernels: activation and weight
+// gradients of one layer in one pass over its largest tensor, all contractions
+// on v_mfma_f32_16x16x4_f32 (fp32 products and sums; lane layout: A[i][k] at
+// lane i + 16k, B[k][j] at lane j + 16k, D[i][j] at lane j + 16(i/4), register
+// i%4).  As many workgroups as the card holds at once (a second, part-filled
+// round doubled the time) walk the 16 x 16 tiles of all slices, the next tile's
+// loads in flight, and add their weight sums into grad[] once.  Both are bound
+// by memory: 402 MB (out) and 285 MB (in) at 16 x 512^2, C = 16.  Each was two
+// kernels, the weight sums on the VALU with two LDS reads a product: out 106 +
+// 310 -> 131 us, in 271 + 310 -> 140 us.
+
+// out[p] = r0[p] + b4 + sum_t W4[t] . a3[p + off(t)]:
+//   dz3[q][ci]  = (a3[q][ci] > 0) sum_t W4[t][ci] dout[q - off(t)]   A = W4^T (K = 9 of 12), B = shifted dout
+//   dW4[t][ci] += sum_q dout[q - off(t)] a3[q][ci],  db4 += sum dout     A = shifted dout, B = a3 (K = pixels)
 template <int C>
 __global__ __launch_bounds__(256) void k_conv_out_bwd(const float* __restrict__ dout, const uint16_t* __restrict__ a3,
-                                                      const float* __restrict__ prm, float* __restrict__ dz3, int n) {
-    __shared__ float w[9 * C];
-    __shared__ float ds[(T + 2) * (T + 2)];
-    const int b = blockIdx.z;
-    const int i0 = blockIdx.y * T, j0 = blockIdx.x * T;
-    for (int t = threadIdx.x; t < 9 * C; t += 256) w[t] = rbf(prm[learned_layout(C).W4 + t]);
-    const float* db = dout + (size_t)b * n * n;
-    for (int t = threadIdx.x; t < (T + 2) * (T + 2); t += 256) {
-        const int ii = i0 + t / (T + 2) - 1, jj = j0 + t % (T + 2) - 1;
-        ds[t] = (ii >= 0 && ii < n && jj >= 0 && jj < n) ? db[(size_t)ii * n + jj] : 0.0f;
-    }
-    __syncthreads();
-    const int ty = threadIdx.x / T, tx = threadIdx.x % T;
-    const size_t p = ((size_t)b * n + i0 + ty) * n + j0 + tx;
-    float g[9];
+                                                      const float* __restrict__ prm, float* __restrict__ dz3,
+                                                      float* __restrict__ grad, int n, int batch) {
+    constexpr LearnedLayout L = learned_layout(C);
+    constexpr int H = C / 16, kW = T + 2;
+    __shared__ float ds[kW * kW];
+    __shared__ __align__(16) uint16_t xa[T * T * C];
+    __shared__ float red[4 * H * 256];
+    const int side = n / T, tiles = side * side, items = tiles * batch;
+    const int lane = threadIdx.x & 63, j16 = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float w[H][3];  // W4[tap 4s + kb][channel 16h + j16]
 #pragma unroll
-    for (int t = 0; t < 9; t++) g[t] = ds[(ty + 2 - t / 3) * (T + 2) + tx + 2 - t % 3];  // dout[q - off(t)]
-    for (int ci = 0; ci < C; ci++) {
-        float s = 0.0f;
+    for (int h = 0; h < H; h++)
 #pragma unroll
-        for (int t = 0; t < 9; t++) s = __builtin_fmaf(w[t * C + ci], g[t], s);
-        dz3[p * C + ci] = bf2f(a3[p * C + ci]) > 0.0f ? s : 0.0f;
-    }
-}
-
-// 16 x 8 pixel tiles for the single-channel layers' backward kernels.
-constexpr int TY = 8;
-// dr0[q] = dout[q] + sum_{t,co} W1[co][t] * dZ1[q - off(t)][co].
-template <int C>
-__global__ __launch_bounds__(128) void k_conv_in_bwd(const float* __restrict__ dz1, const float* __restrict__ dout,
-                                                     const float* __restrict__ prm, float* __restrict__ dr0, int n) {
-    __shared__ float w[C * 9];
-    __shared__ float ds[(TY + 2) * (T + 2) * (C + 1)];  // pixel pitch C+1: distinct banks per lane
-    const int b = blockIdx.z;
-    const int i0 = blockIdx.y * TY, j0 = blockIdx.x * T;
-    for (int t = threadIdx.x; t < C * 9; t += 128) w[t] = rbf(prm[learned_layout(C).W1 + t]);
-    const float* db = dz1 + (size_t)b * n * n * C;
-    for (int t = threadIdx.x; t < (TY + 2) * (T + 2) * C; t += 128) {
-        const int pix = t / C, c = t % C;
-        const int ii = i0 + pix / (T + 2) - 1, jj = j0 + pix % (T + 2) - 1;
-        ds[pix * (C + 1) + c] = (ii >= 0 && ii < n && jj >= 0 && jj < n) ? db[((size_t)ii * n + jj) * C + c] : 0.0f;
-    }
-    __syncthreads();
-    const int ty = threadIdx.x / T, tx = threadIdx.x % T;
-    float s = 0.0f;
-    for (int tap = 0; tap < 9; tap++) {
-        const float* gp = ds + ((ty + 2 - tap / 3) * (T + 2) + tx + 2 - tap % 3) * (C + 1);
-#pragma unroll
-        for (int co = 0; co < C; co++) s = __builtin_fmaf(w[co * 9 + tap], gp[co], s);
-    }
-    const size_t p = ((size_t)b * n + i0 + ty) * n + j0 + tx;
-    dr0[p] = dout[p] + s;
-}
-
-// ---------------------------------------------------------------------------
-// backward: weight gradients, tile partial sums added into grad[] with atomics
-// ---------------------------------------------------------------------------
-
-// dW[co][t][ci] += sum_p dZ[p][co] * X[p + off(t)][ci]; db[co] += sum_p dZ[p][co].
-// X: bf16 NHWC (xc channels) or fp32 single channel (xc == 1, xf != null).
-// dZ: fp32 NHWC with zc channels.  16 x 8 pixel tiles; a workgroup sums its
-// tile over the slices b = blockIdx.z, blockIdx.z + gridDim.z, ... in
-// registers and adds the partial sums into grad[] with atomics once.
-template <int C>
-__global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dz, int zc, const uint16_t* __restrict__ xh,
-                                               const float* __restrict__ xf, int xc, float* __restrict__ grad, int woff,
-                                               int boff, int wlayout_tc, int n, int batch) {
-    extern __shared__ float sm[];
-    float* zs = sm;                        // TY*T*zc
-    float* xs = sm + TY * T * zc;          // (TY+2)(T+2)*xc
-    const int i0 = blockIdx.y * TY, j0 = blockIdx.x * T;
-    constexpr int kWgPer = 9 * C * C / 256;  // weights per thread (largest layer)
-    const int nw = zc * 9 * xc;
-    float acc[kWgPer];
-#pragma unroll
-    for (int r = 0; r < kWgPer; r++) acc[r] = 0.0f;
-    float bacc = 0.0f;
-    for (int b = blockIdx.z; b < batch; b += gridDim.z) {
-        __syncthreads();
-        const float* zb = dz + (size_t)b * n * n * zc;
-        for (int t = threadIdx.x; t < TY * T * zc; t += 256) {
-            const int pix = t / zc, c = t % zc;
-            zs[t] = zb[((size_t)(i0 + pix / T) * n + j0 + pix % T) * zc + c];
+        for (int k = 0; k < 3; k++) {
+            const int t = 4 * k + kb;
+            w[h][k] = t < 9 ? rbf(prm[L.W4 + t * C + 16 * h + j16]) : 0.0f;
         }
-        for (int t = threadIdx.x; t < (TY + 2) * (T + 2) * xc; t += 256) {
-            const int pix = t / xc, c = t % xc;
-            const int ii = i0 + pix / (T + 2) - 1, jj = j0 + pix % (T + 2) - 1;
+    // dout[q - off(t)] of tile pixel (y, x) is ds[(y + 2 - t/3) kW + x + 2 - t%3]
+    const float* bt[3];  // B of the activation gradient: tap 4s + kb (clamped), pixel column j16
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int t = min(4 * k + kb, 8);
+        bt[k] = ds + (2 - t / 3) * kW + j16 + 2 - t % 3;
+    }
+    const int ta = min(j16, 8);
+    const float* at = ds + (2 - ta / 3) * kW + kb + 2 - ta % 3;  // A of the weight gradient: tap j16, pixel 4g + kb
+    f32x4 acc[H];
+#pragma unroll
+    for (int h = 0; h < H; h++) acc[h] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    float bsum = 0.0f;
+    // the next slice's tile is loaded into registers while this one's is worked on
+    constexpr int kDs = (kW * kW + 255) / 256, kXa = T * T * (C / 8) / 256;
+    float dnext[kDs];
+    uint4 xnext[kXa];
+    auto load = [&](int item) {
+        const int b = item / tiles, tile = item - b * tiles;
+        const int i0 = (tile / side) * T, j0 = (tile % side) * T;
+        const float* db = dout + (size_t)b * n * n;
+#pragma unroll
+        for (int e = 0; e < kDs; e++) {
+            const int t = threadIdx.x + 256 * e, ii = i0 + t / kW - 1, jj = j0 + t % kW - 1;
+            dnext[e] = (t < kW * kW && ii >= 0 && ii < n && jj >= 0 && jj < n) ? db[(size_t)ii * n + jj] : 0.0f;
+        }
+#pragma unroll
+        for (int e = 0; e < kXa; e++) {
+            const int t = threadIdx.x + 256 * e, px = t / (C / 8);
+            const size_t q = ((size_t)b * n + i0 + px / T) * n + j0 + px % T;
+            xnext[e] = *(const uint4*)(a3 + q * C + 8 * (t % (C / 8)));
+        }
+    };
+    load(blockIdx.x);
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int b = item / tiles, tile = item - b * tiles;
+        const int i0 = (tile / side) * T, j0 = (tile % side) * T;
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kDs; e++)
+            if ((int)threadIdx.x + 256 * e < kW * kW) ds[threadIdx.x + 256 * e] = dnext[e];
+#pragma unroll
+        for (int e = 0; e < kXa; e++) *(uint4*)(xa + 8 * (threadIdx.x + 256 * e)) = xnext[e];
+        __syncthreads();
+        if (item + (int)gridDim.x < items) load(item + gridDim.x);
+        bsum += ds[(threadIdx.x / T + 1) * kW + threadIdx.x % T + 1];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int y = 4 * wave + r;
+            float v[3];
+#pragma unroll
+            for (int k = 0; k < 3; k++) v[k] = bt[k][y * kW];
+#pragma unroll
+            for (int h = 0; h < H; h++) {
+                f32x4 d = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < 3; k++) d = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][k], v[k], d, 0, 0, 0);
+                // lane (j16, kb): channels 16h + 4kb .. +3 of pixel (y, j16)
+                const uint2 xv = *(const uint2*)(xa + (y * T + j16) * C + 16 * h + 4 * kb);
+                float4 o;
+                o.x = __uint_as_float(xv.x << 16) > 0.0f ? d[0] : 0.0f;
+                o.y = __uint_as_float(xv.x & 0xffff0000u) > 0.0f ? d[1] : 0.0f;
+                o.z = __uint_as_float(xv.y << 16) > 0.0f ? d[2] : 0.0f;
+                o.w = __uint_as_float(xv.y & 0xffff0000u) > 0.0f ? d[3] : 0.0f;
+                *(float4*)(dz3 + (((size_t)b * n + i0 + y) * n + j0 + j16) * C + 16 * h + 4 * kb) = o;
+            }
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const float a = at[y * kW + 4 * g];
+#pragma unroll
+                for (int h = 0; h < H; h++)
+                    acc[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        a, bf2f(xa[(y * T + 4 * g + kb) * C + 16 * h + j16]), acc[h], 0, 0, 0);
+            }
+        }
+    }
+    // lane (j16, kb) holds dW4[4kb + r][16h + j16]: the four waves' sums, then grad[]
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[(wave * H + h) * 256 + (4 * kb + r) * 16 + j16] = acc[h][r];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+        const int t = threadIdx.x / 16, c = threadIdx.x % 16;
+        float v = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) v += red[(q * H + h) * 256 + threadIdx.x];
+        if (t < 9) atomicAdd(grad + L.W4 + t * C + 16 * h + c, v);
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) bsum += __shfl_xor(bsum, o);
+    if (lane == 0) atomicAdd(grad + L.B4, bsum);
+}
+
+// a1 = relu(b1 + sum_t W1[.][t] r0[p + off(t)]), out = r0 + ...:
+//   dr0[q]      = dout[q] + sum_t P[t][q - off(t)],  P[t][p] = sum_co W1[co][t] dz1[p][co]   A = W1^T, B = dz1
+//   dW1[co][t] += sum_p dz1[p][co] r0[p + off(t)],   db1[co] += sum_p dz1[p][co]             A = dz1, B = shifted r0
+// P is formed for the tile and its one-pixel halo; the bias is a tenth column of ones in B.
+template <int C>
+__global__ __launch_bounds__(256) void k_conv_in_bwd(const float* __restrict__ dz1, const float* __restrict__ dout,
+                                                     const float* __restrict__ r0, const float* __restrict__ prm,
+                                                     float* __restrict__ dr0, float* __restrict__ grad, int n,
+                                                     int batch) {
+    constexpr LearnedLayout L = learned_layout(C);
+    constexpr int H = C / 16, kW = T + 2, kN = kW * kW;
+    constexpr int kPz = C + 4;  // pixel pitch (floats): 16 pixels x 4 channels of a B operand on distinct banks
+    __shared__ __align__(16) float zs[kN * kPz];
+    __shared__ float xs[kN];
+    __shared__ float P[9 * kN];
+    const int side = n / T, tiles = side * side, items = tiles * batch;
+    const int lane = threadIdx.x & 63, j16 = lane & 15, kb = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float w[C / 4];  // W1[channel 4s + kb][tap j16]
+#pragma unroll
+    for (int k = 0; k < C / 4; k++) w[k] = j16 < 9 ? rbf(prm[L.W1 + (4 * k + kb) * 9 + j16]) : 0.0f;
+    const int tb = min(j16, 8);
+    const float* xt = xs + (tb / 3) * kW + kb + tb % 3;  // r0[p + off(j16)] of tile pixel (y, 4g + kb): + y kW + 4g
+    const float xfix = j16 == 9 ? 1.0f : 0.0f;
+    f32x4 acc[H];
+#pragma unroll
+    for (int h = 0; h < H; h++) acc[h] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+    // the next slice's tile is loaded into registers while this one's is worked on
+    constexpr int kZ = (kN * (C / 4) + 255) / 256, kX = (kN + 255) / 256;
+    float4 znext[kZ];
+    float xnext[kX];
+    auto load = [&](int item) {
+        const int b = item / tiles, tile = item - b * tiles;
+        const int i0 = (tile / side) * T, j0 = (tile % side) * T;
+#pragma unroll
+        for (int e = 0; e < kZ; e++) {
+            const int t = threadIdx.x + 256 * e, px = t / (C / 4);
+            const int ii = i0 + px / kW - 1, jj = j0 + px % kW - 1;
+            znext[e] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (px < kN && ii >= 0 && ii < n && jj >= 0 && jj < n)
+                znext[e] = *(const float4*)(dz1 + (((size_t)b * n + ii) * n + jj) * C + 4 * (t % (C / 4)));
+        }
+#pragma unroll
+        for (int e = 0; e < kX; e++) {
+            const int t = threadIdx.x + 256 * e, ii = i0 + t / kW - 1, jj = j0 + t % kW - 1;
+            xnext[e] = (t < kN && ii >= 0 && ii < n && jj >= 0 && jj < n) ? rbf(r0[((size_t)b * n + ii) * n + jj]) : 0.0f;
+        }
+    };
+    load(blockIdx.x);
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int b = item / tiles, tile = item - b * tiles;
+        const int i0 = (tile / side) * T, j0 = (tile % side) * T;
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kZ; e++) {
+            const int t = threadIdx.x + 256 * e, px = t / (C / 4);
+            if (px < kN) *(float4*)(zs + px * kPz + 4 * (t % (C / 4))) = znext[e];
+        }
+#pragma unroll
+        for (int e = 0; e < kX; e++)
+            if ((int)threadIdx.x + 256 * e < kN) xs[threadIdx.x + 256 * e] = xnext[e];
+        __syncthreads();
+        if (item + (int)gridDim.x < items) load(item + gridDim.x);
+        for (int g = wave; g < (kN + 15) / 16; g += 4) {
+            const int px = min(16 * g + j16, kN - 1);
+            f32x4 d = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int k = 0; k < C / 4; k++)
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k], zs[px * kPz + 4 * k + kb], d, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (4 * kb + r < 9) P[(4 * kb + r) * kN + px] = d[r];
+        }
+        // weight gradient: tile rows 4 wave .. +3, four pixels at a time
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const int y = 4 * wave + r;
+                const float xv = xt[y * kW + 4 * g];
+                const float bv = j16 < 9 ? xv : xfix;
+#pragma unroll
+                for (int h = 0; h < H; h++)
+                    acc[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        zs[((y + 1) * kW + 4 * g + kb + 1) * kPz + 16 * h + j16], bv, acc[h], 0, 0, 0);
+            }
+        __syncthreads();
+        {
+            const int ty = threadIdx.x / T, tx = threadIdx.x % T;
+            const size_t q = ((size_t)b * n + i0 + ty) * n + j0 + tx;
             float v = 0.0f;
-            if (ii >= 0 && ii < n && jj >= 0 && jj < n) {
-                const size_t q = ((size_t)b * n + ii) * n + jj;
-                v = xf ? rbf(xf[q]) : bf2f(xh[q * xc + c]);
-            }
-            xs[t] = v;
-        }
-        __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kWgPer; r++) {
-            const int wi = threadIdx.x + 256 * r;
-            if (wi < nw) {
-                // weight index -> (co, tap, ci) in the layer's layout
-                int co, tap, ci;
-                if (wlayout_tc) {  // [t][ci] (zc == 1)
-                    co = 0;
-                    tap = wi / xc;
-                    ci = wi % xc;
-                } else {           // [co][t][ci]
-                    co = wi / (9 * xc);
-                    const int rm = wi % (9 * xc);
-                    tap = rm / xc;
-                    ci = rm % xc;
-                }
-                const int oy = tap / 3, ox = tap % 3;
-                float s = acc[r];
-                for (int py = 0; py < TY; py++)
-                    for (int px = 0; px < T; px++)
-                        s = __builtin_fmaf(zs[(py * T + px) * zc + co],
-                                           xs[((py + oy) * (T + 2) + px + ox) * xc + ci], s);
-                acc[r] = s;
-            }
+            for (int t = 0; t < 9; t++) v += P[t * kN + (ty + 2 - t / 3) * kW + tx + 2 - t % 3];
+            dr0[q] = dout[q] + v;
         }
-        if ((int)threadIdx.x < zc)
-            for (int pix = 0; pix < TY * T; pix++) bacc += zs[pix * zc + threadIdx.x];
     }
+    // lane (j16, kb) holds dW1[16h + 4kb + r][j16] (j16 < 9) and db1 (j16 == 9)
+    __syncthreads();
+    float* red = zs;  // 4 waves x H x 256 floats
+    static_assert(4 * H * 256 <= kN * kPz, "the reduction fits the tile buffer");
 #pragma unroll
-    for (int r = 0; r < kWgPer; r++) {
-        const int wi = threadIdx.x + 256 * r;
-        if (wi < nw) atomicAdd(grad + woff + wi, acc[r]);
+    for (int h = 0; h < H; h++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[(wave * H + h) * 256 + (4 * kb + r) * 16 + j16] = acc[h][r];
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+        const int co = 16 * h + threadIdx.x / 16, t = threadIdx.x % 16;
+        float v = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) v += red[(q * H + h) * 256 + threadIdx.x];
+        if (t < 9)
+            atomicAdd(grad + L.W1 + co * 9 + t, v);
+        else if (t == 9)
+            atomicAdd(grad + L.B1 + co, v);
     }
-    if ((int)threadIdx.x < zc) atomicAdd(grad + boff + threadIdx.x, bacc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1038,76 +1151,181 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(const float* __restrict__ dz
 // filter and back-projector gradients
 // ---------------------------------------------------------------------------
 
-// Adjoint of k_fbp_backproject as a gather: dq[a][k] = sum over the pixels
-// p with floor(kf_p) in {k - 1, k} of p's weight on bin k -- v - w v when
-// floor(kf_p) = k, w v when it is k - 1 (w = kf_p - floor(kf_p), v = scale *
-// dr[p]) -- with kf_p = (x c + y sn) / delta + det_c computed as the
-// back-projection computes it.  One thread per (slice, angle, bin).  It walks
-// the rows (the columns when |c| < |sn|) in ascending order; in each, kf is
-// linear along the row with slope c (sn) per pixel, so the pixels with kf in
-// [k - 1, k + 1) are a run of at most 2 / max(|c|, |sn|) + 1 <= 3.9 whose
-// ends follow from the row's kf at pixel 0; the run, widened by one pixel
-// each side, is tested pixel by pixel.  Fixed order, no atomics.
-// drT: dr transposed per slice, read on column walks so that a wave's
-// neighbouring bins read neighbouring addresses there too.
-__global__ __launch_bounds__(256) void k_bp_adjoint_gather(const float* __restrict__ dr,
-                                                           const float* __restrict__ drT, float* __restrict__ dq,
-                                                           const float2* __restrict__ cs, FbpGeom g, float scale) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x, a = blockIdx.y, b = blockIdx.z;
-    if (k >= g.ndet) return;
-    const float2 t2 = cs[a];
-    const float c = t2.x, sn = t2.y;
-    const float inv = 1.0f / g.delta;
-    const bool rows = fabsf(c) >= fabsf(sn);  // walk rows: kf varies along j with slope c
-    const float* const im = (rows ? dr : drT) + (size_t)b * g.n * g.n;  // line u at im + u n
-    const float slope = rows ? c : -sn;        // d kf / d (index along the walk), about
-    const float rsl = 1.0f / slope;
-    const int cnt = (int)(2.0f * fabsf(rsl)) + 3;  // candidates per line: the run, one more each side
-    float acc = 0.0f;
-    for (int u = 0; u < g.n; u++) {
-        // kf at index 0 of line u (row u: j = 0; column u: i = 0), approximate
-        const float fu = ((float)u + 0.5f) * g.delta;
-        const float kf0 = rows ? ((0.5f * g.delta - 1.0f) * c + (1.0f - fu) * sn) * inv + g.det_c
-                               : ((fu - 1.0f) * c + (1.0f - 0.5f * g.delta) * sn) * inv + g.det_c;
-        // indices t with kf0 + t slope in [k - 1, k + 1)
-        const float ta = ((float)k - 1.0f - kf0) * rsl, tb = ((float)k + 1.0f - kf0) * rsl;
-        const int t0 = (int)floorf(fminf(ta, tb)) - 1;
-        for (int q = 0; q < cnt; q++) {
-            const int t = t0 + q;
-            if (t < 0 || t >= g.n) continue;
-            const int i = rows ? u : t, j = rows ? t : u;
-            const float x = ((float)j + 0.5f) * g.delta - 1.0f, y = 1.0f - ((float)i + 0.5f) * g.delta;
-            const float kf = (x * c + y * sn) * inv + g.det_c;
-            const float fk = floorf(kf);
-            const int k0 = (int)fk;
-            if (k0 != k && k0 != k - 1) continue;
-            const float w = kf - fk;
-            const float v = im[(size_t)u * g.n + t] * scale;
-            acc += (k0 == k) ? v - w * v : w * v;
+// Adjoint of k_fbp_backproject as a gather: dq[a][k] = scale sum over the
+// pixels p of max(0, 1 - |kf_p - k|) dr[p], kf_p = (x c + y sn) / delta + det_c
+// (the lerp's weight of bin k).  One thread per (angle, bin) and four slices:
+// it walks the rows (the columns when |c| < |sn|); along a line kf is linear
+// with a slope of magnitude as >= 0.7, so the pixels within one bin of k are
+// at most three, from t = ceil(tc - 1/as), tc the position where kf = k, with
+// weights 1 - |t - tc| as.  Their positions and weights serve the four slices,
+// which k_adjoint_lines interleaves (float4 per pixel, four zero pixels at
+// each end of a line, so t needs one clamp and no test).  The lines are cut in
+// `nchunk` shares, one workgroup each, whose sums k_adjoint_sum adds in order.
+// Fixed order, no atomics.  16 x 512^2, 60 angles x 725 bins: one slice a
+// thread with five tested candidates a line took 1,129 us (VALU); now 118 +
+// 15 (lines) + 6 (sum), bound by the L1 reads of 48 B a line and thread.
+constexpr int kAdjPad = 4;
+__global__ __launch_bounds__(256) void k_adjoint_lines(const float* __restrict__ dr, float4* __restrict__ rows,
+                                                       float4* __restrict__ cols, int n, int batch) {
+    __shared__ float tile[4][32][33];
+    const int g = blockIdx.z, b0 = 4 * g;
+    const int x0 = (int)blockIdx.x * 32 - kAdjPad, y0 = (int)blockIdx.y * 32 - kAdjPad;  // tile corner, image coordinates
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+    const int pitch = n + 2 * kAdjPad;
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+        for (int k = ty; k < 32; k += 8) {
+            const int i = y0 + k, j = x0 + tx;
+            tile[s][k][tx] = (b0 + s < batch && i >= 0 && i < n && j >= 0 && j < n)
+                                 ? dr[((size_t)(b0 + s) * n + i) * n + j] : 0.0f;
         }
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+        const int i = y0 + k, j = x0 + tx;
+        if (i >= 0 && i < n && j < n + kAdjPad)
+            rows[((size_t)g * n + i) * pitch + j + kAdjPad] =
+                make_float4(tile[0][k][tx], tile[1][k][tx], tile[2][k][tx], tile[3][k][tx]);
+        const int jc = x0 + k, ic = y0 + tx;
+        if (jc >= 0 && jc < n && ic < n + kAdjPad)
+            cols[((size_t)g * n + jc) * pitch + ic + kAdjPad] =
+                make_float4(tile[0][tx][k], tile[1][tx][k], tile[2][tx][k], tile[3][tx][k]);
     }
-    dq[((size_t)b * g.nang + a) * g.ndet + k] = acc;
 }
 
-// dh[m + ndet - 1] += sum_k dq[row][k] * p[row][k - m] for every row.
-__global__ __launch_bounds__(256) void k_filter_grad(const float* __restrict__ dq, const float* __restrict__ p,
-                                                     float* __restrict__ dh, int ndet) {
+__global__ __launch_bounds__(256) void k_bp_adjoint(const float4* __restrict__ rows, const float4* __restrict__ cols,
+                                                    float* __restrict__ part, const float2* __restrict__ cs, FbpGeom g,
+                                                    float scale, int batch, int nchunk) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x, a = blockIdx.y;
+    const int grp = blockIdx.z / nchunk, ch = blockIdx.z - grp * nchunk;
+    const int n = g.n, pitch = n + 2 * kAdjPad;
+    const float2 t2 = cs[a];
+    const float c = t2.x, sn = t2.y;
+    const bool walk_rows = fabsf(c) >= fabsf(sn);
+    const float4* const im = (walk_rows ? rows : cols) + (size_t)grp * n * pitch + kAdjPad;
+    // kf of line u, position t: A + u B + t slope
+    const float m = 0.5f * (float)n - 0.5f;
+    const float slope = walk_rows ? c : -sn, B = walk_rows ? -sn : c;
+    const float A = g.det_c + m * (sn - c);
+    const float rsl = 1.0f / slope, as = fabsf(slope), half = fabsf(rsl);
+    const float tc0 = ((float)k - A) * rsl, dt = -B * rsl;
+    const int per = (n + nchunk - 1) / nchunk;
+    int u0 = ch * per, u1 = min(u0 + per, n);
+    {   // lines whose pixels a lane of this wave can reach: -2 < tc < n + 1 (two lines of margin)
+        float lo = (float)u0, hi = (float)u1;
+        if (fabsf(dt) > 1e-3f) {
+            const float ua = (-2.0f - tc0) / dt, ub = ((float)n + 1.0f - tc0) / dt;
+            lo = fmaxf(lo, floorf(fminf(ua, ub)) - 2.0f);
+            hi = fminf(hi, ceilf(fmaxf(ua, ub)) + 3.0f);
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            lo = fminf(lo, __shfl_xor(lo, off, 64));
+            hi = fmaxf(hi, __shfl_xor(hi, off, 64));
+        }
+        u0 = __builtin_amdgcn_readfirstlane((int)lo);
+        u1 = __builtin_amdgcn_readfirstlane((int)hi);
+    }
+    const float tmax = (float)n;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 2
+    for (int u = u0; u < u1; u++) {
+        const float tc = __builtin_fmaf((float)u, dt, tc0);
+        const float tf = ceilf(tc - half);
+        const float d = (tf - tc) * as;
+        const float w0 = fmaxf(1.0f - fabsf(d), 0.0f), w1 = fmaxf(1.0f - fabsf(d + as), 0.0f),
+                    w2 = fmaxf(1.0f - fabsf(__builtin_fmaf(2.0f, as, d)), 0.0f);
+        // clamped, the three pixels are padding
+        const int t = (int)__builtin_amdgcn_fmed3f(tf, -3.0f, tmax);
+        const float4* p = im + (size_t)u * pitch + t;
+        const float4 v0 = p[0], v1 = p[1], v2 = p[2];
+        acc[0] = __builtin_fmaf(w2, v2.x, __builtin_fmaf(w1, v1.x, __builtin_fmaf(w0, v0.x, acc[0])));
+        acc[1] = __builtin_fmaf(w2, v2.y, __builtin_fmaf(w1, v1.y, __builtin_fmaf(w0, v0.y, acc[1])));
+        acc[2] = __builtin_fmaf(w2, v2.z, __builtin_fmaf(w1, v1.z, __builtin_fmaf(w0, v0.z, acc[2])));
+        acc[3] = __builtin_fmaf(w2, v2.w, __builtin_fmaf(w1, v1.w, __builtin_fmaf(w0, v0.w, acc[3])));
+    }
+    if (k >= g.ndet) return;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int b = 4 * grp + s;
+        if (b < batch) part[(((size_t)ch * batch + b) * g.nang + a) * g.ndet + k] = acc[s] * scale;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_adjoint_sum(const float* __restrict__ part, float* __restrict__ dq,
+                                                     size_t count, int nchunk) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    float v = part[i];
+    for (int c = 1; c < nchunk; c++) v += part[c * count + i];
+    dq[i] = v;
+}
+
+// dh[m + ndet - 1] += sum_k dq[row][k] * p[row][k - m] for every row.  A
+// thread sums eight consecutive lags m0 .. m0 + 7 over kFgRows rows: per eight
+// k it reads eight values of dq (wave-uniform addresses) and eight new ones of
+// p for 64 products (two LDS reads a product before).  p stands in LDS with
+// zeros around it, so no lag needs its own range; a wave walks the k its lags
+// reach.  Groups of eight p are nine words apart, so the lanes' reads (eight
+// p apart) fall on distinct banks (eight words apart: 141 us).  960 rows of
+// 725 bins: 110 -> 53 us.
+constexpr int kFgRows = 2, kFgLags = 8, kFgThreads = 192;
+constexpr size_t filter_grad_lds(int ndet) {  // dq row, then p in groups of eight at a pitch of nine
+    const size_t nk = ((size_t)ndet + 7) & ~(size_t)7;
+    return sizeof(float) * (nk + 9 * (nk / 8 + kFgThreads));
+}
+__global__ __launch_bounds__(kFgThreads) void k_filter_grad(const float* __restrict__ dq, const float* __restrict__ p,
+                                                            float* __restrict__ dh, int ndet, int rows) {
     extern __shared__ float sm[];
-    float* gs = sm;
-    float* ps = sm + ndet;
-    const size_t row = blockIdx.x;
-    for (int t = threadIdx.x; t < ndet; t += 256) {
-        gs[t] = dq[row * ndet + t];
-        ps[t] = p[row * ndet + t];
+    const int nk = (ndet + 7) & ~7;         // k in steps of 8 (dq zero past ndet)
+    const int lags = 2 * ndet - 1;
+    const int lag0 = (int)blockIdx.y * kFgThreads * kFgLags;  // this workgroup's first lag index m + ndet - 1
+    float* const gs = sm;
+    float* const ps = sm + nk;              // p[xlo + 8 c + i] at ps[9 c + i]
+    // lag index mi at k needs p[k - mi + ndet - 1]
+    const int xlo = ndet - 1 - lag0 - kFgThreads * kFgLags, nx = kFgThreads * kFgLags + nk;
+    const int mi = lag0 + (int)threadIdx.x * kFgLags;
+    // k that some lag of this wave reaches: [m_first, ndet + m_last)
+    const int w0 = lag0 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u)) * kFgLags;
+    const int klo = max(w0 - (ndet - 1), 0) & ~7, khi = min(nk, w0 + 64 * kFgLags);
+    float acc[kFgLags];
+#pragma unroll
+    for (int i = 0; i < kFgLags; i++) acc[i] = 0.0f;
+    for (int rr = 0; rr < kFgRows; rr++) {
+        const int row = (int)blockIdx.x * kFgRows + rr;
+        if (row >= rows) break;  // uniform
+        __syncthreads();
+        for (int t = threadIdx.x; t < nk; t += kFgThreads) gs[t] = t < ndet ? dq[(size_t)row * ndet + t] : 0.0f;
+        for (int t = threadIdx.x; t < nx; t += kFgThreads) {
+            const int x = xlo + t;
+            ps[9 * (t >> 3) + (t & 7)] = (x >= 0 && x < ndet) ? p[(size_t)row * ndet + x] : 0.0f;
+        }
+        __syncthreads();
+        // p[k - mi + ndet - 1 + i], i = 0..7, is the group kFgThreads - threadIdx.x + k/8; lag mi + i at
+        // k + u takes w[7 + u - i]
+        const float* q = ps + 9 * (kFgThreads - (int)threadIdx.x + (klo >> 3));
+        float w[2 * kFgLags - 1];
+#pragma unroll
+        for (int i = 0; i < kFgLags - 1; i++) w[i] = q[i + 1 - 9];
+        for (int k = klo; k < khi; k += 8, q += 9) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) w[kFgLags - 1 + i] = q[i];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const float gv = gs[k + u];
+#pragma unroll
+                for (int i = 0; i < kFgLags; i++) acc[i] = __builtin_fmaf(gv, w[kFgLags - 1 + u - i], acc[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < kFgLags - 1; i++) w[i] = w[i + 8];
+        }
     }
+    // through LDS, so that a wave's atomics cover consecutive lags
     __syncthreads();
-    for (int mi = threadIdx.x; mi < 2 * ndet - 1; mi += 256) {
-        const int m = mi - (ndet - 1);
-        const int klo = m > 0 ? m : 0, khi = m > 0 ? ndet : ndet + m;
-        float s = 0.0f;
-        for (int k = klo; k < khi; k++) s = __builtin_fmaf(gs[k], ps[k - m], s);
-        atomicAdd(dh + mi, s);
-    }
+#pragma unroll
+    for (int i = 0; i < kFgLags; i++) ps[9 * (int)threadIdx.x + i] = acc[i];
+    __syncthreads();
+    for (int t = threadIdx.x; t < kFgThreads * kFgLags && lag0 + t < lags; t += kFgThreads)
+        atomicAdd(dh + lag0 + t, ps[9 * (t >> 3) + (t & 7)]);
 }
 
 // Symmetric taps: full[m + ndet - 1] = sym[|m|].
@@ -1196,8 +1414,6 @@ __global__ void k_noise(float* __restrict__ sino, size_t count, float i0, float 
 // launchers
 // ---------------------------------------------------------------------------
 
-#define SKE_GRID(n, b) dim3((n) / T, (n) / T, (b))
-
 template <int C>
 hipError_t pack_weights_t(const float* prm, uint16_t* wb, hipStream_t s) {
     hipLaunchKernelGGL(k_pack_weights<C>, dim3((9 * C * C + 255) / 256), dim3(256), 0, s, prm, wb);
@@ -1237,27 +1453,19 @@ template <int C>
 hipError_t backward_t(const LearnedBufs& B, const float* prm, const float* dout, float* grad, int n, int batch,
                       hipStream_t s) {
     constexpr LearnedLayout L = learned_layout(C);
-    // activation gradients
-    hipLaunchKernelGGL(k_conv_out_bwd<C>, SKE_GRID(n, batch), dim3(256), 0, s, dout, B.a3, prm, B.dz3, n);
     const dim3 g16(n / kFT, n / kFT, batch);
-    hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, B.wt3, B.dz2, n);
-    hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, B.wt2, B.dz1, n);
-    dim3 g8(n / T, n / TY, batch);
-    hipLaunchKernelGGL(k_conv_in_bwd<C>, g8, dim3(128), 0, s, B.dz1, dout, prm, B.dr0, n);
-    // weight gradients: about 2048 workgroups, each summing over a share of
-    // the slices
-    const int tiles = (n / T) * (n / TY);
-    const dim3 gw(n / T, n / TY, (unsigned)std::max(1, std::min(batch, 2048 / tiles)));
-    const size_t lw4 = sizeof(float) * (TY * T * 1 + (TY + 2) * (T + 2) * C);
-    hipLaunchKernelGGL(k_wgrad<C>, gw, dim3(256), lw4, s, dout, 1, B.a3, (const float*)nullptr, C, grad, L.W4, L.B4, 1,
-                       n, batch);
+    // weight gradients sum over a share of the slices: about 2048 workgroups
     const int tiles16 = (n / kFT) * (n / kFT);
     const dim3 gm(n / kFT, n / kFT, (unsigned)std::max(1, std::min(batch, 2048 / tiles16)));
+    // workgroups the card holds: four (out), four or two (in, by its LDS) per CU of 256
+    const unsigned items = (unsigned)tiles16 * (unsigned)batch;
+    const unsigned out_wgs = std::min(items, 1024u), in_wgs = std::min(items, C == 16 ? 1024u : 512u);
+    hipLaunchKernelGGL(k_conv_out_bwd<C>, dim3(out_wgs), dim3(256), 0, s, dout, B.a3, prm, B.dz3, grad, n, batch);
+    hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, B.wt3, B.dz2, n);
+    hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, B.wt2, B.dz1, n);
     hipLaunchKernelGGL(k_wgrad_mfma<C>, gm, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, grad, L.W3, L.B3, n, batch);
     hipLaunchKernelGGL(k_wgrad_mfma<C>, gm, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, grad, L.W2, L.B2, n, batch);
-    const size_t lw1 = sizeof(float) * (TY * T * C + (TY + 2) * (T + 2) * 1);
-    hipLaunchKernelGGL(k_wgrad<C>, gw, dim3(256), lw1, s, B.dz1, C, (const uint16_t*)nullptr, B.r0, 1, grad, L.W1,
-                       L.B1, 0, n, batch);
+    hipLaunchKernelGGL(k_conv_in_bwd<C>, dim3(in_wgs), dim3(256), 0, s, B.dz1, dout, B.r0, prm, B.dr0, grad, n, batch);
     return hipGetLastError();
 }
 
@@ -1266,28 +1474,26 @@ hipError_t launch_cnn_backward(const LearnedBufs& B, const float* prm, const flo
     return B.C == 32 ? backward_t<32>(B, prm, dout, grad, n, batch, s) : backward_t<16>(B, prm, dout, grad, n, batch, s);
 }
 
-// out[b][j][i] = in[b][i][j] for n x n slices, through 32 x 32 LDS tiles.
-__global__ __launch_bounds__(256) void k_transpose(const float* __restrict__ in, float* __restrict__ out, int n) {
-    __shared__ float tile[32][33];
-    const size_t off = (size_t)blockIdx.z * n * n;
-    const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    for (int k = ty; k < 32; k += 8)
-        if (y0 + k < n && x0 + tx < n) tile[k][tx] = in[off + (size_t)(y0 + k) * n + x0 + tx];
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8)
-        if (x0 + k < n && y0 + tx < n) out[off + (size_t)(x0 + k) * n + y0 + tx] = tile[tx][k];
-}
-
-hipError_t launch_filter_backward(const float* dr0, float* drT, float* dq, const float* sino, float* dfull,
-                                  float* dsym, const float2* cs, const FbpGeom& g, int batch, hipStream_t s) {
+hipError_t launch_filter_backward(const float* dr0, float* lines, float* part, float* dq, const float* sino,
+                                  float* dfull, float* dsym, const float2* cs, const FbpGeom& g, int batch,
+                                  hipStream_t s) {
     const float scale = (float)(M_PI / g.nang);
-    hipLaunchKernelGGL(k_transpose, dim3((g.n + 31) / 32, (g.n + 31) / 32, batch), dim3(256), 0, s, dr0, drT, g.n);
-    hipLaunchKernelGGL(k_bp_adjoint_gather, dim3((g.ndet + 255) / 256, g.nang, batch), dim3(256), 0, s, dr0, drT, dq,
-                       cs, g, scale);
-    const size_t lds = sizeof(float) * 2 * (size_t)g.ndet;
-    hipLaunchKernelGGL(k_filter_grad, dim3((unsigned)((size_t)batch * g.nang)), dim3(256), lds, s, dq, sino, dfull,
-                       g.ndet);
+    const unsigned groups = (unsigned)(batch + 3) / 4, tiles = (unsigned)(g.n + 2 * kAdjPad + 31) / 32;
+    float4* const rows = reinterpret_cast<float4*>(lines);
+    float4* const cols = rows + (size_t)groups * g.n * (g.n + 2 * kAdjPad);
+    hipLaunchKernelGGL(k_adjoint_lines, dim3(tiles, tiles, groups), dim3(256), 0, s, dr0, rows, cols, g.n, batch);
+    const int nchunk = adjoint_chunks(g.n);
+    hipLaunchKernelGGL(k_bp_adjoint, dim3((g.ndet + 255) / 256, g.nang, groups * nchunk), dim3(256), 0, s, rows, cols,
+                       nchunk > 1 ? part : dq, cs, g, scale, batch, nchunk);
+    const size_t count = (size_t)batch * g.nang * g.ndet;
+    if (nchunk > 1)
+        hipLaunchKernelGGL(k_adjoint_sum, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, part, dq, count,
+                           nchunk);
+    const int nrow = batch * g.nang;
+    hipLaunchKernelGGL(k_filter_grad,
+                       dim3((unsigned)(nrow + kFgRows - 1) / kFgRows,
+                            (unsigned)((2 * g.ndet - 1 + kFgThreads * kFgLags - 1) / (kFgThreads * kFgLags))),
+                       dim3(kFgThreads), filter_grad_lds(g.ndet), s, dq, sino, dfull, g.ndet, nrow);
     hipLaunchKernelGGL(k_taps_fold, dim3((g.ndet + 255) / 256), dim3(256), 0, s, dfull, dsym, g.ndet);
     return hipGetLastError();
 }

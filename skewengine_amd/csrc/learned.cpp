@@ -27,7 +27,7 @@ struct ske_learned {
     bool derived = false;          // full taps and bf16 weights match prm (cleared whenever prm changes)
     DevBuf<float> prm, grad, m1, m2, full, dq, dfull, dout;
     DevBuf<double> loss;
-    DevBuf<float> r0, dz, dr0, drT;  // dz: three layers back to back; drT: dr0 transposed
+    DevBuf<float> r0, dz, dr0, drL, dqp;  // dz: three layers back to back; drL, dqp: the adjoint's lines and partial sums
     DevBuf<uint16_t> act, wb;      // act: a1, a2, a3 back to back; wb: bf16 weights (learned_wb_size)
     DevBuf<float> ell;
     size_t pix(int batch) const { return (size_t)f->g.n * f->g.n * (size_t)batch; }
@@ -130,7 +130,8 @@ int ensure_train(ske_learned* l) {
     const FbpGeom& g = l->f->g;
     SKE_TRY(l->dz.ensure(3 * l->pix(mb) * l->C));
     SKE_TRY(l->dr0.ensure(l->pix(mb)));
-    SKE_TRY(l->drT.ensure(l->pix(mb)));
+    SKE_TRY(l->drL.ensure(adjoint_lines_floats(g.n, mb)));
+    if (adjoint_chunks(g.n) > 1) SKE_TRY(l->dqp.ensure((size_t)adjoint_chunks(g.n) * mb * g.nang * g.ndet));
     SKE_TRY(l->dout.ensure(l->pix(mb)));
     SKE_TRY(l->dq.ensure((size_t)mb * g.nang * g.ndet));
     SKE_TRY(l->dfull.ensure(2 * (size_t)g.ndet - 1));
@@ -155,7 +156,7 @@ int gradient(ske_learned* l, int batch) {
     return f->timer.launch(s, "filter_backward", [&] {
         hipError_t e = launch_fill_f32(l->dfull.p, 2 * (size_t)g.ndet - 1, 0.0f, s);
         if (e != hipSuccess) return e;
-        return launch_filter_backward(l->dr0.p, l->drT.p, l->dq.p, f->buf[SKE_FBP_SINO].p, l->dfull.p,
+        return launch_filter_backward(l->dr0.p, l->drL.p, l->dqp.p, l->dq.p, f->buf[SKE_FBP_SINO].p, l->dfull.p,
                                       l->grad.p + l->L.Taps, f->cs.p, g, batch, s);
     });
 }
