@@ -73,8 +73,12 @@ int ske_fbp_create(int n, int n_angles, int n_det, const float* angles, int max_
     ramlak_taps(n_det, 2.0 / n, f->taps_host);
     SKE_TRY(f->taps.upload(f->taps_host.data(), f->taps_host.size(), f->stream));
     for (int w = 0; w < 4; w++) SKE_TRY(f->buf[w].ensure(f->elems(w, max_batch)));
-    f->pt = proj_tiling(n);
-    SKE_TRY(f->part.ensure((size_t)max_batch * n_angles * f->pt.ntx * f->pt.ntx * f->pt.kw));
+    // the projector's partial sums: room for its four-slice tiles (about 1.5
+    // times the one-slice tiles') unless that is over 8 GiB or not to be had
+    const size_t part1 = proj_part_floats(n, n_angles, max_batch, 1);
+    const size_t part4 = max_batch > 1 ? proj_part_floats(n, n_angles, max_batch, 4) : 0;
+    if (part4 <= part1 || part4 * sizeof(float) > (8ull << 30) || f->part.ensure(part4) != SKE_OK)
+        SKE_TRY(f->part.ensure(part1));
     SKE_TRY(f->timer.sync(f->stream));
     *out = f.release();
     return SKE_OK;
@@ -115,7 +119,7 @@ int ske_fbp_buffer(ske_fbp* f, int which, float** d_ptr) {
 int ske_fbp_project(ske_fbp* f, int batch) {
     SKE_TRY(check_batch(f, batch));
     return f->timer.launch(f->stream, "fbp_project", [&] {
-        return launch_fbp_project(f->buf[SKE_FBP_IMAGE].p, f->part.p, f->buf[SKE_FBP_SINO].p, f->cs.p, f->g, f->pt,
+        return launch_fbp_project(f->buf[SKE_FBP_IMAGE].p, f->part.p, f->part.n, f->buf[SKE_FBP_SINO].p, f->cs.p, f->g,
                                   batch, f->stream);
     });
 }

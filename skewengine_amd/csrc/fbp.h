@@ -16,26 +16,35 @@ struct FbpGeom {
     float pad;
 };
 
-// Tiles of the projector: the base pixels [-1, n) of each axis in ntx tiles
-// of side ts <= kPtMax; kw partial sums per (slice, angle, tile), enough for
-// every bin that can cross a tile (ts sqrt(2) plus margins).
-constexpr int kPtMax = 129;
-constexpr int kPtAngles = 12;  // angles per projector workgroup
+// Tiles of the projector for S slices at a time (1 or 4): the base pixels
+// [-1, n) of each axis in ntx tiles of side ts <= kPtMaxS; kw partial sums per
+// (slice, angle, tile), enough for every bin that can cross a tile (ts sqrt(2)
+// plus margins).
+constexpr int kPtMax1 = 129, kPtMax4 = 67;
+constexpr int kPtAngles = 12;  // angles per projector workgroup, at most
 struct ProjTiling {
     int ntx;
     int ts;
     int kw;
 };
-inline ProjTiling proj_tiling(int n) {
+inline ProjTiling proj_tiling(int n, int slices) {
+    const int most = slices == 1 ? kPtMax1 : kPtMax4;
     ProjTiling t;
-    t.ntx = (n + 1 + kPtMax - 1) / kPtMax;
+    t.ntx = (n + 1 + most - 1) / most;
     t.ts = (n + 1 + t.ntx - 1) / t.ntx;
     t.kw = (t.ts * 1415 + 999) / 1000 + 8;
     return t;
 }
-// img: batch x n x n; part: batch x nang x ntx^2 x kw floats of scratch.
-hipError_t launch_fbp_project(const float* img, float* part, float* sino, const float2* cs, const FbpGeom& g,
-                              const ProjTiling& pt, int batch, hipStream_t s);
+// Partial sums (floats) of `batch` slices projected `slices` at a time.
+inline size_t proj_part_floats(int n, int nang, int batch, int slices) {
+    const ProjTiling t = proj_tiling(n, slices);
+    return (size_t)batch * nang * t.ntx * t.ntx * t.kw;
+}
+// img: batch x n x n; part: `part_floats` floats of scratch, at least
+// proj_part_floats(n, nang, batch, 1); four slices at a time where it holds
+// theirs.
+hipError_t launch_fbp_project(const float* img, float* part, size_t part_floats, float* sino, const float2* cs,
+                              const FbpGeom& g, int batch, hipStream_t s);
 hipError_t launch_fbp_filter(const float* sino, float* filt, const float* taps, const FbpGeom& g, int batch,
                              hipStream_t s);
 hipError_t launch_fbp_backproject(const float* filt, float* img, const float2* cs, const FbpGeom& g, int batch,

@@ -16,7 +16,6 @@ struct ske_fbp {
     ske::DevBuf<float> taps;
     std::vector<float> taps_host;
     ske::DevBuf<float> buf[4];  // image, sinogram, filtered, reconstruction
-    ske::ProjTiling pt{};
     ske::DevBuf<float> part;    // the projector's partial sums per tile
     ske::LaunchTimer timer;
     ~ske_fbp() {
