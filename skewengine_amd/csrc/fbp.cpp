@@ -6,6 +6,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <memory>
 #include <vector>
 
@@ -73,10 +74,11 @@ int ske_fbp_create(int n, int n_angles, int n_det, const float* angles, int max_
     ramlak_taps(n_det, 2.0 / n, f->taps_host);
     SKE_TRY(f->taps.upload(f->taps_host.data(), f->taps_host.size(), f->stream));
     for (int w = 0; w < 4; w++) SKE_TRY(f->buf[w].ensure(f->elems(w, max_batch)));
-    // the projector's partial sums: room for its four-slice tiles (about 1.5
-    // times the one-slice tiles') unless that is over 8 GiB or not to be had
+    // the projector's partial sums: room for eight slices of its four-slice
+    // tiles (larger batches go through in turn) unless that is over 8 GiB or
+    // not to be had
     const size_t part1 = proj_part_floats(n, n_angles, max_batch, 1);
-    const size_t part4 = max_batch > 1 ? proj_part_floats(n, n_angles, max_batch, 4) : 0;
+    const size_t part4 = max_batch > 1 ? proj_part_floats(n, n_angles, std::min(max_batch, 8), 4) : 0;
     if (part4 <= part1 || part4 * sizeof(float) > (8ull << 30) || f->part.ensure(part4) != SKE_OK)
         SKE_TRY(f->part.ensure(part1));
     SKE_TRY(f->timer.sync(f->stream));

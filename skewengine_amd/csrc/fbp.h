@@ -42,7 +42,7 @@ inline size_t proj_part_floats(int n, int nang, int batch, int slices) {
 }
 // img: batch x n x n; part: `part_floats` floats of scratch, at least
 // proj_part_floats(n, nang, batch, 1); four slices at a time where it holds
-// theirs.
+// the partial sums of as many.
 hipError_t launch_fbp_project(const float* img, float* part, size_t part_floats, float* sino, const float2* cs,
                               const FbpGeom& g, int batch, hipStream_t s);
 hipError_t launch_fbp_filter(const float* sino, float* filt, const float* taps, const FbpGeom& g, int batch,

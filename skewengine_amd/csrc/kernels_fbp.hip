@@ -620,16 +620,21 @@ static hipError_t project_t(const float* img, float* part, float* sino, const fl
 
 // Four slices at a time, the last group with empty slices; where one group
 // fills the card, a single last slice goes by itself (it takes 0.4 of a group).
+// Batches whose partial sums do not fit `part` at once go through it in turn.
 hipError_t launch_fbp_project(const float* img, float* part, size_t part_floats, float* sino, const float2* cs,
                               const FbpGeom& g, int batch, hipStream_t s) {
     const ProjTiling pt = proj_tiling(g.n, 4);
     const bool fills = (long long)pt.ntx * pt.ntx * ((g.nang + kPtAngles - 1) / kPtAngles) >= 512;
+    const int fit = (int)std::min((size_t)batch, part_floats / proj_part_floats(g.n, g.nang, 1, 4));
     int four = batch == 1 ? 0 : (batch % 4 == 1 && fills) ? batch - 1 : batch;
-    if (proj_part_floats(g.n, g.nang, four, 4) > part_floats) four = 0;
-    if (four > 0) {
-        const hipError_t e = project_t<4>(img, part, sino, cs, g, four, s);
-        if (e != hipSuccess || four == batch) return e;
+    if (fit < std::min(four, 4)) four = 0;
+    const int step = fit >= four ? std::max(four, 1) : fit & ~3;
+    for (int b = 0; b < four; b += step) {
+        const hipError_t e = project_t<4>(img + (size_t)b * g.n * g.n, part, sino + (size_t)b * g.nang * g.ndet, cs, g,
+                                          std::min(step, four - b), s);
+        if (e != hipSuccess) return e;
     }
+    if (four == batch) return hipSuccess;
     return project_t<1>(img + (size_t)four * g.n * g.n, part, sino + (size_t)four * g.nang * g.ndet, cs, g,
                         batch - four, s);
 }
