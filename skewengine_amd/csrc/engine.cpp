@@ -84,6 +84,7 @@ struct Chunk {
     struct Part {
         int img;
         int range[8];
+        int init;  // bit t: the run's first sectors of orientation t of this grid
     };
     std::vector<Part> parts;
     DevBuf<DeskewPart> dparts;  // the parts for the one-launch deskew
@@ -161,6 +162,7 @@ struct Core {
     int ncu = 0;
     hipStream_t stream = nullptr;
     std::vector<Image> imgs;
+    std::vector<ReduceImage> rimgs;  // the same for the reduce
     DevBuf<float> in4, acc, out;
     int present[4] = {0, 0, 0, 0};  // per run, same for every grid (same sector range)
     // constant tables
@@ -316,6 +318,7 @@ struct Core {
             im.out_off = tot;
             tot += N;
             imgs.push_back(im);
+            rimgs.push_back(ReduceImage{im.acc_off, im.out_off, im.n, 0});
         }
         SKE_TRY(in4.ensure(4 * (size_t)tot));
         SKE_TRY(acc.ensure(4 * (size_t)tot));
@@ -361,6 +364,8 @@ struct Core {
                 for (int r = 0; r < 8; r++) dp[k].range[r] = cur->parts[k].range[r];
                 dp[k].acc_off = im.acc_off;
                 dp[k].dimx = dp[k].dimy = im.n;
+                dp[k].init = cur->parts[k].init;
+                dp[k].pad0 = 0;
                 cur->max_n = std::max(cur->max_n, im.n);
             }
             SKE_TRY(cur->dparts.upload(dp.data(), dp.size(), stream));
@@ -375,7 +380,7 @@ struct Core {
         };
         for (int gi = 0; gi < (int)imgs.size(); gi++) {
             const int n = imgs[gi].n;
-            int a = s0;
+            int a = s0, seen = 0;  // seen: orientations with sectors in an earlier part
             while (a < s1) {
                 // extend this grid's run of sectors while it fits the chunk
                 int b = a;
@@ -394,6 +399,11 @@ struct Core {
                 Chunk::Part part;
                 part.img = gi;
                 plan_append(n, n, a, b, imgs[gi].in_off, cur->plan.ip, part.range);
+                int has = 0;
+                for (int t = 0; t < 4; t++)
+                    if (part.range[2 * t] < part.range[2 * t + 1]) has |= 1 << t;
+                part.init = has & ~seen;
+                seen |= has;
                 cur->parts.push_back(part);
                 a = b;
                 if (a < s1) SKE_TRY(flush());
@@ -468,8 +478,6 @@ struct Core {
         const bool local = kernel_id == SKE_KERNEL_RADON && radon_local;
         const bool radon = kernel_id == SKE_KERNEL_RADON && !local;
         const int is_max = kernel_id == SKE_KERNEL_CEPSTRUM ? 1 : 0;
-        const size_t acc_n = acc.n;
-        SKE_TRY(launch("fill", [&] { return launch_fill_f32(acc.p, acc_n, 0.0f, stream); }));
         const bool samples = local && !sample_xy.empty();
         if (samples) {
             const size_t nout = (size_t)SKE_MAX_SECTOR * (sample_xy.size() / 2) * 256;
@@ -521,27 +529,21 @@ struct Core {
             const int source = radon ? kDeskewRadon : kDeskewArena;
             if (radon) {  // latency-bound per image: every image of the chunk in one launch
                 SKE_TRY(launch("deskew", [&] {
-                    return launch_deskew_parts(v, cp->dparts.p, (int)cp->parts.size(), cp->max_n, src, source, is_max,
-                                               acc.p, stream);
+                    return launch_deskew_parts(v, cp->dparts.p, (int)cp->parts.size(), cp->max_n, src, acc.p, stream);
                 }));
             } else {  // grids sized to each image (a chunk's images may differ in size)
                 for (const Chunk::Part& part : cp->parts) {
                     const Image& im = imgs[part.img];
                     SKE_TRY(launch("deskew", [&] {
-                        return launch_deskew(v, part.range, src, source, is_max, acc.p, im.n, im.n, im.acc_off,
-                                             stream);
+                        return launch_deskew(v, part.range, src, source, is_max, part.init, acc.p, im.n, im.n,
+                                             im.acc_off, stream);
                     }));
                 }
             }
         }
-        const size_t out_n = out.n;
-        SKE_TRY(launch("fill", [&] { return launch_fill_f32(out.p, out_n, 0.0f, stream); }));
-        for (const Image& im : imgs) {
-            SKE_TRY(launch("reduce", [&] {
-                return launch_reduce(acc.p + im.acc_off, present, out.p + im.out_off, im.n, im.n, is_max, stream);
-            }));
-        }
-        return SKE_OK;
+        return launch("reduce", [&] {
+            return launch_reduce_images(acc.p, present, out.p, rimgs.data(), (int)rimgs.size(), is_max, stream);
+        });
     }
 
     int run(int kernel_id, int s0, int s1, float povh) {
@@ -880,7 +882,7 @@ int sector_deskew(ske_engine* e, int is_max) {
         SKE_TRY(c.launch("fill", [&] { return launch_fill_f32(c.acc.p + (size_t)t * e->N, (size_t)e->N, 0.0f, c.stream); }));
     }
     SKE_TRY(c.launch("deskew", [&] {
-        return launch_deskew(v, range, e->SO.p, kDeskewDense, is_max ? 1 : 0, c.acc.p, e->dimx, e->dimy, 0, c.stream);
+        return launch_deskew(v, range, e->SO.p, kDeskewDense, is_max ? 1 : 0, 0, c.acc.p, e->dimx, e->dimy, 0, c.stream);
     }));
     e->present[t] = 1;
     return SKE_OK;

@@ -160,20 +160,6 @@ __device__ __forceinline__ float so_cell(const SecDesc* __restrict__ secs, int s
     return 0.0f;
 }
 
-// Tap (r, j) of sector si with the common case r < H read without branches:
-// the row index is clamped into the sector (in bounds of its H x dim_i slot)
-// and the value masked by the row's first/last range afterwards.  Rows r >= H
-// are patched by the caller through so_cell.
-template <int kSource>
-__device__ __forceinline__ float so_tap(const SecDesc& sd, const uint32_t* __restrict__ fl,
-                                        const float* __restrict__ src, int r, int j) {
-    if (kSource == kDeskewDense) return src[(size_t)r * sd.dim_i + j];
-    const int rc = min(r, sd.H - 1);
-    const uint32_t v = fl[sd.rows + rc];
-    const float x = (kSource == kDeskewArena) ? src[sd.so + (size_t)rc * sd.dim_i + j] : src[sd.q + rc];
-    return (j >= fl_first(v) && j < fl_last(v)) ? x : 0.0f;
-}
-
 template <int kMax>
 __device__ __forceinline__ float deskew_acc(float O, float a, float b, float wj, int angle) {
     if (kMax) {
@@ -183,34 +169,54 @@ __device__ __forceinline__ float deskew_acc(float O, float a, float b, float wj,
     return O + ((1.0f - wj) * a + wj * b);
 }
 
-// One output cell over sectors [sb, se), in ascending order.
-template <int kSource, int kMax>
-__device__ void deskew_cell(const SecDesc* __restrict__ secs, const int* __restrict__ target,
-                            const float* __restrict__ weight, const uint32_t* __restrict__ fl,
-                            const float* __restrict__ src, int sb, int se, int i, int j, float* o) {
-    float O = *o;
-    for (int si = sb; si < se; ++si) {
-        const SecDesc& sd = secs[si];
-        const int tj = target[sd.tab + j];
-        const float wj = weight[sd.tab + j];
-        const float a = so_cell<kSource>(secs, si, sd, fl, src, i + tj, j);
-        const float b = so_cell<kSource>(secs, si, sd, fl, src, i + tj + 1, j);
-        O = deskew_acc<kMax>(O, a, b, wj, sd.angle);
+// Which taps need a look at first/last.  Output cell (i, j) reads the skewed
+// rows t_j + i and t_j + i + 1, i.e. t_j + e with 0 <= e <= n (n = dim_o).  In
+// a sector's maps j lies in [first, last) of the rows t_j + 1 .. t_j + n - 1
+// always (t rises by 0 or 1 per column; first is exact, last at most one short,
+// and one short only for the column whose t is the row itself), so only e = 0
+// may fall outside, and e = n where the sector has no such row (newAngle 0).
+// Checked over all sectors of many sides on the CPU: tests/test_deskew_taps.py.
+
+// Taps e = i0 .. i0 + kRows of column j: interior blocks (0 < i0, i0 + kRows <
+// n) read them unseen, the first and the last block look at e = 0 and e = n;
+// taps past the last row are not used.
+template <int kSource, int kRows>
+__device__ __forceinline__ void deskew_taps(const SecDesc* __restrict__ secs, int si, const SecDesc& sd,
+                                            const uint32_t* __restrict__ fl, const float* __restrict__ src, int i0,
+                                            int tj, int j, int dim_o, bool edge, float (&v)[kRows + 1]) {
+    const int r = i0 + tj;
+    if (!edge) {
+        const float* p = kSource == kDeskewRadon ? src + sd.q + r
+                         : src + (kSource == kDeskewArena ? sd.so : 0) + (size_t)r * sd.dim_i + j;
+        const size_t step = kSource == kDeskewRadon ? 1 : sd.dim_i;
+#pragma unroll
+        for (int m = 0; m <= kRows; ++m) v[m] = p[m * step];
+        return;
     }
-    *o = O;
+    const int last = min(kRows, dim_o - i0);
+#pragma unroll
+    for (int m = 0; m <= kRows; ++m) {
+        const int e = i0 + m;
+        if (m > last)
+            v[m] = 0.0f;
+        else if (e == 0 || e == dim_o)
+            v[m] = so_cell<kSource>(secs, si, sd, fl, src, r + m, j);
+        else if (kSource == kDeskewRadon)
+            v[m] = src[sd.q + r + m];
+        else
+            v[m] = src[(kSource == kDeskewArena ? sd.so : 0) + (size_t)(r + m) * sd.dim_i + j];
+    }
 }
 
-constexpr int kDeskewRows = 16;  // output rows per thread
-
-// kRows consecutive output rows per thread: the kRows + 1 taps of a sector
-// are shared by neighbouring rows.  kU sectors per pass: their table reads,
-// then their gathers are issued together, and each row accumulates in
-// ascending sector order afterwards.  Orientation t of one image: sectors
-// [sb, se), accumulators acc (four dimx*dimy buffers).
-template <int kSource, int kMax, int kRows, int kU>
+// kRows consecutive output rows per thread: the kRows + 1 taps of a sector are
+// shared by neighbouring rows; each row accumulates in ascending sector order.
+// While a sector is added, the taps of the next and the table entries of the
+// one after are on their way.  Orientation t of one image: sectors [sb, se),
+// accumulators acc (four dimx*dimy buffers), started from zero with `init`.
+template <int kSource, int kMax, int kRows>
 __device__ __forceinline__ void deskew_body(const SecDesc* __restrict__ secs, const int* __restrict__ target,
                                             const float* __restrict__ weight, const uint32_t* __restrict__ fl,
-                                            const float* __restrict__ src, int t, int sb, int se,
+                                            const float* __restrict__ src, int t, int sb, int se, bool init,
                                             float* __restrict__ acc, int dimx, int dimy) {
     if (sb >= se) return;
     const bool tr = (t == 1 || t == 2);
@@ -220,60 +226,52 @@ __device__ __forceinline__ void deskew_body(const SecDesc* __restrict__ secs, co
     if (i0 >= dim_o || j >= dim_i) return;
     const size_t N = (size_t)dimx * dimy;
     float* o = acc + (size_t)t * N + (size_t)i0 * dim_i + j;
-    if (i0 + kRows > dim_o) {  // last rows of the image
-        for (int k = 0; k < dim_o - i0; ++k)
-            deskew_cell<kSource, kMax>(secs, target, weight, fl, src, sb, se, i0 + k, j, o + (size_t)k * dim_i);
-        return;
-    }
+    const bool edge = i0 == 0 || i0 + kRows >= dim_o;  // uniform
+    const int nrow = min(kRows, dim_o - i0);
     float O[kRows];
 #pragma unroll
-    for (int k = 0; k < kRows; ++k) O[k] = o[(size_t)k * dim_i];
-    int si = sb;
-    for (; si + kU <= se; si += kU) {
-        int tj[kU];
-        float wj[kU], v[kU][kRows + 1];
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const SecDesc& sd = secs[si + u];
-            tj[u] = target[sd.tab + j];
-            wj[u] = weight[sd.tab + j];
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-#pragma unroll
-            for (int m = 0; m <= kRows; ++m) v[u][m] = so_tap<kSource>(secs[si + u], fl, src, i0 + tj[u] + m, j);
-        }
-        if (kSource != kDeskewDense) {
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-                const SecDesc& sd = secs[si + u];
-                if (i0 + tj[u] + kRows >= sd.H) {
-#pragma unroll
-                    for (int m = 0; m <= kRows; ++m)
-                        if (i0 + tj[u] + m >= sd.H) v[u][m] = so_cell<kSource>(secs, si + u, sd, fl, src, i0 + tj[u] + m, j);
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-            const int angle = secs[si + u].angle;
-#pragma unroll
-            for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<kMax>(O[k], v[u][k], v[u][k + 1], wj[u], angle);
-        }
+    for (int k = 0; k < kRows; ++k) O[k] = (!init && k < nrow) ? o[(size_t)k * dim_i] : 0.0f;
+    float v[kRows + 1], vn[kRows + 1];
+    int tn = target[secs[sb].tab + j];
+    float w = weight[secs[sb].tab + j], wn = 0.0f;
+    deskew_taps<kSource, kRows>(secs, sb, secs[sb], fl, src, i0, tn, j, dim_o, edge, v);
+    if (sb + 1 < se) {
+        tn = target[secs[sb + 1].tab + j];
+        wn = weight[secs[sb + 1].tab + j];
     }
-    for (; si < se; ++si) {
-        const SecDesc& sd = secs[si];
-        const int tj = target[sd.tab + j];
-        const float wj = weight[sd.tab + j];
-        float v[kRows + 1];
+    for (int si = sb; si < se; ++si) {
+        int t2 = 0;
+        float w2 = 0.0f;
+        if (si + 2 < se) {
+            t2 = target[secs[si + 2].tab + j];
+            w2 = weight[secs[si + 2].tab + j];
+        }
+        if (si + 1 < se)
+            deskew_taps<kSource, kRows>(secs, si + 1, secs[si + 1], fl, src, i0, tn, j, dim_o, edge, vn);
+        const int angle = secs[si].angle;
 #pragma unroll
-        for (int m = 0; m <= kRows; ++m) v[m] = so_cell<kSource>(secs, si, sd, fl, src, i0 + tj + m, j);
+        for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<kMax>(O[k], v[k], v[k + 1], w, angle);
 #pragma unroll
-        for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<kMax>(O[k], v[k], v[k + 1], wj, sd.angle);
+        for (int m = 0; m <= kRows; ++m) v[m] = vn[m];
+        w = wn;
+        wn = w2;
+        tn = t2;
     }
 #pragma unroll
-    for (int k = 0; k < kRows; ++k) o[(size_t)k * dim_i] = O[k];
+    for (int k = 0; k < kRows; ++k)
+        if (k < nrow) o[(size_t)k * dim_i] = O[k];
 }
+
+// Bound by the latency of the gathers (an arena is read once: 500^2 moves 190
+// MB).  With every tap tested against its row's range, one sector at a time and
+// the last rows of an odd side one by one, all sectors took 250 us at 500^2 and
+// 1,450 us at 1501^2; now 130 and 870 us.  Below four workgroups of 16 rows per
+// CU more, shorter threads hide more of it: 500^2 138 us with 16 rows, 130 with
+// 8; the Radon source 44 us with 4 rows unstaged, 40 staged (one 512^2 image;
+// 49 before).
+constexpr int kDeskewRows = 16;      // output rows per thread
+constexpr int kDeskewSmallRows = 8;  // of an arena below 1024 workgroups of the former
+constexpr int kDeskewRadonRows = 4;  // of the Radon source below 1024 workgroups
 
 __device__ __forceinline__ int range_begin(int t, int4 lo, int4 hi) {
     return (t == 0) ? lo.x : (t == 1) ? lo.z : (t == 2) ? hi.x : hi.z;
@@ -282,48 +280,39 @@ __device__ __forceinline__ int range_end(int t, int4 lo, int4 hi) {
     return (t == 0) ? lo.y : (t == 1) ? lo.w : (t == 2) ? hi.y : hi.w;
 }
 
-// One image: blockIdx.z = orientation.
-template <int kSource, int kMax, int kRows, int kU>
+// One image: blockIdx.z = orientation; bit t of `init`: orientation t starts
+// from zero.
+template <int kSource, int kMax, int kRows>
 __global__ __launch_bounds__(256) void k_deskew(const SecDesc* __restrict__ secs, const int* __restrict__ target,
                                                 const float* __restrict__ weight, const uint32_t* __restrict__ fl,
-                                                const float* __restrict__ src, int4 rlo, int4 rhi,
+                                                const float* __restrict__ src, int4 rlo, int4 rhi, int init,
                                                 float* __restrict__ acc, int dimx, int dimy) {
     const int t = blockIdx.z;
-    deskew_body<kSource, kMax, kRows, kU>(secs, target, weight, fl, src, t, range_begin(t, rlo, rhi),
-                                          range_end(t, rlo, rhi), acc, dimx, dimy);
-}
-
-// Every image of a chunk in one launch: blockIdx.z = 4 * part + orientation,
-// so the images' cells run side by side instead of one launch after another.
-template <int kSource, int kMax, int kRows, int kU>
-__global__ __launch_bounds__(256) void k_deskew_parts(const SecDesc* __restrict__ secs,
-                                                      const int* __restrict__ target,
-                                                      const float* __restrict__ weight,
-                                                      const uint32_t* __restrict__ fl, const float* __restrict__ src,
-                                                      const DeskewPart* __restrict__ parts, float* __restrict__ acc) {
-    const DeskewPart& P = parts[blockIdx.z >> 2];
-    const int t = blockIdx.z & 3;
-    deskew_body<kSource, kMax, kRows, kU>(secs, target, weight, fl, src, t, P.range[2 * t], P.range[2 * t + 1],
-                                          acc + P.acc_off, P.dimx, P.dimy);
+    deskew_body<kSource, kMax, kRows>(secs, target, weight, fl, src, t, range_begin(t, rlo, rhi),
+                                      range_end(t, rlo, rhi), (init >> t) & 1, acc, dimx, dimy);
 }
 
 // The Radon deskew with the taps staged in LDS.  A Radon skewOutput row r
 // holds q[r] on [first_r, last_r), so a sector's taps for a workgroup's 256
-// columns j0 .. j0+255 and rows i0 .. i0+15 are q and first|last of the rows
-// i0 + t_j .. i0 + t_j + 16: since t is nondecreasing with steps of 0 or 1,
-// the rows i0 + t_{j0} .. i0 + t_{jlast} + 16, at most 272.  A pass stages
-// them for kRadonU sectors (rows past H as empty rows), then every thread
-// reads its 17 taps per sector from LDS: the values so_cell gives, added in
+// columns j0 .. j0+255 and rows i0 .. i0+15 are q of the rows i0 + t_j ..
+// i0 + t_j + 16: since t is nondecreasing with steps of 0 or 1, the rows
+// i0 + t_{j0} .. i0 + t_{j0} + 271, at most.  A pass stages them for kRadonU
+// sectors (zeros past H), two sectors a wave; the next pass's rows and table
+// entries are loaded into registers while this one's are added.  Then every
+// thread reads its 17 taps per sector from LDS: the values so_cell gives
+// (first/last matter for the tap of row t_j alone, see above), added in
 // ascending sector order, so the result is the k_deskew one bit for bit.
-constexpr int kRadonU = 8, kRadonStage = 288;  // 18 KB of LDS: eight sectors per pass
+// Bound by VALU and LDS issue at four workgroups per CU: 16 x 512^2 189 us (260
+// with the row ranges staged and tested too and no loads in flight meanwhile).
+constexpr int kRadonU = 8, kRadonStage = 288;  // 9 KB of LDS: eight sectors per pass
+template <int kRows>
 __device__ __forceinline__ void deskew_radon_body(const SecDesc* __restrict__ secs, const int* __restrict__ target,
                                                   const float* __restrict__ weight,
                                                   const uint32_t* __restrict__ fl, const float* __restrict__ q,
-                                                  int t, int sb, int se, float* __restrict__ acc, int dimx,
+                                                  int t, int sb, int se, bool init, float* __restrict__ acc, int dimx,
                                                   int dimy) {
-    constexpr int kRows = kDeskewRows;
+    constexpr int kPer = kRadonU / 4, kLoads = (kRadonStage + 63) / 64;
     __shared__ float sq[kRadonU * kRadonStage];
-    __shared__ uint32_t sfl[kRadonU * kRadonStage];
     if (sb >= se) return;  // uniform
     const bool tr = (t == 1 || t == 2);
     const int dim_i = tr ? dimy : dimx, dim_o = tr ? dimx : dimy;
@@ -332,44 +321,67 @@ __device__ __forceinline__ void deskew_radon_body(const SecDesc* __restrict__ se
     if (i0 >= dim_o || j0 >= dim_i) return;  // uniform
     const int j = min(j0 + (int)threadIdx.x, dim_i - 1);
     const bool col = j0 + (int)threadIdx.x < dim_i;
-    const int jlast = min(j0 + (int)blockDim.x - 1, dim_i - 1);
     const size_t N = (size_t)dimx * dimy;
     float* o = acc + (size_t)t * N + (size_t)i0 * dim_i + j;
     const int nrow = min(kRows, dim_o - i0);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     float O[kRows];
 #pragma unroll
-    for (int k = 0; k < kRows; ++k) O[k] = (col && k < nrow) ? o[(size_t)k * dim_i] : 0.0f;
+    for (int k = 0; k < kRows; ++k) O[k] = (!init && col && k < nrow) ? o[(size_t)k * dim_i] : 0.0f;
+    // sector si + u: this thread's table entries (d: its row past the stage's first), the wave's stage rows
+    int dn[kRadonU];
+    float wn[kRadonU], sn[kPer][kLoads];
+    auto load = [&](int si) {
+#pragma unroll
+        for (int u = 0; u < kRadonU; ++u) {
+            const int tab = secs[min(si + u, se - 1)].tab;
+            dn[u] = target[tab + j] - target[tab + j0];
+            wn[u] = weight[tab + j];
+        }
+#pragma unroll
+        for (int c = 0; c < kPer; ++c) {
+            const SecDesc& sd = secs[min(si + kPer * wave + c, se - 1)];
+            const int r0 = i0 + target[sd.tab + j0];
+#pragma unroll
+            for (int e = 0; e < kLoads; ++e) {
+                const int r = r0 + 64 * e + lane;
+                sn[c][e] = r < sd.H ? q[sd.q + r] : 0.0f;
+            }
+        }
+    };
+    load(sb);
     for (int si = sb; si < se; si += kRadonU) {
         const int nu = min(kRadonU, se - si);
+        int d[kRadonU];
+        float w[kRadonU];
         __syncthreads();  // the previous pass's reads are done
-        for (int e = threadIdx.x; e < nu * kRadonStage; e += blockDim.x) {
-            const int u = e / kRadonStage, x = e - u * kRadonStage;
-            const SecDesc& sd = secs[si + u];
-            const int rlo = i0 + target[sd.tab + j0];
-            const int len = min(target[sd.tab + jlast] - target[sd.tab + j0] + kRows + 1, kRadonStage);
-            const int r = rlo + x;
-            const bool in = x < len && r < sd.H;
-            sq[e] = in ? q[sd.q + r] : 0.0f;
-            sfl[e] = in ? fl[sd.rows + r] : 0u;
+#pragma unroll
+        for (int c = 0; c < kPer; ++c)
+#pragma unroll
+            for (int e = 0; e < kLoads; ++e)
+                if (64 * e + lane < kRadonStage) sq[(kPer * wave + c) * kRadonStage + 64 * e + lane] = sn[c][e];
+#pragma unroll
+        for (int u = 0; u < kRadonU; ++u) {
+            d[u] = dn[u];
+            w[u] = wn[u];
         }
         __syncthreads();
+        if (si + kRadonU < se) load(si + kRadonU);
 #pragma unroll
         for (int u = 0; u < kRadonU; ++u) {
             if (u >= nu) break;  // uniform
-            const SecDesc& sd = secs[si + u];
-            const int tj = target[sd.tab + j];
-            const float wj = weight[sd.tab + j];
-            // stage index of row i0 + tj (tj - t_{j0} <= j - j0 <= 255; the clamp only
-            // guards the stage's bounds)
-            const int base = u * kRadonStage + min(tj - target[sd.tab + j0], kRadonStage - kRows - 1);
+            // stage index of row i0 + t_j (t_j - t_{j0} <= j - j0 <= 255; the clamp only guards the stage's bounds)
+            const float* p = sq + u * kRadonStage + min(d[u], kRadonStage - kRows - 1);
             float v[kRows + 1];
 #pragma unroll
-            for (int m = 0; m <= kRows; ++m) {
-                const uint32_t f = sfl[base + m];
-                v[m] = (j >= fl_first(f) && j < fl_last(f)) ? sq[base + m] : 0.0f;
+            for (int m = 0; m <= kRows; ++m) v[m] = p[m];
+            if (i0 == 0) {  // uniform: the tap of row t_j
+                const SecDesc& sd = secs[si + u];
+                if (j >= fl_last(fl[sd.rows + target[sd.tab + j]])) v[0] = 0.0f;
             }
 #pragma unroll
-            for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<0>(O[k], v[k], v[k + 1], wj, sd.angle);
+            for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<0>(O[k], v[k], v[k + 1], w[u], 0);
         }
     }
     if (col) {
@@ -379,17 +391,19 @@ __device__ __forceinline__ void deskew_radon_body(const SecDesc* __restrict__ se
     }
 }
 
+template <int kRows>
 __global__ __launch_bounds__(256) void k_deskew_radon(const SecDesc* __restrict__ secs,
                                                       const int* __restrict__ target,
                                                       const float* __restrict__ weight,
                                                       const uint32_t* __restrict__ fl, const float* __restrict__ q,
-                                                      int4 rlo, int4 rhi, float* __restrict__ acc, int dimx,
+                                                      int4 rlo, int4 rhi, int init, float* __restrict__ acc, int dimx,
                                                       int dimy) {
     const int t = blockIdx.z;
-    deskew_radon_body(secs, target, weight, fl, q, t, range_begin(t, rlo, rhi), range_end(t, rlo, rhi), acc, dimx,
-                      dimy);
+    deskew_radon_body<kRows>(secs, target, weight, fl, q, t, range_begin(t, rlo, rhi), range_end(t, rlo, rhi),
+                      (init >> t) & 1, acc, dimx, dimy);
 }
 
+template <int kRows>
 __global__ __launch_bounds__(256) void k_deskew_radon_parts(const SecDesc* __restrict__ secs,
                                                             const int* __restrict__ target,
                                                             const float* __restrict__ weight,
@@ -399,66 +413,53 @@ __global__ __launch_bounds__(256) void k_deskew_radon_parts(const SecDesc* __res
                                                             float* __restrict__ acc) {
     const DeskewPart& P = parts[blockIdx.z >> 2];
     const int t = blockIdx.z & 3;
-    deskew_radon_body(secs, target, weight, fl, q, t, P.range[2 * t], P.range[2 * t + 1], acc + P.acc_off, P.dimx,
-                      P.dimy);
+    deskew_radon_body<kRows>(secs, target, weight, fl, q, t, P.range[2 * t], P.range[2 * t + 1], (P.init >> t) & 1,
+                      acc + P.acc_off, P.dimx, P.dimy);
 }
 
-// 16 rows, one sector per pass: measured fastest on the batched viewshed
-// (129 VGPRs; 8 rows 1.2x, 4 rows 1.9x, 1 row 4.1x slower, 24 or 32 rows
-// 1.45x slower at 151 / 191 VGPRs; a second sector per pass only adds
-// registers).  The Radon deskew reads a short vector q per sector (L1/L2
-// resident), so its time is the chain of dependent table and tap reads over
-// the sectors: four sectors per pass.
-constexpr int kDeskewU = 1, kDeskewRadonU = 4;
-
-hipError_t launch_deskew(const DevPlan& p, const int range[8], const float* src, int source, int is_max,
+hipError_t launch_deskew(const DevPlan& p, const int range[8], const float* src, int source, int is_max, int init,
                          float* acc, int dimx, int dimy, long long img_acc, hipStream_t s) {
     const int dl = dimx > dimy ? dimx : dimy;
-    dim3 grid((dl + 255) / 256, (dl + kDeskewRows - 1) / kDeskewRows, 4);
     int4 lo = make_int4(range[0], range[1], range[2], range[3]);
     int4 hi = make_int4(range[4], range[5], range[6], range[7]);
     float* a = acc + img_acc;
-#define SKE_DESKEW(SRC, MX)                                                                                  \
-    hipLaunchKernelGGL((k_deskew<SRC, MX, kDeskewRows, kDeskewU>), grid, dim3(256), 0, s, p.secs, p.target, \
-                       p.weight, p.fl, src, lo, hi, a, dimx, dimy)
+    const unsigned gx = (unsigned)(dl + 255) / 256;
+#define SKE_DESKEW(SRC, MX, ROWS)                                                                                    \
+    hipLaunchKernelGGL((k_deskew<SRC, MX, ROWS>), dim3(gx, (unsigned)(dl + ROWS - 1) / ROWS, 4), dim3(256), 0, s,    \
+                       p.secs, p.target, p.weight, p.fl, src, lo, hi, init, a, dimx, dimy)
+#define SKE_DESKEW_RADON(ROWS)                                                                                         \
+    hipLaunchKernelGGL((k_deskew_radon<ROWS>), dim3(gx, (unsigned)(dl + ROWS - 1) / ROWS, 4), dim3(256), 0, s, p.secs, \
+                       p.target, p.weight, p.fl, src, lo, hi, init, a, dimx, dimy)
     if (source == kDeskewDense) {
-        if (is_max) SKE_DESKEW(kDeskewDense, 1); else SKE_DESKEW(kDeskewDense, 0);
+        if (is_max) SKE_DESKEW(kDeskewDense, 1, kDeskewRows); else SKE_DESKEW(kDeskewDense, 0, kDeskewRows);
     } else if (source == kDeskewArena) {
-        if (is_max) SKE_DESKEW(kDeskewArena, 1); else SKE_DESKEW(kDeskewArena, 0);
-    } else if ((size_t)grid.x * grid.y * grid.z >= 1024) {
-        hipLaunchKernelGGL(k_deskew_radon, grid, dim3(256), 0, s, p.secs, p.target, p.weight, p.fl, src, lo, hi, a,
-                           dimx, dimy);
+        if ((size_t)gx * ((dl + kDeskewRows - 1) / kDeskewRows) * 4 >= 1024) {
+            if (is_max) SKE_DESKEW(kDeskewArena, 1, kDeskewRows); else SKE_DESKEW(kDeskewArena, 0, kDeskewRows);
+        } else {
+            if (is_max) SKE_DESKEW(kDeskewArena, 1, kDeskewSmallRows); else SKE_DESKEW(kDeskewArena, 0, kDeskewSmallRows);
+        }
+    } else if ((size_t)gx * ((dl + kDeskewRows - 1) / kDeskewRows) * 4 >= 1024) {
+        SKE_DESKEW_RADON(kDeskewRows);
     } else {
-        hipLaunchKernelGGL((k_deskew<kDeskewRadon, 0, kDeskewRows, kDeskewRadonU>), grid, dim3(256), 0, s, p.secs,
-                           p.target, p.weight, p.fl, src, lo, hi, a, dimx, dimy);
+        SKE_DESKEW_RADON(kDeskewRadonRows);
     }
 #undef SKE_DESKEW
+#undef SKE_DESKEW_RADON
     return hipGetLastError();
 }
 
-hipError_t launch_deskew_parts(const DevPlan& p, const DeskewPart* parts, int nparts, int max_dim, const float* src,
-                               int source, int is_max, float* acc, hipStream_t s) {
+hipError_t launch_deskew_parts(const DevPlan& p, const DeskewPart* parts, int nparts, int max_dim, const float* q,
+                               float* acc, hipStream_t s) {
     if (nparts <= 0) return hipSuccess;
     if (nparts > 16383) return hipErrorInvalidValue;
-    dim3 grid((max_dim + 255) / 256, (max_dim + kDeskewRows - 1) / kDeskewRows, 4 * nparts);
-#define SKE_DESKEW_P(SRC, MX, U)                                                                                  \
-    hipLaunchKernelGGL((k_deskew_parts<SRC, MX, kDeskewRows, U>), grid, dim3(256), 0, s, p.secs, p.target, p.weight, \
-                       p.fl, src, parts, acc)
-    if (source == kDeskewArena) {
-        if (is_max) SKE_DESKEW_P(kDeskewArena, 1, kDeskewU); else SKE_DESKEW_P(kDeskewArena, 0, kDeskewU);
-    } else if (source == kDeskewRadon) {
-        // staged taps pay off with four or more workgroups per CU (a batch of
-        // images); a single small image runs its sector chains with four
-        // sectors' gathers in flight instead (one 512^2 image: 50 us against
-        // 87 us staged)
-        if ((size_t)grid.x * grid.y * grid.z >= 1024)
-            hipLaunchKernelGGL(k_deskew_radon_parts, grid, dim3(256), 0, s, p.secs, p.target, p.weight, p.fl, src,
-                               parts, acc);
-        else
-            SKE_DESKEW_P(kDeskewRadon, 0, kDeskewRadonU);
-    } else {
-        return hipErrorInvalidValue;  // the dense source has one image per call
-    }
+    const unsigned gx = (unsigned)(max_dim + 255) / 256, gz = 4u * (unsigned)nparts;
+#define SKE_DESKEW_P(ROWS)                                                                                             \
+    hipLaunchKernelGGL((k_deskew_radon_parts<ROWS>), dim3(gx, (unsigned)(max_dim + ROWS - 1) / ROWS, gz), dim3(256),   \
+                       0, s, p.secs, p.target, p.weight, p.fl, q, parts, acc)
+    if ((size_t)gx * gz * ((max_dim + kDeskewRows - 1) / kDeskewRows) >= 1024)
+        SKE_DESKEW_P(kDeskewRows);
+    else
+        SKE_DESKEW_P(kDeskewRadonRows);
 #undef SKE_DESKEW_P
     return hipGetLastError();
 }
@@ -466,11 +467,12 @@ hipError_t launch_deskew_parts(const DevPlan& p, const DeskewPart* parts, int np
 // ---------------------------------------------------------------------------
 // reduce (src/skewEngine.cuh:885-912).  out[i,j] (+)= o0[i,j], o1[cj,ci],
 // o2[j,ci], o3[i,cj] in that order.  o1/o2 are read through an LDS tile so
-// that their transposed accesses stay coalesced.
+// that their transposed accesses stay coalesced.  kInit: out starts from zero
+// (it is written, not read).
 // ---------------------------------------------------------------------------
-template <int kMax>
-__global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ acc, int4 present,
-                                                float* __restrict__ out, int dimx, int dimy) {
+template <int kMax, bool kInit>
+__device__ __forceinline__ void reduce_body(const float* __restrict__ acc, int4 present, float* __restrict__ out,
+                                            int dimx, int dimy) {
     __shared__ float t1[32][33];
     __shared__ float t2[32][33];
     const size_t N = (size_t)dimx * dimy;
@@ -479,9 +481,11 @@ __global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ acc, i
     const float* o2 = acc + 2 * N;
     const float* o3 = acc + 3 * N;
     const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
+    if (x0 >= dimx || y0 >= dimy) return;  // uniform: a smaller image of a batch
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     // o1 rows cj = dimx-1-j (j in [x0, x0+32)), columns ci = dimy-1-i;
     // o2 rows j, columns ci.  Load both tiles with ci along threadIdx.x.
+#pragma unroll
     for (int k = ty; k < 32; k += 8) {
         const int j = x0 + k;
         const int i = y0 + 31 - tx;  // ci = dimy-1-i runs forward with tx
@@ -492,11 +496,12 @@ __global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ acc, i
         }
     }
     __syncthreads();
+#pragma unroll
     for (int k = ty; k < 32; k += 8) {
         const int i = y0 + k, j = x0 + tx;
         if (i >= dimy || j >= dimx) continue;
         const size_t oi = (size_t)i * dimx + j;
-        float v = out[oi];
+        float v = kInit ? 0.0f : out[oi];
         const int cj = dimx - 1 - j;
         if (kMax) {
             if (present.x) { const float u = o0[oi]; v = (v > u) ? v : u; }
@@ -513,6 +518,26 @@ __global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ acc, i
     }
 }
 
+template <int kMax>
+__global__ __launch_bounds__(256) void k_reduce(const float* __restrict__ acc, int4 present,
+                                                float* __restrict__ out, int dimx, int dimy) {
+    reduce_body<kMax, false>(acc, present, out, dimx, dimy);
+}
+
+// Up to kReduceImages images of an engine or batch in one launch (blockIdx.z),
+// written from zero: 16 maps of 512^2 in 16 us (16 launches of 7 us and a fill
+// of 10 us before).
+constexpr int kReduceImages = 64;
+struct ReduceGroup {
+    ReduceImage im[kReduceImages];  // 1.5 KB of kernel arguments
+};
+template <int kMax>
+__global__ __launch_bounds__(256) void k_reduce_images(const float* __restrict__ acc, int4 present,
+                                                       float* __restrict__ out, ReduceGroup g) {
+    const ReduceImage im = g.im[blockIdx.z];
+    reduce_body<kMax, true>(acc + im.acc_off, present, out + im.out_off, im.n, im.n);
+}
+
 hipError_t launch_reduce(const float* acc, const int present[4], float* out, int dimx, int dimy, int is_max,
                          hipStream_t s) {
     dim3 grid((dimx + 31) / 32, (dimy + 31) / 32);
@@ -521,6 +546,26 @@ hipError_t launch_reduce(const float* acc, const int present[4], float* out, int
         hipLaunchKernelGGL(k_reduce<1>, grid, dim3(256), 0, s, acc, pr, out, dimx, dimy);
     else
         hipLaunchKernelGGL(k_reduce<0>, grid, dim3(256), 0, s, acc, pr, out, dimx, dimy);
+    return hipGetLastError();
+}
+
+hipError_t launch_reduce_images(const float* acc, const int present[4], float* out, const ReduceImage* imgs, int count,
+                                int is_max, hipStream_t s) {
+    const int4 pr = make_int4(present[0], present[1], present[2], present[3]);
+    for (int first = 0; first < count; first += kReduceImages) {
+        ReduceGroup g{};
+        const int m = count - first < kReduceImages ? count - first : kReduceImages;
+        int side = 1;
+        for (int i = 0; i < m; ++i) {
+            g.im[i] = imgs[first + i];
+            side = g.im[i].n > side ? g.im[i].n : side;
+        }
+        const dim3 grid((unsigned)(side + 31) / 32, (unsigned)(side + 31) / 32, (unsigned)m);
+        if (is_max)
+            hipLaunchKernelGGL(k_reduce_images<1>, grid, dim3(256), 0, s, acc, pr, out, g);
+        else
+            hipLaunchKernelGGL(k_reduce_images<0>, grid, dim3(256), 0, s, acc, pr, out, g);
+    }
     return hipGetLastError();
 }
 

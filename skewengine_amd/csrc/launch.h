@@ -85,18 +85,24 @@ hipError_t launch_radn_smear(const DevPlan& p, const float* q, float* SO, hipStr
 // Deskew sectors [first of each type ... ] of a plan into the four
 // orientation accumulators acc[4*N] (src/skewEngine.cuh:755-793), in
 // ascending sector order per orientation.  range[t] = {begin, end} indices
-// into p.secs of the sectors of type t.
+// into p.secs of the sectors of type t; bit t of `init` starts accumulator t
+// from zero instead of its contents.
 hipError_t launch_deskew(const DevPlan& p, const int range[8], const float* src, int source,
-                         int is_max, float* acc, int dimx, int dimy, long long img_acc,
+                         int is_max, int init, float* acc, int dimx, int dimy, long long img_acc,
                          hipStream_t s);
-// The same for every image of a chunk in one launch: parts[k] holds image k's
-// sector ranges, accumulator offset and sides (max_dim: the largest side).
-hipError_t launch_deskew_parts(const DevPlan& p, const DeskewPart* parts, int nparts, int max_dim, const float* src,
-                               int source, int is_max, float* acc, hipStream_t s);
+// The same for the Radon source and every image of a chunk in one launch:
+// parts[k] holds image k's sector ranges, accumulator offset and sides
+// (max_dim: the largest side).
+hipError_t launch_deskew_parts(const DevPlan& p, const DeskewPart* parts, int nparts, int max_dim, const float* q,
+                               float* acc, hipStream_t s);
 
 // reduce(): out (+)= o0, o1, o2, o3 with the inverse orientation maps
 // (src/skewEngine.cuh:885-912).  present[t] == 0 skips buffer t.
 hipError_t launch_reduce(const float* acc, const int present[4], float* out, int dimx, int dimy,
                          int is_max, hipStream_t s);
+// out = o0 + o1 + o2 + o3 (or their maximum with zero) of `count` images, many
+// to a launch; imgs in host memory.
+hipError_t launch_reduce_images(const float* acc, const int present[4], float* out, const ReduceImage* imgs, int count,
+                                int is_max, hipStream_t s);
 
 }  // namespace ske

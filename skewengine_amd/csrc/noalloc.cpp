@@ -285,7 +285,7 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
             SKE_HIP(launch_op_unit(v, in4, nullptr, arena, stream));
             break;
         }
-        SKE_HIP(launch_deskew(v, ch.range, radon ? q : arena, radon ? kDeskewRadon : kDeskewArena, is_max, acc, n, n,
+        SKE_HIP(launch_deskew(v, ch.range, radon ? q : arena, radon ? kDeskewRadon : kDeskewArena, is_max, 0, acc, n, n,
                               0, stream));
     }
     SKE_HIP(launch_fill_f32(d_output, N, 0.0f, stream));

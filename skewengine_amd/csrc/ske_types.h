@@ -45,12 +45,24 @@ struct SecDesc {
 
 // One image of a chunk for the deskew: its sector range of orientation t
 // ([range[2t], range[2t+1]) indices into the chunk's sectors), the element
-// offset of its four accumulators and its sides.
+// offset of its four accumulators and its sides; bit t of init: the part holds
+// the run's first sectors of orientation t, whose accumulator starts from zero.
 struct DeskewPart {
     int range[8];
     long long acc_off;
     int dimx;
     int dimy;
+    int init;
+    int pad0;
+};
+
+// One image of a reduce over several: its side and the element offsets of its
+// accumulators and output.
+struct ReduceImage {
+    long long acc_off;
+    long long out_off;
+    int n;
+    int pad0;
 };
 
 // One row of one sector: the unit of work of the row kernels.
