@@ -145,13 +145,28 @@ __device__ __forceinline__ double rowsum_cols_walk(const int* __restrict__ tt, c
     return acc;
 }
 
-__global__ __launch_bounds__(256) void k_radn_rowsum_cols(const SecDesc* __restrict__ secs,
+//
+// Bound by latency: the 64 lanes' taps are one partner row, and an L2 miss in
+// any of a pass's eight rows stalls the wave.  Workgroups go to the eight XCDs
+// in turn, so runs of 23 sectors (an image's 180 over all eight; nearly always
+// one partner copy) are laid on one XCD, whose L2 then serves them: 8 x 955^2
+// passes 1,498 -> 855 us.  A workgroup is one wave: rows of a sector differ in
+// length by up to 8 times, and waves that share a workgroup leave their slots
+// to the next one only together.  16 x 512^2: 500 -> 387 us for both.  Not
+// faster: scalar offsets with two or three taps per load (unaligned wide
+// loads), passes in flight from tables held in lanes (540 to 670 us).
+constexpr int kXcdSectors = 23, kRowsumWaves = 1;
+__global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const SecDesc* __restrict__ secs,
                                                           const float* __restrict__ in4,
                                                           const int* __restrict__ target,
                                                           const float* __restrict__ weight,
-                                                          const uint32_t* __restrict__ fl, double* __restrict__ P) {
-    const SecDesc sd = secs[blockIdx.y];
-    const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 64;
+                                                          const uint32_t* __restrict__ fl, double* __restrict__ P,
+                                                          int nsec, int nblk) {
+    const int at = blockIdx.x >> 3, k = at / nblk;
+    const int si = (k / kXcdSectors * 8 + (blockIdx.x & 7)) * kXcdSectors + k % kXcdSectors;
+    if (si >= nsec) return;
+    const SecDesc sd = secs[si];
+    const int r0 = ((at - k * nblk) * kRowsumWaves + (threadIdx.x >> 6)) * 64;
     if (r0 >= sd.H) return;  // wave-uniform
     const int lane = threadIdx.x & 63;
     const int r = r0 + lane;
@@ -201,8 +216,10 @@ __global__ __launch_bounds__(256) void k_radn_rowsum_cols(const SecDesc* __restr
 hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* Sbuf, double* P, hipStream_t s) {
     if (!Sbuf) {  // writes every row r < H of every sector (rows without cells: 0)
         if (p.nsec == 0 || p.maxH <= 0) return hipSuccess;
-        hipLaunchKernelGGL(k_radn_rowsum_cols, dim3((p.maxH + 255) / 256, p.nsec), dim3(256), 0, s, p.secs, in4,
-                           p.target, p.weight, p.fl, P);
+        const int nblk = (p.maxH + 64 * kRowsumWaves - 1) / (64 * kRowsumWaves);
+        const unsigned units = (unsigned)(p.nsec + 8 * kXcdSectors - 1) / (8 * kXcdSectors);
+        hipLaunchKernelGGL(k_radn_rowsum_cols, dim3(8 * kXcdSectors * units * nblk), dim3(64 * kRowsumWaves), 0, s, p.secs,
+                           in4, p.target, p.weight, p.fl, P, p.nsec, nblk);
         return hipGetLastError();
     }
     if (p.nwork == 0) return hipSuccess;  // writes the rows of the work list only: P zeroed by the caller
@@ -211,77 +228,132 @@ hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* S
     return hipGetLastError();
 }
 
-// One DIF pass over re/im in LDS (src/helper.h:65-82) followed by the
-// bit-reversal permutation (:84-100).
-__device__ void lds_fft(double* re, double* im, int N, int m, const double2* __restrict__ tw) {
-    for (int n = N; n > 1; n >>= 1) {
-        const int k = n >> 1;
-        const double2* T = tw + (N - n);
-        for (int beta = threadIdx.x; beta < (N >> 1); beta += blockDim.x) {
+// The DIF stages of a transform over re/im in LDS (src/helper.h:65-82), two a
+// pass: a thread takes the four points l, l + n/4, l + n/2, l + 3n/4 of a block
+// of n through the stages n and n/2 in registers (the same butterflies and
+// twiddles, half the LDS passes and barriers).  The result stands in
+// bit-reversed order; the caller reads it there.  kPad: one double of padding
+// per 16, which spreads the power-of-two strides over the banks.
+template <bool kPad>
+__device__ __forceinline__ int fft_at(int i) { return kPad ? i + (i >> 4) : i; }
+
+struct Cplx {
+    double r, i;
+};
+__device__ __forceinline__ void dif_butterfly(Cplx& a, Cplx& b, double2 t) {
+    const double tr = a.r - b.r, ti = a.i - b.i;
+    a.r = a.r + b.r;
+    a.i = a.i + b.i;
+    b.r = tr * t.x - ti * t.y;
+    b.i = tr * t.y + ti * t.x;
+}
+
+template <bool kPad>
+__device__ void lds_fft(double* re, double* im, int N, const double2* __restrict__ tw) {
+    int n = N;
+    for (; n > 2; n >>= 2) {
+        const int k = n >> 2, sh = __ffs(k) - 1;
+        const double2* T = tw + (N - n);             // stage n: entries 0 .. n/2 - 1
+        const double2* T2 = tw + (N - (n >> 1));     // stage n/2
+        for (int beta = threadIdx.x; beta < (N >> 2); beta += blockDim.x) {
             const int l = beta & (k - 1);
-            const int a = (beta >> (__ffs(k) - 1)) * n + l;  // (beta / k) * n + l
-            const int b = a + k;
-            const double2 t = T[l];
-            const double tr = re[a] - re[b], ti = im[a] - im[b];
-            re[a] = re[a] + re[b];
-            im[a] = im[a] + im[b];
-            re[b] = tr * t.x - ti * t.y;
-            im[b] = tr * t.y + ti * t.x;
+            const int a = ((beta >> sh) << (sh + 2)) + l;
+            const int p0 = fft_at<kPad>(a), p1 = fft_at<kPad>(a + k), p2 = fft_at<kPad>(a + 2 * k),
+                      p3 = fft_at<kPad>(a + 3 * k);
+            Cplx x0{re[p0], im[p0]}, x1{re[p1], im[p1]}, x2{re[p2], im[p2]}, x3{re[p3], im[p3]};
+            const double2 ta = T[l], tb = T[l + k], tc = T2[l];
+            dif_butterfly(x0, x2, ta);
+            dif_butterfly(x1, x3, tb);
+            dif_butterfly(x0, x1, tc);
+            dif_butterfly(x2, x3, tc);
+            re[p0] = x0.r, im[p0] = x0.i;
+            re[p1] = x1.r, im[p1] = x1.i;
+            re[p2] = x2.r, im[p2] = x2.i;
+            re[p3] = x3.r, im[p3] = x3.i;
         }
         __syncthreads();
     }
-    for (int a = threadIdx.x; a < N; a += blockDim.x) {
-        const int b = (int)(__brev((unsigned)a) >> (32 - m));
-        if (b > a) {
-            double t = re[a]; re[a] = re[b]; re[b] = t;
-            t = im[a]; im[a] = im[b]; im[b] = t;
+    if (n == 2) {
+        const double2 t = tw[N - 2];
+        for (int beta = threadIdx.x; beta < (N >> 1); beta += blockDim.x) {
+            const int p0 = fft_at<kPad>(2 * beta), p1 = fft_at<kPad>(2 * beta + 1);
+            Cplx x0{re[p0], im[p0]}, x1{re[p1], im[p1]};
+            dif_butterfly(x0, x1, t);
+            re[p0] = x0.r, im[p0] = x0.i;
+            re[p1] = x1.r, im[p1] = x1.i;
         }
+        __syncthreads();
     }
-    __syncthreads();
 }
 
+// Between the transforms the ramp reads the spectrum from its bit-reversed
+// places, into registers (16 values a thread at most: H2 <= 4096), and writes
+// it in order for the second transform; the result is read bit-reversed too.
+// Bound by LDS passes and their barriers (two radix-2 stages a pass, no
+// permutation passes: 2,880 sectors of 512^2 slices 69 -> FFTIME us).
+template <bool kPad>
 __global__ __launch_bounds__(256) void k_radn_filter(const SecDesc* __restrict__ secs, const double* __restrict__ P,
                                                      float* __restrict__ q, const double2* __restrict__ tw,
-                                                     const int* __restrict__ tw_off) {
+                                                     const int* __restrict__ tw_off, int maxH2) {
     extern __shared__ double buf[];
-    const SecDesc sd = secs[blockIdx.x];
+    const SecDesc& sd = secs[blockIdx.x];
     const int H = sd.H;
     const int m = (H <= 1) ? 0 : 32 - __clz(H - 1);  // H2 = 2^ceil(log2 H)
     const int H2 = 1 << m;
     double* re = buf;
-    double* im = buf + H2;
+    double* im = buf + fft_at<kPad>(maxH2);
     for (int i = threadIdx.x; i < H2; i += blockDim.x) {
-        re[i] = (i < H) ? P[sd.q + i] : 0.0;
-        im[i] = 0.0;
+        re[fft_at<kPad>(i)] = (i < H) ? P[sd.q + i] : 0.0;
+        im[fft_at<kPad>(i)] = 0.0;
     }
     __syncthreads();
-    if (H2 > 1) lds_fft(re, im, H2, m, tw + tw_off[m]);
+    const double2* T = tw + tw_off[m];
+    auto rev = [&](int i) { return fft_at<kPad>(m ? (int)(__brev((unsigned)i) >> (32 - m)) : 0); };
+    if (H2 > 1) lds_fft<kPad>(re, im, H2, T);
     // ramp: zero above H/2, gain (double)i/H below (kernelRADN.h:247);
     // then the conj of ifft's first step.
-    for (int i = threadIdx.x; i < H2; i += blockDim.x) {
-        if (i > H / 2) {
-            re[i] = 0.0;
-            im[i] = -0.0;
-        } else {
+    constexpr int kPer = (1 << 12) / 256;
+    Cplx x[kPer];
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+        const int i = threadIdx.x + 256 * e;
+        x[e] = Cplx{0.0, -0.0};
+        if (i < H2 && i <= H / 2) {
             const double g = (double)i / H;
-            re[i] = g * re[i];
-            im[i] = -(g * im[i]);
+            x[e].r = g * re[rev(i)];
+            x[e].i = -(g * im[rev(i)]);
         }
     }
     __syncthreads();
-    if (H2 > 1) lds_fft(re, im, H2, m, tw + tw_off[m]);
+#pragma unroll
+    for (int e = 0; e < kPer; e++) {
+        const int i = threadIdx.x + 256 * e;
+        if (i < H2) {
+            re[fft_at<kPad>(i)] = x[e].r;
+            im[fft_at<kPad>(i)] = x[e].i;
+        }
+    }
+    __syncthreads();
+    if (H2 > 1) lds_fft<kPad>(re, im, H2, T);
     for (int i = threadIdx.x; i < H; i += blockDim.x) {
-        const double x = re[i] / H2;
-        q[sd.q + i] = (float)(0.0 + x);  // skewOutput (zero) += Re
+        const double v = re[rev(i)] / H2;
+        q[sd.q + i] = (float)(0.0 + v);  // skewOutput (zero) += Re
     }
 }
 
 hipError_t launch_radn_filter(const DevPlan& p, const double* P, float* q, const double* tw, const int* tw_off,
                               int maxH2, hipStream_t s) {
     if (p.nsec == 0) return hipSuccess;
-    const size_t lds = sizeof(double) * 2 * (size_t)maxH2;
-    hipLaunchKernelGGL(k_radn_filter, dim3(p.nsec), dim3(256), lds, s, p.secs, P, q,
-                       reinterpret_cast<const double2*>(tw), tw_off);
+    // padded up to 2048 points (35 KB); 4096 points take 64 KB unpadded
+    if (maxH2 <= 2048) {
+        const size_t lds = sizeof(double) * 2 * (size_t)(maxH2 + maxH2 / 16 + 1);
+        hipLaunchKernelGGL(k_radn_filter<true>, dim3(p.nsec), dim3(256), lds, s, p.secs, P, q,
+                           reinterpret_cast<const double2*>(tw), tw_off, maxH2);
+    } else {
+        const size_t lds = sizeof(double) * 2 * (size_t)maxH2;
+        hipLaunchKernelGGL(k_radn_filter<false>, dim3(p.nsec), dim3(256), lds, s, p.secs, P, q,
+                           reinterpret_cast<const double2*>(tw), tw_off, maxH2);
+    }
     return hipGetLastError();
 }
 

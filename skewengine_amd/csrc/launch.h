@@ -62,7 +62,7 @@ hipError_t launch_op_blur(const DevPlan& p, const float* in4, const float* Sbuf,
                           const double* tab, hipStream_t s);
 hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* Sbuf, double* P,
                               hipStream_t s);
-// Per-sector ramp filter of the row sums in LDS (FFT length H2 <= 2^15).
+// Per-sector ramp filter of the row sums in LDS (FFT length H2 <= 4096).
 hipError_t launch_radn_filter(const DevPlan& p, const double* P, float* q, const double* tw,
                               const int* tw_off, int maxH2, hipStream_t s);
 
