@@ -20,6 +20,8 @@
 // rounds to exactly RN(a/d): two VALU operations instead of the ~10 of the
 // IEEE divide sequence.  The tests check both variants against each other
 // and against the oracle.
+#include <float.h>
+
 #include <algorithm>
 
 #include "device_common.h"
@@ -45,6 +47,47 @@ __device__ __forceinline__ void sdem_step(float sk, float h, const float4 t, flo
     cv = closing ? cv + (t.w - od2) : cv;    // cv += d*d - od*od
 }
 
+// Chunk c of 64 observers: every step of both scans.
+template <int kVariant>
+__device__ __forceinline__ void sdem_steps_chunk(const float* row, int L, int c, float povh,
+                                                 const float4* __restrict__ rtab, float* __restrict__ so, float R) {
+    const int lane = threadIdx.x & 63;
+    const int j0 = c << 6;
+    const int jj = j0 + lane;
+    const bool valid = jj < L;
+    const float h = row[jj] + povh;
+    float cv = 0.0f;
+    {   // right scan: k = j+1 .. last-1
+        float M = -2000.0f, od2 = 0.0f;
+        bool vis = true;
+        const int myR = valid ? (L - 1 - jj) : 0;
+        const int dall = L - 1 - (j0 + 63);  // every lane active up to here
+        const int dmax = L - 1 - j0;
+        int d = 1;
+        for (; d <= dall; ++d) sdem_step<kVariant>(row[jj + d], h, rtab[d], M, od2, vis, cv);
+        for (; d <= dmax; ++d) {
+            const float4 t = rtab[d];
+            const float sk = row[jj + d];
+            if (d <= myR) sdem_step<kVariant>(sk, h, t, M, od2, vis, cv);
+        }
+    }
+    {   // left scan: k = j-1 .. first
+        float M = -2000.0f, od2 = 0.0f;
+        bool vis = true;
+        const int myL = valid ? jj : 0;
+        const int dall = (j0 + 63 < L) ? j0 : -1;
+        const int dmax = (j0 + 63 < L) ? (j0 + 63) : (L - 1);
+        int d = 1;
+        for (; d <= dall; ++d) sdem_step<kVariant>(row[jj - d], h, rtab[d], M, od2, vis, cv);
+        for (; d <= dmax; ++d) {
+            const float4 t = rtab[d];
+            const float sk = row[jj - d];
+            if (d <= myL) sdem_step<kVariant>(sk, h, t, M, od2, vis, cv);
+        }
+    }
+    if (valid) so[jj] = cv * R;
+}
+
 template <int kVariant>
 __global__ __launch_bounds__(256) void k_op_sdem(const SecDesc* __restrict__ secs,
                                                  const RowWork* __restrict__ work,
@@ -67,46 +110,9 @@ __global__ __launch_bounds__(256) void k_op_sdem(const SecDesc* __restrict__ sec
     stage_row(row, sd, r, f, L, in4, target, weight, Sbuf);
     __syncthreads();
 
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
     const int nchunk = (L + 63) >> 6;
     float* so = arena + sd.so + (size_t)r * sd.dim_i + f;
-    for (int c = wave; c < nchunk; c += 4) {
-        const int j0 = c << 6;
-        const int jj = j0 + lane;
-        const bool valid = jj < L;
-        const float h = row[jj] + povh;
-        float cv = 0.0f;
-        {   // right scan: k = j+1 .. last-1
-            float M = -2000.0f, od2 = 0.0f;
-            bool vis = true;
-            const int myR = valid ? (L - 1 - jj) : 0;
-            const int dall = L - 1 - (j0 + 63);  // every lane active up to here
-            const int dmax = L - 1 - j0;
-            int d = 1;
-            for (; d <= dall; ++d) sdem_step<kVariant>(row[jj + d], h, rtab[d], M, od2, vis, cv);
-            for (; d <= dmax; ++d) {
-                const float4 t = rtab[d];
-                const float sk = row[jj + d];
-                if (d <= myR) sdem_step<kVariant>(sk, h, t, M, od2, vis, cv);
-            }
-        }
-        {   // left scan: k = j-1 .. first
-            float M = -2000.0f, od2 = 0.0f;
-            bool vis = true;
-            const int myL = valid ? jj : 0;
-            const int dall = (j0 + 63 < L) ? j0 : -1;
-            const int dmax = (j0 + 63 < L) ? (j0 + 63) : (L - 1);
-            int d = 1;
-            for (; d <= dall; ++d) sdem_step<kVariant>(row[jj - d], h, rtab[d], M, od2, vis, cv);
-            for (; d <= dmax; ++d) {
-                const float4 t = rtab[d];
-                const float sk = row[jj - d];
-                if (d <= myL) sdem_step<kVariant>(sk, h, t, M, od2, vis, cv);
-            }
-        }
-        if (valid) so[jj] = cv * sd.R;
-    }
+    for (int c = threadIdx.x >> 6; c < nchunk; c += 4) sdem_steps_chunk<kVariant>(row, L, c, povh, rtab, so, sd.R);
 }
 
 // ---------------------------------------------------------------------------
@@ -131,21 +137,27 @@ __global__ __launch_bounds__(256) void k_op_sdem(const SecDesc* __restrict__ sec
 // run to its first lane's row end, up to 95 cells past the row (128); with
 // lane compaction a block only runs while some lane's row continues, so
 // every read stays within 32 cells of the row (and of the safe positions).
-template <int kG>
-constexpr int pad_bits() { return kG > 1 ? 32 : 128; }
-constexpr int kChunksMax = 128;  // 32-cell chunks of a row of <= 4096 cells
+// Long rows may also take the per-step scans (kPad).
+template <int kG, bool kLong = false>
+constexpr int pad_bits() { return kLong ? kPad : kG > 1 ? 32 : 128; }
+// 32-cell chunks of a row of <= 4096 cells, and of the longest (16,000 cells).
+constexpr int kChunksMax = 128, kChunksLong = 512;
 // Chunk-maximum tables of a staged row, each indexed by chunk c in
-// [-kTabLo, kChunksMax + kTabHi): level 0 cm[c] = max row[32c .. 32c+31],
+// [-kTabLo, kCh + kTabHi): level 0 cm[c] = max row[32c .. 32c+31],
 // level 1..3 the maxima of 2, 4 and 8 consecutive chunks starting at c,
 // then suffix and prefix maxima.  Chunks outside the row hold -inf (the
 // prefix table repeats the row maximum past the end).
 constexpr int kTabLo = 16, kTabHi = 16;
-constexpr int kTabN = kTabLo + kChunksMax + kTabHi;
+template <int kCh>
+constexpr int tab_n() { return kTabLo + kCh + kTabHi; }
 enum { kTabL0 = 0, kTabL1 = 1, kTabL2 = 2, kTabL3 = 3, kTabSuf = 4, kTabPre = 5, kTabs = 6 };
 
 // LDS of the bit-block kernels: guard band, row, guard band, chunk tables.
 inline size_t sdem_bits_lds(int maxL, int group = 1) {
-    return sizeof(float) * ((size_t)maxL + 2 * (group > 1 ? pad_bits<4>() : pad_bits<1>()) + kTabs * kTabN);
+    return sizeof(float) * ((size_t)maxL + 2 * (group > 1 ? pad_bits<4>() : pad_bits<1>()) + kTabs * tab_n<kChunksMax>());
+}
+inline size_t sdem_long_lds(int maxL) {
+    return sizeof(float) * ((size_t)maxL + 2 * pad_bits<4, true>() + kTabs * tab_n<kChunksLong>());
 }
 
 __device__ __forceinline__ int lshl1_add(int a, int b) {
@@ -170,6 +182,37 @@ __device__ __forceinline__ void flush_block(uint32_t w, int d0, int& A, int& s) 
     uint32_t f;
     asm("v_ffbl_b32 %0, %1" : "=v"(f) : "v"(~w));
     s = max(s, (int)__builtin_elementwise_sub_sat((uint32_t)(d0 + 33), f));
+}
+
+// Rows past 4096 cells: the sums pass 2^24, so the float additions round and
+// their order counts.  cv then takes the closed runs of a block one by one, as
+// the reference does (a few per lane and block; none in most blocks).  cv holds
+// the sum; s the open run's d_o^2 with the flag of the last step as its sign.
+// A run in progress at the end of the row adds nothing; steps past the row end
+// are recorded as visible and close none.
+__device__ __forceinline__ float square(int d) {
+#pragma clang fp contract(off)
+    return (float)d * (float)d;
+}
+__device__ __forceinline__ float add_run(float cv, int dc, float od2) {
+#pragma clang fp contract(off)
+    return cv + (square(dc) - od2);  // cv += d*d - od*od
+}
+__device__ __forceinline__ void flush_runs(uint32_t w, int d0, bool live, int& A, int& s) {
+    const uint32_t prev = (w >> 1) | ((uint32_t)s & 0x80000000u);  // each step's predecessor
+    const uint32_t open = w & ~prev;
+    uint32_t close = live ? prev & ~w : 0u;
+    float cv = __int_as_float(A), od2 = __int_as_float(s & 0x7FFFFFFF);
+    while (close) {
+        const int p = __clz(close);  // step d0 + 1 + p
+        const uint32_t before = open & ~(0xFFFFFFFFu >> p);
+        if (before) od2 = square(d0 + 33 - __ffs(before));
+        cv = add_run(cv, d0 + 1 + p, od2);
+        close &= ~(0x80000000u >> p);
+    }
+    if (open) od2 = square(d0 + 33 - __ffs(open));
+    A = __float_as_int(cv);
+    s = (int)(__float_as_uint(od2) | (w << 31));
 }
 
 // The visibility flag is the sign of t = M - q: rounding preserves the sign
@@ -237,9 +280,12 @@ __device__ __forceinline__ uint32_t scan_half(const float* rowj, float h, const 
 // kClamp: clamp the nearest-target position into the row (callers whose
 // lanes may lie far past their row end); without it p must lie in
 // [-32, L + 31], which the chunk tables' padding covers.
-template <int kDir, bool kClamp = true>
+// kCh > kChunksMax: distances are cut to L in the reciprocal table, which ends
+// 32 entries past the longest row; a segment that starts past L holds no target.
+template <int kDir, bool kClamp = true, int kCh = kChunksMax>
 __device__ __forceinline__ float exit_bound(const float* __restrict__ tab, int jj, int L, float h, int db,
                                             const float2* __restrict__ ytab, float invL) {
+    constexpr int kTabN = tab_n<kCh>();
     const int e = db + 1;
     int p = jj + kDir * e;  // nearest remaining target
     if (kClamp) p = p < 0 ? 0 : (p > L - 1 ? L - 1 : p);
@@ -258,7 +304,8 @@ __device__ __forceinline__ float exit_bound(const float* __restrict__ tab, int j
     }
     const float a1 = s1 - h, a2 = s2 - h, a3 = s3 - h, a4 = s4 - h;
     const float amax = fmaxf(fmaxf(a1, a2), fmaxf(a3, a4));
-    float b = fmaxf(fmaxf(a1 * ytab[e].x, a2 * ytab[e + 32].x), fmaxf(a3 * ytab[e + 96].x, a4 * ytab[e + 224].x));
+    auto y = [&](int d) { return ytab[kCh > kChunksMax ? min(d, L) : d].x; };
+    float b = fmaxf(fmaxf(a1 * y(e), a2 * y(e + 32)), fmaxf(a3 * y(e + 96), a4 * y(e + 224)));
     b = fmaxf(b, amax * invL);
     return __builtin_fmaf(fabsf(b), 9.5367431640625e-7f, b);  // b + |b| 2^-20
 }
@@ -293,10 +340,11 @@ __device__ __forceinline__ int scan_dir(const float* rowj, float h, const float4
     return myLen > d0 ? A : A - ((d0 + 1) * (d0 + 1) - s * s);
 }
 
-// Build the chunk tables of a staged row of L <= 4096 cells (see kTabN).
+// Build the chunk tables of a staged row of L <= 32 kCh cells (see tab_n).
 // Ends with a barrier.
-template <int kWaves>
+template <int kWaves, int kCh>
 __device__ __forceinline__ void row_tables(const float* row, int L, float* tab) {
+    constexpr int kTabN = tab_n<kCh>(), kPer = kCh / 64;
     const int nch = (L + 31) >> 5;
     float* t0 = tab + kTabLo;
     for (int i = threadIdx.x; i < kTabs * kTabN; i += 64 * kWaves) tab[i] = -INFINITY;
@@ -309,10 +357,15 @@ __device__ __forceinline__ void row_tables(const float* row, int L, float* tab) 
         if ((t & 31) == 0 && t < nch * 32) t0[kTabL0 * kTabN + (t >> 5)] = v;
     }
     __syncthreads();
-    if (threadIdx.x < 64) {  // one wave: suffix and prefix maxima, two chunks per lane
+    if (threadIdx.x < 64) {  // one wave: suffix and prefix maxima, kPer chunks per lane
         const int l = threadIdx.x;
-        const float x0 = t0[kTabL0 * kTabN + 2 * l], x1 = t0[kTabL0 * kTabN + 2 * l + 1];  // -inf past nch
-        float vs = fmaxf(x0, x1), vp = vs;
+        float x[kPer];  // -inf past nch
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) x[i] = t0[kTabL0 * kTabN + kPer * l + i];
+        float vs = x[0];
+#pragma unroll
+        for (int i = 1; i < kPer; ++i) vs = fmaxf(vs, x[i]);
+        float vp = vs;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
             const float us = __shfl_down(vs, o), up = __shfl_up(vp, o);  // own value when out of range
@@ -322,12 +375,17 @@ __device__ __forceinline__ void row_tables(const float* row, int L, float* tab) 
         float ns = __shfl_down(vs, 1), np = __shfl_up(vp, 1);
         if (l == 63) ns = -INFINITY;
         if (l == 0) np = -INFINITY;
-        const float s1 = fmaxf(x1, ns), p0 = fmaxf(x0, np), p1 = fmaxf(x1, p0);
-        t0[kTabSuf * kTabN + 2 * l] = fmaxf(x0, s1);
-        t0[kTabSuf * kTabN + 2 * l + 1] = s1;
-        t0[kTabPre * kTabN + 2 * l] = p0;
-        t0[kTabPre * kTabN + 2 * l + 1] = p1;
-        if (l < kTabHi) t0[kTabPre * kTabN + kChunksMax + l] = __shfl(p1, 63);  // whole-row maximum
+#pragma unroll
+        for (int i = kPer - 1; i >= 0; --i) {
+            ns = fmaxf(x[i], ns);
+            t0[kTabSuf * kTabN + kPer * l + i] = ns;
+        }
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            np = fmaxf(x[i], np);
+            t0[kTabPre * kTabN + kPer * l + i] = np;
+        }
+        if (l < kTabHi) t0[kTabPre * kTabN + kCh + l] = __shfl(np, 63);  // whole-row maximum
     }
     for (int lev = 1; lev <= 3; ++lev) {  // level lev from level lev-1: max of two runs 2^(lev-1) apart
         const int off = 1 << (lev - 1);
@@ -379,11 +437,15 @@ __device__ __forceinline__ int nth_set_bit(uint64_t m, int r) {
     return pos;
 }
 
-template <int kDir, int kG>
+template <int kDir, int kG, bool kLong>
 __device__ __forceinline__ void scan_group(const float* row, int L, float povh, int c0, int nck,
                                            const float* __restrict__ tab, const float4* __restrict__ rtab,
                                            float* __restrict__ so, float R, int& nblk) {
     const float2* __restrict__ ytab = reinterpret_cast<const float2*>(rtab + kMaxDim + 1);
+    constexpr int kCh = kLong ? kChunksLong : kChunksMax;
+    // a scan's first state: A counts the observer's own cell; long rows go on
+    // with the right scan's sum, visible from d = 0
+    constexpr int kA0 = kLong ? 0 : 1, kS0 = kLong ? (int)0x80000000 : 0;
     int* __restrict__ soi = reinterpret_cast<int*>(so);
     const float invL = ytab[L].x;
     const int lane = threadIdx.x & 63;
@@ -400,15 +462,15 @@ __device__ __forceinline__ void scan_group(const float* row, int L, float povh, 
             if (kDir > 0)
                 soi[j] = 0;
             else
-                so[j] = (float)soi[j] * R;
+                so[j] = (kLong ? so[j] : (float)soi[j]) * R;
         }
         const bool a = in && myLen > 0;
         act[k] = __builtin_amdgcn_ballot_w64(a);
         jj[k] = a ? j : safe;
         h[k] = row[jj[k]] + povh;
         M[k] = -2000.0f;
-        A[k] = 1;
-        s[k] = 0;
+        A[k] = kLong && kDir < 0 && a ? soi[j] : kA0;
+        s[k] = kS0;
     }
     int ns = nck;
     for (int d0 = 0; ns > 0; d0 += 32) {
@@ -433,7 +495,10 @@ __device__ __forceinline__ void scan_group(const float* row, int L, float povh, 
                     w |= (1u << e) - 1u;
                     ends = true;
                 }
-                flush_block(w, d0, A[k], s[k]);
+                if (kLong)
+                    flush_runs(w, d0, (act[k] >> lane) & 1, A[k], s[k]);
+                else
+                    flush_block(w, d0, A[k], s[k]);
             }
         }
         const int db = d0 + 32;
@@ -453,8 +518,15 @@ __device__ __forceinline__ void scan_group(const float* row, int L, float povh, 
                 const int myLen = kDir > 0 ? L - 1 - jj[k] : jj[k];
                 bool done = myLen <= db;
                 // active lanes and empty lanes (jj = safe) keep the bound's table reads in range
-                if (tb) done = done | (exit_bound<kDir, false>(tab, jj[k], L, h[k], db, ytab, invL) <= M[k]);
-                if (a && done) {
+                if (tb) done = done | (exit_bound<kDir, false, kCh>(tab, jj[k], L, h[k], db, ytab, invL) <= M[k]);
+                if (kLong) {
+                    if (a && done) {
+                        float cv = __int_as_float(A[k]);
+                        // only invisible steps ahead: a run still open closes at the next one
+                        if (myLen > db && s[k] < 0) cv = add_run(cv, db + 1, __int_as_float(s[k] & 0x7FFFFFFF));
+                        so[jj[k]] = kDir > 0 ? cv : cv * R;
+                    }
+                } else if (a && done) {
                     const int cv = myLen > db ? A[k] : A[k] - ((db + 1) * (db + 1) - s[k] * s[k]);
                     if (kDir > 0)
                         soi[jj[k]] = cv;
@@ -499,7 +571,7 @@ __device__ __forceinline__ void scan_group(const float* row, int L, float povh, 
                     }
                     if (p >= T) sk = -1;  // lane left empty
                     const int sa = nth_set_bit(m, p >= T ? 0 : p - base) << 2;  // ds_bpermute byte address
-                    int nj = safe, nA = 1, nS = 0;
+                    int nj = safe, nA = kA0, nS = kS0;
                     float nh = 0.0f, nM = -2000.0f;
 #pragma unroll
                     for (int k = k2; k < kG; ++k) {
@@ -535,7 +607,7 @@ __device__ __forceinline__ void scan_group(const float* row, int L, float povh, 
 // of 64 observers (kG = 1), or groups of kG chunks with lane compaction,
 // handed out by an LDS counter.  Ends with a barrier so the caller may
 // restage LDS.
-template <int kWaves, int kG>
+template <int kWaves, int kG, bool kLong = false>
 __device__ __forceinline__ void sdem_bits_row(const RowWork w, const SecDesc* __restrict__ secs,
                                               const float* __restrict__ in4, const int* __restrict__ target,
                                               const float* __restrict__ weight, const uint32_t* __restrict__ fl,
@@ -548,24 +620,37 @@ __device__ __forceinline__ void sdem_bits_row(const RowWork w, const SecDesc* __
     const int f = fl_first(v);
     const int L = fl_last(v) - f;
     if (L <= 0) return;  // uniform; the work list holds only rows with L > 0
-    stage_row(row, sd, r, f, L, in4, target, weight, Sbuf, pad_bits<kG>());
+    stage_row(row, sd, r, f, L, in4, target, weight, Sbuf, pad_bits<kG, kLong>());
     if (kG > 1 && threadIdx.x == 0) *gnext = kWaves;
     __syncthreads();
-    float* tab = row + L + pad_bits<kG>();  // past the right guard band
-    row_tables<kWaves>(row, L, tab);
+    const int nchunk = (L + 63) >> 6;
+    float* so = arena + sd.so + (size_t)r * sd.dim_i + f;
+    if (kLong) {
+        // The bit of a step is the sign of M - q, which is not q > M once a
+        // difference is infinite or no number.  Heights in [-FLT_MAX, 1e30]
+        // keep every one finite (1e30 is below half an ulp of FLT_MAX); a row
+        // with any other takes the per-step scans.
+        bool plain = fabsf(povh) <= 1e30f;
+        for (int i = threadIdx.x; i < L; i += 64 * kWaves) plain &= row[i] >= -FLT_MAX && row[i] <= 1e30f;
+        if (!__syncthreads_and(plain)) {
+            for (int c = threadIdx.x >> 6; c < nchunk; c += kWaves)
+                sdem_steps_chunk<0>(row, L, c, povh, rtab, so, sd.R);
+            return;
+        }
+    }
+    float* tab = row + L + pad_bits<kG, kLong>();  // past the right guard band
+    row_tables<kWaves, kLong ? kChunksLong : kChunksMax>(row, L, tab);
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int nchunk = (L + 63) >> 6;
-    float* so = arena + sd.so + (size_t)r * sd.dim_i + f;
     int nblk = 0;  // 32-step blocks this wave ran (both directions)
     if (kG > 1) {
         const int ngroups = (nchunk + kG - 1) / kG;
         for (int g = wave; g < ngroups;) {
             const int c0 = g * kG;
             const int nck = min(kG, nchunk - c0);
-            scan_group<+1, kG>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
-            scan_group<-1, kG>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
+            scan_group<+1, kG, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
+            scan_group<-1, kG, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
             int ng = 0;
             if (lane == 0) ng = atomicAdd(gnext, 1);
             g = __builtin_amdgcn_readfirstlane(ng);
@@ -609,6 +694,30 @@ __global__ __launch_bounds__(64 * kWaves) void k_op_sdem_bits(const SecDesc* __r
                               lds + pad_bits<kG>(), steps, &gnext);
 }
 
+// Rows past 4096 cells (see flush_runs), one workgroup per row.  Bound by VALU,
+// like the shorter rows.  Eight waves share a staged row and its tables (64 KB
+// and 13 KB at the longest), so that two workgroups fill a CU.  Twelve sectors
+// of a 4600^2 DEM: 256 ms with every step of every scan (k_op_sdem), 43 ms
+// here.
+constexpr int kLongWaves = 8;
+__global__ __launch_bounds__(64 * kLongWaves) void k_op_sdem_long(
+    const SecDesc* __restrict__ secs, const RowWork* __restrict__ work, const float* __restrict__ in4,
+    const int* __restrict__ target, const float* __restrict__ weight, const uint32_t* __restrict__ fl,
+    const float* __restrict__ Sbuf, const float4* __restrict__ rtab, float povh, float* __restrict__ arena,
+    unsigned long long* __restrict__ steps) {
+    extern __shared__ float lds[];
+    __shared__ int gnext;
+    sdem_bits_row<kLongWaves, 4, true>(work[blockIdx.x], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
+                                       lds + pad_bits<4, true>(), steps, &gnext);
+}
+
+static hipError_t launch_op_sdem_long(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
+                                      const float4* rtab, float povh, unsigned long long* steps, hipStream_t s) {
+    hipLaunchKernelGGL(k_op_sdem_long, dim3(p.nwork), dim3(64 * kLongWaves), sdem_long_lds(p.maxL), s, p.secs, p.work,
+                       in4, p.target, p.weight, p.fl, Sbuf, rtab, povh, arena, steps);
+    return hipGetLastError();
+}
+
 // Persistent: a fixed grid pulls rows off the (cost-sorted) work list with
 // an atomic counter until the list is exhausted; every workgroup exits once
 // the counter passes nwork.  The counter is cleared by the launcher.
@@ -642,7 +751,7 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
                                 const float4* rtab, float povh, const SdemTuning& t, int* counter,
                                 unsigned long long* steps, hipStream_t s) {
     if (p.nwork == 0) return hipSuccess;
-    if (p.maxL > 4096) return launch_op_sdem(p, in4, Sbuf, arena, rtab, povh, 2, s);
+    if (p.maxL > 32 * kChunksMax) return launch_op_sdem_long(p, in4, Sbuf, arena, rtab, povh, steps, s);
     const int G = t.group > 1 ? 4 : 1;
     const size_t lds = sdem_bits_lds(p.maxL, G);
     if (t.persistent_wgs_per_cu > 0 && counter) {
@@ -687,7 +796,8 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
 hipError_t launch_op_sdem(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
                           const float4* rtab, float povh, int variant, hipStream_t s) {
     if (p.nwork == 0) return hipSuccess;
-    if (variant == 0 && p.maxL <= 4096) {
+    if (variant == 0) {
+        if (p.maxL > 32 * kChunksMax) return launch_op_sdem_long(p, in4, Sbuf, arena, rtab, povh, nullptr, s);
         const size_t lds = sdem_bits_lds(p.maxL);
         hipLaunchKernelGGL((k_op_sdem_bits<4, 1>), dim3(p.nwork), dim3(256), lds, s, p.secs, p.work, in4, p.target,
                            p.weight, p.fl, Sbuf, rtab, povh, arena, nullptr);
