@@ -56,17 +56,33 @@ __device__ __forceinline__ void stage_row(float* row, const SecDesc& sd, int r, 
                                           const int* __restrict__ target,
                                           const float* __restrict__ weight,
                                           const float* __restrict__ Sbuf, int pad = kPad) {
+    // kStage cells a thread and pass: their table reads, then their taps are in
+    // flight together (columns past the row: its last one, not stored)
+    constexpr int kStage = 4;
     const float* src = in4 + sd.img + (size_t)sd.type * sd.N;
-    for (int jj = (int)threadIdx.x - pad; jj < L + pad; jj += (int)blockDim.x) {
-        float v = 0.0f;
-        if (jj >= 0 && jj < L) {
-            const int j = f + jj;
-            if (Sbuf)
-                v = Sbuf[(size_t)r * sd.dim_i + j];
-            else
-                v = skew_cell(src, target[sd.tab + j], weight[sd.tab + j], r, j, sd.dim_i, sd.dim_o);
+    const int step = (int)blockDim.x;
+    for (int i = (int)threadIdx.x; i < pad; i += step) row[i - pad] = row[L + i] = 0.0f;
+    for (int j0 = (int)threadIdx.x; j0 < L; j0 += kStage * step) {
+        float x[kStage];
+        if (Sbuf) {
+#pragma unroll
+            for (int u = 0; u < kStage; ++u) x[u] = Sbuf[(size_t)r * sd.dim_i + f + min(j0 + u * step, L - 1)];
+        } else {
+            int t[kStage];
+            float w[kStage];
+#pragma unroll
+            for (int u = 0; u < kStage; ++u) {
+                const int j = f + min(j0 + u * step, L - 1);
+                t[u] = target[sd.tab + j];
+                w[u] = weight[sd.tab + j];
+            }
+#pragma unroll
+            for (int u = 0; u < kStage; ++u)
+                x[u] = skew_cell_sel(src, t[u], w[u], r, f + min(j0 + u * step, L - 1), sd.dim_i, sd.dim_o);
         }
-        row[jj] = v;
+#pragma unroll
+        for (int u = 0; u < kStage; ++u)
+            if (j0 + u * step < L) row[j0 + u * step] = x[u];
     }
 }
 
