@@ -144,13 +144,11 @@ __device__ __forceinline__ float so_cell(const SecDesc* __restrict__ secs, int s
     if (kSource == kDeskewDense) return src[(size_t)r * sd.dim_i + j];  // single reused buffer
     if (r < sd.H) {
         const uint32_t v = fl[sd.rows + r];
-        if (j < fl_first(v) || j >= fl_last(v)) return 0.0f;
-        if (kSource == kDeskewArena) return src[sd.so + (size_t)r * sd.dim_i + j];
-        return src[sd.q + r];
+        return j < fl_first(v) || j >= fl_last(v) ? 0.0f : src[sd.so + (size_t)r * sd.dim_i + j];
     }
     // r == H happens only when newAngle == 0 (weight 0).  The reference reads
     // the row the previously processed sector left in its reused buffer.
-    if (kSource == kDeskewArena && sd.stale >= 0) {
+    if (sd.stale >= 0) {
         const SecDesc pv = secs[sd.stale];
         if (r < pv.H && pv.dim_i == sd.dim_i) {
             const uint32_t v = fl[pv.rows + r];
@@ -171,70 +169,85 @@ __device__ __forceinline__ float deskew_acc(float O, float a, float b, float wj,
 
 // Which taps need a look at first/last.  Output cell (i, j) reads the skewed
 // rows t_j + i and t_j + i + 1, i.e. t_j + e with 0 <= e <= n (n = dim_o).  In
-// a sector's maps j lies in [first, last) of the rows t_j + 1 .. t_j + n - 1
-// always (t rises by 0 or 1 per column; first is exact, last at most one short,
-// and one short only for the column whose t is the row itself), so only e = 0
-// may fall outside, and e = n where the sector has no such row (newAngle 0).
+// a sector's maps j lies in [first, last) of the rows t_j + 1 .. t_j + n always
+// (t rises by 0 or 1 per column; first is exact, last at most one short, and
+// one short only for the column whose t is the row itself), so only e = 0 may
+// fall outside, and e = n where the sector has no such row (newAngle 0).
 // Checked over all sectors of many sides on the CPU: tests/test_deskew_taps.py.
 
-// Taps e = i0 .. i0 + kRows of column j: interior blocks (0 < i0, i0 + kRows <
-// n) read them unseen, the first and the last block look at e = 0 and e = n;
-// taps past the last row are not used.
+// Taps e = i0 .. i0 + kRows of column j in the first or the last block of rows:
+// taps past e = n are not used, e = 0 is tested by the caller.
 template <int kSource, int kRows>
-__device__ __forceinline__ void deskew_taps(const SecDesc* __restrict__ secs, int si, const SecDesc& sd,
-                                            const uint32_t* __restrict__ fl, const float* __restrict__ src, int i0,
-                                            int tj, int j, int dim_o, bool edge, float (&v)[kRows + 1]) {
-    const int r = i0 + tj;
-    if (!edge) {
-        const float* p = kSource == kDeskewRadon ? src + sd.q + r
-                         : src + (kSource == kDeskewArena ? sd.so : 0) + (size_t)r * sd.dim_i + j;
-        const size_t step = kSource == kDeskewRadon ? 1 : sd.dim_i;
+__device__ __forceinline__ void deskew_edge_taps(const SecDesc* __restrict__ secs, int si, const SecDesc& sd,
+                                                 const uint32_t* __restrict__ fl, const float* __restrict__ src, int i0,
+                                                 int tj, int j, int dim_o, float (&v)[kRows + 1]) {
+    const float* p = src + (kSource == kDeskewArena ? sd.so : 0);
 #pragma unroll
-        for (int m = 0; m <= kRows; ++m) v[m] = p[m * step];
-        return;
-    }
-    const int last = min(kRows, dim_o - i0);
+    for (int m = 0; m <= kRows; ++m) v[m] = p[(size_t)min(tj + min(i0 + m, dim_o), sd.H - 1) * sd.dim_i + j];
+    if (i0 + kRows >= dim_o && sd.newAngle == 0) {  // uniform
+        const float x = so_cell<kSource>(secs, si, sd, fl, src, tj + dim_o, j);
 #pragma unroll
-    for (int m = 0; m <= kRows; ++m) {
-        const int e = i0 + m;
-        if (m > last)
-            v[m] = 0.0f;
-        else if (e == 0 || e == dim_o)
-            v[m] = so_cell<kSource>(secs, si, sd, fl, src, r + m, j);
-        else if (kSource == kDeskewRadon)
-            v[m] = src[sd.q + r + m];
-        else
-            v[m] = src[(kSource == kDeskewArena ? sd.so : 0) + (size_t)(r + m) * sd.dim_i + j];
+        for (int m = 0; m <= kRows; ++m)
+            if (i0 + m == dim_o) v[m] = x;
     }
+}
+
+// The same taps in an inner block (0 < i0, i0 + kRows < n), which need no look.
+// Lane j's taps are the rows i0 + t_j .. i0 + t_j + kRows of its column: taken
+// in that order, the 64 lanes of a steep sector read 64 rows at once, and a
+// line comes from L2 again for every lane that shares it.  Each lane starts
+// (t_j - t_0) mod (kRows + 1) rows further up instead and wraps, so that at
+// every load the lanes of a band of kRows + 1 rows read one row; a pass through
+// the wave's own LDS puts the taps back in order.  The row blocks start at
+// different rows of the band: with a side of 1024 they would otherwise all
+// read rows a multiple of 64 KB apart, and so few memory channels, at a time.
+template <int kRows>
+__device__ __forceinline__ int deskew_shift(int tj, unsigned by) {
+    return (int)((unsigned)(tj - __builtin_amdgcn_readfirstlane(tj)) + 5u * by) % (kRows + 1);
+}
+template <int kSource, int kRows>
+__device__ __forceinline__ void deskew_inner_taps(const SecDesc& sd, const float* __restrict__ src, int i0, int tj,
+                                                  int shift, int j, float (&v)[kRows + 1]) {
+    const float* p = src + (kSource == kDeskewArena ? sd.so : 0);
+    // loads k < shift are the last taps, k >= shift the first
+    const unsigned lo = (unsigned)(i0 + tj - shift) * (unsigned)sd.dim_i + (unsigned)j;
+    const unsigned hi = lo + (unsigned)((kRows + 1) * sd.dim_i);
+#pragma unroll
+    for (int k = 0; k <= kRows; ++k) v[k] = (p + (size_t)k * sd.dim_i)[k < shift ? hi : lo];
+}
+// `lds`: this lane's column of (kRows + 1) x 64, with kRows x 64 in front.
+template <int kRows>
+__device__ __forceinline__ void deskew_order(float* lds, int shift, float (&v)[kRows + 1]) {
+    float* const lo = lds - 64 * shift;
+    float* const hi = lo + 64 * (kRows + 1);
+#pragma unroll
+    for (int k = 0; k <= kRows; ++k) (k < shift ? hi : lo)[64 * k] = v[k];
+#pragma unroll
+    for (int m = 0; m <= kRows; ++m) v[m] = lds[64 * m];
 }
 
 // kRows consecutive output rows per thread: the kRows + 1 taps of a sector are
 // shared by neighbouring rows; each row accumulates in ascending sector order.
 // While a sector is added, the taps of the next and the table entries of the
-// one after are on their way.  Orientation t of one image: sectors [sb, se),
-// accumulators acc (four dimx*dimy buffers), started from zero with `init`.
-template <int kSource, int kMax, int kRows>
-__device__ __forceinline__ void deskew_body(const SecDesc* __restrict__ secs, const int* __restrict__ target,
+// one after are on their way.
+template <int kSource, int kMax, int kRows, bool kEdge>
+__device__ __forceinline__ void deskew_rows(const SecDesc* __restrict__ secs, const int* __restrict__ target,
                                             const float* __restrict__ weight, const uint32_t* __restrict__ fl,
-                                            const float* __restrict__ src, int t, int sb, int se, bool init,
-                                            float* __restrict__ acc, int dimx, int dimy) {
-    if (sb >= se) return;
-    const bool tr = (t == 1 || t == 2);
-    const int dim_i = tr ? dimy : dimx, dim_o = tr ? dimx : dimy;
-    const int i0 = blockIdx.y * kRows;
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i0 >= dim_o || j >= dim_i) return;
-    const size_t N = (size_t)dimx * dimy;
-    float* o = acc + (size_t)t * N + (size_t)i0 * dim_i + j;
-    const bool edge = i0 == 0 || i0 + kRows >= dim_o;  // uniform
-    const int nrow = min(kRows, dim_o - i0);
-    float O[kRows];
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) O[k] = (!init && k < nrow) ? o[(size_t)k * dim_i] : 0.0f;
+                                            const float* __restrict__ src, int sb, int se, int i0, int j, int dim_o,
+                                            unsigned by, float* own, float (&O)[kRows]) {
     float v[kRows + 1], vn[kRows + 1];
-    int tn = target[secs[sb].tab + j];
+    uint32_t f = 0, fn = 0;  // the row range of e = 0
+    auto load = [&](int si, int t, int shift, uint32_t& fx, float (&x)[kRows + 1]) {
+        if constexpr (kEdge) {
+            if (kSource != kDeskewDense && i0 == 0) fx = fl[secs[si].rows + t];
+            deskew_edge_taps<kSource, kRows>(secs, si, secs[si], fl, src, i0, t, j, dim_o, x);
+        } else {
+            deskew_inner_taps<kSource, kRows>(secs[si], src, i0, t, shift, j, x);
+        }
+    };
+    int tn = target[secs[sb].tab + j], shift = deskew_shift<kRows>(tn, by), shift_n = 0;
     float w = weight[secs[sb].tab + j], wn = 0.0f;
-    deskew_taps<kSource, kRows>(secs, sb, secs[sb], fl, src, i0, tn, j, dim_o, edge, v);
+    load(sb, tn, shift, f, v);
     if (sb + 1 < se) {
         tn = target[secs[sb + 1].tab + j];
         wn = weight[secs[sb + 1].tab + j];
@@ -246,31 +259,74 @@ __device__ __forceinline__ void deskew_body(const SecDesc* __restrict__ secs, co
             t2 = target[secs[si + 2].tab + j];
             w2 = weight[secs[si + 2].tab + j];
         }
-        if (si + 1 < se)
-            deskew_taps<kSource, kRows>(secs, si + 1, secs[si + 1], fl, src, i0, tn, j, dim_o, edge, vn);
+        if (si + 1 < se) {
+            shift_n = deskew_shift<kRows>(tn, by);
+            load(si + 1, tn, shift_n, fn, vn);
+        }
+        if constexpr (kEdge) {
+            if (kSource != kDeskewDense && i0 == 0 && (j < fl_first(f) || j >= fl_last(f))) v[0] = 0.0f;
+        } else {
+            deskew_order<kRows>(own, shift, v);
+        }
         const int angle = secs[si].angle;
 #pragma unroll
         for (int k = 0; k < kRows; ++k) O[k] = deskew_acc<kMax>(O[k], v[k], v[k + 1], w, angle);
 #pragma unroll
         for (int m = 0; m <= kRows; ++m) v[m] = vn[m];
+        f = fn;
         w = wn;
         wn = w2;
         tn = t2;
+        shift = shift_n;
     }
+}
+
+// Orientation t of one image: sectors [sb, se), accumulators acc (four
+// dimx*dimy buffers), started from zero with `init`.
+template <int kSource, int kMax, int kRows>
+__device__ __forceinline__ void deskew_body(const SecDesc* __restrict__ secs, const int* __restrict__ target,
+                                            const float* __restrict__ weight, const uint32_t* __restrict__ fl,
+                                            const float* __restrict__ src, int t, int sb, int se, bool init,
+                                            float* __restrict__ acc, int dimx, int dimy) {
+    __shared__ float lds[64 * (kRows + 4 * (kRows + 1))];
+    if (sb >= se) return;
+    const bool tr = (t == 1 || t == 2);
+    const int dim_i = tr ? dimy : dimx, dim_o = tr ? dimx : dimy;
+    // Workgroups go to the eight XCDs in turn: each XCD takes a run of blocks, so
+    // that a line which two neighbouring row blocks share comes to one L2 once.
+    const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y, xcd = lin & 7;
+    const unsigned at = xcd * (total >> 3) + min(xcd, total & 7) + (lin >> 3);
+    const unsigned by = at / gridDim.x, bx = at - by * gridDim.x;
+    const int i0 = (int)by * kRows;
+    const int j = (int)(bx * blockDim.x + threadIdx.x);
+    if (i0 >= dim_o || j >= dim_i) return;
+    const size_t N = (size_t)dimx * dimy;
+    float* o = acc + (size_t)t * N + (size_t)i0 * dim_i + j;
+    const int nrow = min(kRows, dim_o - i0);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float* const own = lds + 64 * (kRows + wave * (kRows + 1)) + lane;
+    float O[kRows];
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) O[k] = (!init && k < nrow) ? o[(size_t)k * dim_i] : 0.0f;
+    if (i0 == 0 || i0 + kRows >= dim_o)  // uniform
+        deskew_rows<kSource, kMax, kRows, true>(secs, target, weight, fl, src, sb, se, i0, j, dim_o, by, own, O);
+    else
+        deskew_rows<kSource, kMax, kRows, false>(secs, target, weight, fl, src, sb, se, i0, j, dim_o, by, own, O);
 #pragma unroll
     for (int k = 0; k < kRows; ++k)
         if (k < nrow) o[(size_t)k * dim_i] = O[k];
 }
 
-// Bound by the latency of the gathers (an arena is read once: 500^2 moves 190
-// MB).  With every tap tested against its row's range, one sector at a time and
-// the last rows of an odd side one by one, all sectors took 250 us at 500^2 and
-// 1,450 us at 1501^2; now 130 and 870 us.  Below four workgroups of 16 rows per
-// CU more, shorter threads hide more of it: 500^2 138 us with 16 rows, 130 with
-// 8; the Radon source 44 us with 4 rows unstaged, 40 staged (one 512^2 image;
-// 49 before).
+// Bound by the reads of the arena (each cell once: 500^2 moves 190 MB, 2048^2 3
+// GB).  All sectors with every tap tested, taken straight down the columns, one
+// sector at a time and the last rows of an odd side one by one -> now: 250^2
+// 536 -> 56 us, 500^2 263 -> 68, 1024^2 260 -> 250 (maximum: 368 -> 253), 1501^2
+// 1,444 -> 435, 2048^2 991 -> 739 us (4.1 TB/s).  Without the rotated order
+// 1501^2 takes 866 us, without the runs of blocks per XCD about 500; 8 rows a
+// thread instead of 16: 500^2 130 -> 158 us, 2048^2 852 -> 1,240.
+// The Radon source below 1024 workgroups: 4 rows 40 us (one 512^2 image; 49
+// with the taps gathered, 16 rows a thread).
 constexpr int kDeskewRows = 16;      // output rows per thread
-constexpr int kDeskewSmallRows = 8;  // of an arena below 1024 workgroups of the former
 constexpr int kDeskewRadonRows = 4;  // of the Radon source below 1024 workgroups
 
 __device__ __forceinline__ int range_begin(int t, int4 lo, int4 hi) {
@@ -433,11 +489,7 @@ hipError_t launch_deskew(const DevPlan& p, const int range[8], const float* src,
     if (source == kDeskewDense) {
         if (is_max) SKE_DESKEW(kDeskewDense, 1, kDeskewRows); else SKE_DESKEW(kDeskewDense, 0, kDeskewRows);
     } else if (source == kDeskewArena) {
-        if ((size_t)gx * ((dl + kDeskewRows - 1) / kDeskewRows) * 4 >= 1024) {
-            if (is_max) SKE_DESKEW(kDeskewArena, 1, kDeskewRows); else SKE_DESKEW(kDeskewArena, 0, kDeskewRows);
-        } else {
-            if (is_max) SKE_DESKEW(kDeskewArena, 1, kDeskewSmallRows); else SKE_DESKEW(kDeskewArena, 0, kDeskewSmallRows);
-        }
+        if (is_max) SKE_DESKEW(kDeskewArena, 1, kDeskewRows); else SKE_DESKEW(kDeskewArena, 0, kDeskewRows);
     } else if ((size_t)gx * ((dl + kDeskewRows - 1) / kDeskewRows) * 4 >= 1024) {
         SKE_DESKEW_RADON(kDeskewRows);
     } else {

@@ -24,6 +24,7 @@ def test_inner_taps_lie_in_their_rows_range(sides):
             # e = 0: never left of the row's first cell; e = n: inside its row where that row exists
             assert (first[t] <= j).all(), (n, a)
             e = t + n
+            assert p.newAngle == 0 or (e < p.skewHeight).all(), (n, a)
             e, je = e[e < p.skewHeight], j[e < p.skewHeight]
             assert ((first[e] <= je) & (je < last[e])).all(), (n, a)
             # column j is inside every row of [t_j + 1, t_j + n - 1] if the rows that exclude it,
