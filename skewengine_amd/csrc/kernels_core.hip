@@ -73,24 +73,39 @@ hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, 
 }
 
 // ---------------------------------------------------------------------------
-// skew, materialised: every cell of the H x dim_i skewed block.
+// skew, materialised: every cell of the H x dim_i skewed block; the output
+// buffer's block is zeroed (resetSkew).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_skew_full(const SecDesc* __restrict__ secs,
                                                    const float* __restrict__ in4,
                                                    const int* __restrict__ target,
                                                    const float* __restrict__ weight,
-                                                   float* __restrict__ S) {
-    const SecDesc sd = secs[0];
+                                                   float* __restrict__ S, float* __restrict__ SO) {
+    const SecDesc& sd = secs[0];
     const int r = blockIdx.y;
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= sd.dim_i) return;
     const float* src = in4 + sd.img + (size_t)sd.type * sd.N;
-    S[(size_t)r * sd.dim_i + j] = skew_cell(src, target[sd.tab + j], weight[sd.tab + j], r, j, sd.dim_i, sd.dim_o);
+    const size_t at = (size_t)r * sd.dim_i + j;
+    SO[at] = 0.0f;
+    S[at] = skew_cell_sel(src, target[sd.tab + j], weight[sd.tab + j], r, j, sd.dim_i, sd.dim_o);
 }
 
-hipError_t launch_skew_full(const DevPlan& p, const SecDesc& h, const float* in4, float* S, hipStream_t s) {
+hipError_t launch_skew_full(const DevPlan& p, const SecDesc& h, const float* in4, float* S, float* SO, hipStream_t s) {
     dim3 grid((h.dim_i + 255) / 256, h.H);
-    hipLaunchKernelGGL(k_skew_full, grid, dim3(256), 0, s, p.secs, in4, p.target, p.weight, S);
+    hipLaunchKernelGGL(k_skew_full, grid, dim3(256), 0, s, p.secs, in4, p.target, p.weight, S, SO);
+    return hipGetLastError();
+}
+
+// n 16-byte words, from pinned host memory to the device.
+__global__ __launch_bounds__(256) void k_copy16(uint4* __restrict__ dst, const uint4* __restrict__ src, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_copy16(void* dst, const void* src, int n, hipStream_t s) {
+    hipLaunchKernelGGL(k_copy16, dim3((unsigned)(n + 255) / 256), dim3(256), 0, s, reinterpret_cast<uint4*>(dst),
+                       reinterpret_cast<const uint4*>(src), n);
     return hipGetLastError();
 }
 

@@ -41,8 +41,10 @@ hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, 
 
 // Materialise the skewInput rows (H*dim_i) of one sector; cells without a
 // tap are zero, as after resetSkew + skew (src/skewEngine.cuh:567,612-621).
-hipError_t launch_skew_full(const DevPlan& p, const SecDesc& h, const float* in4, float* S,
-                            hipStream_t s);
+// Zeroes the same cells of SO (resetSkew).
+hipError_t launch_skew_full(const DevPlan& p, const SecDesc& h, const float* in4, float* S, float* SO, hipStream_t s);
+// Copy n 16-byte words from pinned host memory.
+hipError_t launch_copy16(void* dst, const void* src, int n, hipStream_t s);
 
 // Operators.  `Sbuf` == nullptr gathers rows from the oriented inputs
 // (fused path); otherwise rows come from a materialised skewInput.

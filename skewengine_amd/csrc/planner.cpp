@@ -94,65 +94,88 @@ void plan_finish(ImagePlan& ip, int order) {
     for (size_t i = 0; i < rows.size(); i++) ip.work[i] = rows[i].w;
 }
 
+namespace {
+
+// Sector `sp` as the next of `ip`; `first`: no sector of the image before it.
+void append_sector(int dimx, int dimy, const SectorPlan& sp, bool first, long long img, ImagePlan& ip, int range8[8]) {
+    SecDesc d{};
+    d.angle = sp.angle;
+    d.newAngle = sp.newAngle;
+    d.type = sp.type;
+    d.dim_i = sp.dim_i;
+    d.dim_o = sp.dim_o;
+    d.H = sp.H;
+    d.offset = sp.offset;
+    d.tab = (int)ip.target.size();
+    d.rows = (int)ip.fl.size();
+    d.stale = -1;
+    // The deskew's zero-weight tap of a newAngle == 0 sector reads row H,
+    // which holds what the previously processed sector left there.
+    if (sp.newAngle == 0 && !first) d.stale = (int)ip.secs.size() - 1;
+    d.pad0 = 0;
+    d.R = (float)(sp.scale * sp.scale);  // (float)pow(scale,2), src/kernelSDEM.h:171
+    d.rscale = (float)(1 / sp.scale);
+    d.img = img;
+    d.so = ip.so_total;
+    d.q = ip.q_total;
+    d.N = dimx * dimy;
+    const int si = (int)ip.secs.size();
+    ip.target.insert(ip.target.end(), sp.target.begin(), sp.target.begin() + sp.dim_i);
+    ip.weight.insert(ip.weight.end(), sp.weight.begin(), sp.weight.begin() + sp.dim_i);
+    for (int r = 0; r < sp.H; r++) {
+        const int f = sp.first[r], l = sp.last[r];
+        ip.fl.push_back((uint32_t)f | ((uint32_t)l << 16));
+        const int L = l - f;
+        if (L > 0) {
+            ip.work.push_back(RowWork{si, r});
+            ip.maxL = std::max(ip.maxL, L);
+            ip.cells += L;
+            ip.steps += (double)L * (L - 1);
+        }
+    }
+    ip.maxH = std::max(ip.maxH, sp.H);
+    ip.maxI = std::max(ip.maxI, sp.dim_i);
+    ip.so_total += (long long)sp.H * sp.dim_i;
+    ip.q_total += sp.H;
+    if (range8[2 * sp.type] == range8[2 * sp.type + 1]) range8[2 * sp.type] = si;
+    range8[2 * sp.type + 1] = si + 1;
+    ip.secs.push_back(d);
+}
+
+}  // namespace
+
 void plan_append(int dimx, int dimy, int s0, int s1, long long img, ImagePlan& ip, int range8[8]) {
     ip.dimx = dimx;
     ip.dimy = dimy;
     ip.s0 = s0;
     ip.s1 = s1;
     for (int t = 0; t < 8; t++) range8[t] = 0;
-    int seen[4] = {0, 0, 0, 0};
     SectorPlan sp;
-    long long so = ip.so_total, q = ip.q_total;
     for (int a = s0; a < s1; a++) {
         plan_sector(dimx, dimy, a, sp);
-        SecDesc d{};
-        d.angle = a;
-        d.newAngle = sp.newAngle;
-        d.type = sp.type;
-        d.dim_i = sp.dim_i;
-        d.dim_o = sp.dim_o;
-        d.H = sp.H;
-        d.offset = sp.offset;
-        d.tab = (int)ip.target.size();
-        d.rows = (int)ip.fl.size();
-        d.stale = -1;
-        // The deskew's zero-weight tap of a newAngle == 0 sector reads row H,
-        // which holds what the previously processed sector left there.
-        if (sp.newAngle == 0 && a > s0) d.stale = (int)ip.secs.size() - 1;
-        d.pad0 = 0;
-        d.R = (float)(sp.scale * sp.scale);  // (float)pow(scale,2), src/kernelSDEM.h:171
-        d.rscale = (float)(1 / sp.scale);
-        d.img = img;
-        d.so = so;
-        d.q = q;
-        d.N = dimx * dimy;
-        const int si = (int)ip.secs.size();
-        ip.target.insert(ip.target.end(), sp.target.begin(), sp.target.begin() + sp.dim_i);
-        ip.weight.insert(ip.weight.end(), sp.weight.begin(), sp.weight.begin() + sp.dim_i);
-        for (int r = 0; r < sp.H; r++) {
-            const int f = sp.first[r], l = sp.last[r];
-            ip.fl.push_back((uint32_t)f | ((uint32_t)l << 16));
-            const int L = l - f;
-            if (L > 0) {
-                ip.work.push_back(RowWork{si, r});
-                ip.maxL = std::max(ip.maxL, L);
-                ip.cells += L;
-                ip.steps += (double)L * (L - 1);
-            }
-        }
-        ip.maxH = std::max(ip.maxH, sp.H);
-        ip.maxI = std::max(ip.maxI, sp.dim_i);
-        so += (long long)sp.H * sp.dim_i;
-        q += sp.H;
-        if (!seen[sp.type]) {
-            seen[sp.type] = 1;
-            range8[2 * sp.type] = si;
-        }
-        range8[2 * sp.type + 1] = si + 1;
-        ip.secs.push_back(d);
+        append_sector(dimx, dimy, sp, a == s0, img, ip, range8);
     }
-    ip.so_total = so;
-    ip.q_total = q;
+}
+
+void plan_one(int dimx, int dimy, const SectorPlan& sp, ImagePlan& ip) {
+    ip.dimx = dimx;
+    ip.dimy = dimy;
+    ip.s0 = sp.angle;
+    ip.s1 = sp.angle + 1;
+    ip.secs.clear();
+    ip.target.clear();
+    ip.weight.clear();
+    ip.fl.clear();
+    ip.work.clear();
+    ip.maxL = ip.maxH = ip.maxI = 0;
+    ip.so_total = ip.q_total = 0;
+    ip.cells = ip.steps = 0;
+    for (int t = 0; t < 8; t++) ip.range[t] = 0;
+    append_sector(dimx, dimy, sp, true, 0, ip, ip.range);
+    std::stable_sort(ip.work.begin(), ip.work.end(), [&](const RowWork& x, const RowWork& y) {
+        const uint32_t a = ip.fl[x.row], b = ip.fl[y.row];
+        return (a >> 16) - (a & 0xffffu) > (b >> 16) - (b & 0xffffu);
+    });
 }
 
 void recip_table(int n, std::vector<float>& tab4) {

@@ -54,6 +54,10 @@ enum WorkOrder { kOrderNatural = 0, kOrderCostDesc = 1 };
 void plan_image(int dimx, int dimy, int s0, int s1, long long img, long long so_base, long long q_base,
                 int order, ImagePlan& ip);
 
+// The plan of one sector already computed by plan_sector (offsets 0), rows by
+// descending L.  Keeps ip's storage.
+void plan_one(int dimx, int dimy, const SectorPlan& sp, ImagePlan& ip);
+
 // Append sectors [s0, s1) of one more image to `ip` (arena and projection
 // offsets continue from ip.so_total / ip.q_total); range8 receives the
 // image's per-type [begin, end) indices into ip.secs.  Call plan_finish once

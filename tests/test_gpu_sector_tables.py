@@ -1,0 +1,44 @@
+"""The per-sector calls' table ring: more sectors than slots without a wait
+between them, sides whose ring has 16 and 2 slots, and several engines in turn;
+each sector's result against the all-sector run of that sector alone."""
+import numpy as np
+import pytest
+
+import skewengine_amd as ske
+from skewengine_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,angles", [(2, range(180)), (50, range(179, -1, -1)), (301, range(0, 180, 4)),
+                                      (2100, (0, 44, 45, 46, 91, 134, 179))])
+def test_sectors_without_waits_equal_the_run(n, angles):
+    g = synth.dem(64 * -(-n // 64), 0.8, n, 1500.0)[:n, :n].copy()
+    with ske.SkewEngine(g) as e, ske.SkewEngine(g) as f, ske.SkewEngine(g) as r:
+        e.set_kernel(ske.KERNEL_IDENTITYDEM)
+        f.set_kernel(ske.KERNEL_IDENTITYDEM)
+        ref = np.zeros((n, n), np.float64)
+        for a in angles:
+            for x in (e, f):
+                x.skew(a)
+                x.kernel()
+                x.deskew()
+            ref += r.run(ske.KERNEL_IDENTITYDEM, a, a + 1)
+        out = e.reduce(np.zeros((n, n), np.float32))
+        assert np.array_equal(out, f.reduce(np.zeros((n, n), np.float32)))
+    # one float32 addition per sector and orientation, of non-negative values
+    assert np.allclose(out, ref, rtol=(len(list(angles)) + 4) * 2.0 ** -24, atol=0)
+
+
+def test_tables_of_the_last_sector():
+    g = synth.dem(64, 0.8, 1, 1500.0)
+    with ske.SkewEngine(g) as e:
+        e.set_kernel(ske.KERNEL_IDENTITYDEM)
+        for a in range(40):
+            e.skew(a)
+        e.kernel()
+        S, SO = e.skew_buffers()
+        _, t, w, f, l = ske.plan_sector(64, 64, 39)
+        for r in range(S.shape[0]):
+            j = np.arange(f[r], l[r])
+            assert np.array_equal(SO[r, j], S[r, j]) and not SO[r, :f[r]].any() and not SO[r, l[r]:].any()
