@@ -174,14 +174,13 @@ int ske_output_device(ske_engine *e, const float **d_output);
 int ske_synchronize(ske_engine *e);
 
 /* Options (no reference counterpart). */
-#define SKE_OPT_SDEM_VARIANT 1  /* viewshed inner loop: 0 bit-block (default; rows <= 4096 cells,
-                                   longer rows use 2), 1 IEEE divide per step, 2 exact fma division
+#define SKE_OPT_SDEM_VARIANT 1  /* viewshed inner loop: 0 bit-block (default), 1 IEEE divide per step, 2 exact fma division
                                    per step.  All three give identical results. */
 #define SKE_OPT_ARENA_BYTES 2   /* device budget for one chunk of skewOutput rows */
 #define SKE_OPT_PROFILE 3       /* 1: time every launch with HIP events on the engine stream */
 #define SKE_OPT_GRAPH 4         /* 1: capture the all-sector run once in a hipGraph and replay it */
-#define SKE_OPT_SDEM_WAVES 5    /* viewshed: waves per workgroup (2, 4, 8); unset: 4, or 2 for rows of
-                                 * fewer than four chunk groups (or chunks) per scan direction.
+#define SKE_OPT_SDEM_WAVES 5    /* viewshed: waves per workgroup (2, 4, 8); unset: by the rows'
+                                 * length (long rows, past 4096 cells, always 8).
                                  * ske_get_option reports the set value (4 while unset), not
                                  * the per-chunk automatic choice */
 #define SKE_OPT_SDEM_PERSISTENT 6 /* viewshed: 0 one workgroup per row, k>0 persistent grid of k per CU */
@@ -191,9 +190,9 @@ int ske_synchronize(ske_engine *e);
 #define SKE_OPT_COUNT_STEPS 9     /* 1: the all-sector bit-block viewshed counts the ray steps its
                                    * lanes execute (counter "op_sdem_lane_steps"; the scans stop
                                    * early once no later target can be visible) */
-#define SKE_OPT_SDEM_GROUP 10      /* viewshed: 4 (default) groups of four 64-observer chunks per
-                                   * wave whose finished scans are replaced by the group's remaining
-                                   * ones (lane compaction); 1 one chunk per wave */
+#define SKE_OPT_SDEM_GROUP 10      /* viewshed: 4 (default) pools of up to four 64-observer chunks
+                                   * per wave, which run only the blocks of a scan that may hold a
+                                   * visible step; 1 one chunk per wave */
 int ske_set_option(ske_engine *e, int option, long long value);
 int ske_get_option(ske_engine *e, int option, long long *value);
 /* Accumulated HIP-event time of the launches named `name` since the last

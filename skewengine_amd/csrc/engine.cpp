@@ -25,6 +25,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <memory>
 #include <string>
@@ -161,6 +162,7 @@ struct Chunk {
     std::vector<Part> parts;
     DevBuf<DeskewPart> dparts;  // the parts for the one-launch deskew
     int max_n = 0;              // largest grid side among the parts
+    std::vector<SdemRun> runs;  // of a row list by descending length: the viewshed's launches
     DevBuf<SampleReq> sreq;  // sample points of the local Radon transform in this chunk
     int nreq = 0;
     int sample_version = -1;  // Core::sample_version the requests were built for
@@ -235,6 +237,7 @@ struct Core {
     hipStream_t stream = nullptr;
     std::vector<Image> imgs;
     std::vector<ReduceImage> rimgs;  // the same for the reduce
+    int odd = 0;  // some grid holds a value that is not finite or above 1e30
     DevBuf<float> in4, acc, out;
     int present[4] = {0, 0, 0, 0};  // per run, same for every grid (same sector range)
     // constant tables
@@ -323,6 +326,7 @@ struct Core {
         return SKE_OK;
     }
 
+    int* odd_flag() { return counter.p + 4; }
     unsigned long long* step_counter() { return reinterpret_cast<unsigned long long*>(counter.p + 2); }
 
     int sync() {
@@ -412,9 +416,10 @@ struct Core {
             SKE_HIP(hipMemcpyAsync(base, inputs[i], N * sizeof(float),
                                    on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, stream));
             SKE_TRY(launch("prepare", [&] {
-                return launch_prepare(base, base + N, base + 2 * N, base + 3 * N, im.n, im.n, stream);
+                return launch_prepare(base, base + N, base + 2 * N, base + 3 * N, im.n, im.n, odd_flag(), stream);
             }));
         }
+        SKE_HIP(hipMemcpyAsync(&odd, odd_flag(), sizeof(int), hipMemcpyDeviceToHost, stream));
         SKE_TRY(launch("fill", [&] { return launch_fill_f32(acc.p, 4 * (size_t)tot, 0.0f, stream); }));
         SKE_TRY(launch("fill", [&] { return launch_fill_f32(out.p, (size_t)tot, 0.0f, stream); }));
         return sync();
@@ -439,6 +444,7 @@ struct Core {
         auto flush = [&]() -> int {
             if (cur->parts.empty()) return SKE_OK;
             plan_finish(cur->plan.ip, order);
+            if (order == kOrderCostDesc) cur->runs = sdem_runs(cur->plan.ip);
             SKE_TRY(cur->plan.upload(stream));
             std::vector<DeskewPart> dp(cur->parts.size());
             for (size_t k = 0; k < cur->parts.size(); k++) {
@@ -540,18 +546,28 @@ struct Core {
         return SKE_OK;
     }
 
-    // Without a caller's or the autotuner's choice, a grid workgroup whose
-    // rows hold fewer than four work units (chunk groups, or chunks) per scan
-    // direction runs 2 waves instead of 4, so that no wave of it idles
-    // (500 x 500 grid: 2.36 instead of 3.19 ms).
-    SdemTuning effective_tuning(int maxL) const {
-        SdemTuning t = tune;
-        if (!waves_set && t.persistent_wgs_per_cu == 0) {
-            const int chunks = (maxL + 63) / 64;
-            const int units = t.group > 1 ? (chunks + t.group - 1) / t.group : chunks;
-            t.waves = units < 4 ? 2 : 4;
+    // The viewshed over a planned row list.  Without a caller's or the
+    // autotuner's choice (`own`) the waves of a grid workgroup follow the run's
+    // rows; with one chunk per wave, rows of fewer than four chunks run 2
+    // instead of 4, so that no wave of it idles.
+    hipError_t launch_sdem(const DevPlan& v, const std::vector<SdemRun>& runs, SdemTuning t, bool own, float* dst,
+                           float povh, unsigned long long* steps) {
+        if (t.group == 1 || (t.persistent_wgs_per_cu > 0 && !odd)) {
+            if (own && t.persistent_wgs_per_cu == 0) t.waves = (v.maxL + 63) / 64 < 4 ? 2 : 4;
+            return launch_op_sdem_tuned(v, in4.p, nullptr, dst, rtab.p, povh, t, counter.p, steps, stream);
         }
-        return t;
+        t.check = odd || !(std::fabs(povh) <= 1e30f);
+        for (const SdemRun& r : runs) {
+            DevPlan p = v;
+            p.work += r.first;
+            p.nwork = r.count;
+            p.maxL = r.maxL;
+            if (own) t.waves = r.waves;
+            const hipError_t e =
+                launch_op_sdem_tuned(p, in4.p, nullptr, dst, rtab.p, povh, t, counter.p, steps, stream);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
     }
 
     // Enqueue the whole all-sector run (no allocation, no synchronisation:
@@ -571,10 +587,9 @@ struct Core {
             switch (kernel_id) {
             case SKE_KERNEL_SDEM:
                 if (sdem_variant == 0) {
-                    const SdemTuning t = effective_tuning(v.maxL);
                     SKE_TRY(launch("op_sdem", [&] {
-                        return launch_op_sdem_tuned(v, in4.p, nullptr, arena.p, rtab.p, povh, t, counter.p,
-                                                    count_steps ? step_counter() : nullptr, stream);
+                        return launch_sdem(v, cp->runs, tune, !waves_set, arena.p, povh,
+                                           count_steps ? step_counter() : nullptr);
                     }));
                 } else {
                     SKE_TRY(launch("op_sdem", [&] {
@@ -635,7 +650,7 @@ struct Core {
         unsigned pbits = 0;
         memcpy(&pbits, &povh, sizeof pbits);
         // every setting that changes what enqueue_run records is part of the key
-        // (waves_set: unset wave counts are chosen per chunk by effective_tuning)
+        // (waves_set: unset wave counts are chosen by launch_sdem)
         snprintf(key, sizeof key, "%d:%d:%d:%08x:%d:%d:%d:%d:%d:%d:%lld:%d:%d:%d", kernel_id, s0, s1, pbits,
                  sdem_variant, tune.waves, waves_set ? 1 : 0, tune.persistent_wgs_per_cu, tune.occupancy, tune.group,
                  arena_bytes, radon_local ? 1 : 0, count_steps ? 1 : 0, sample_version);
@@ -765,7 +780,9 @@ struct Core {
         SKE_TRY(scratch.ensure((size_t)sample->ip.so_total));
         const DevPlan v = sample->view();
         // Listed with the shape that measures fastest on the 180-sector batches first.
-        const SdemTuning cands[] = {{4, 0, 0, 4}, {4, 0, 0, 1}, {8, 0, 0, 4}, {2, 0, 0, 4}, {4, 8, 6, 4},
+        // Waves 0: by each run's rows (reported as 4, like the default).
+        const std::vector<SdemRun> runs = sdem_runs(sample->ip);
+        const SdemTuning cands[] = {{0, 0, 0, 4}, {4, 0, 0, 4}, {4, 0, 0, 1}, {8, 0, 0, 4}, {2, 0, 0, 4}, {4, 8, 6, 4},
                                     {4, 8, 0, 4}, {4, 8, 8, 1}, {4, 16, 8, 1}, {8, 8, 8, 1}, {2, 16, 8, 1}};
         hipEvent_t a = take_event(), b = take_event();
         constexpr int kCands = (int)(sizeof(cands) / sizeof(cands[0]));
@@ -773,11 +790,11 @@ struct Core {
         double best = 1e300;
         for (int ci = 0; ci < kCands; ci++) {
             const SdemTuning& c = cands[ci];
-            SKE_HIP(launch_op_sdem_tuned(v, in4.p, nullptr, scratch.p, rtab.p, povh, c, counter.p, nullptr, stream));
+            SKE_HIP(launch_sdem(v, runs, c, c.waves == 0, scratch.p, povh, nullptr));
             t[ci] = 1e300;
             for (int rep = 0; rep < 3; rep++) {
                 SKE_HIP(hipEventRecord(a, stream));
-                SKE_HIP(launch_op_sdem_tuned(v, in4.p, nullptr, scratch.p, rtab.p, povh, c, counter.p, nullptr, stream));
+                SKE_HIP(launch_sdem(v, runs, c, c.waves == 0, scratch.p, povh, nullptr));
                 SKE_HIP(hipEventRecord(b, stream));
                 SKE_HIP(hipEventSynchronize(b));
                 float ms = 0.0f;
@@ -796,8 +813,9 @@ struct Core {
         event_pool.push_back(a);
         event_pool.push_back(b);
         SKE_HIP(hipStreamSynchronize(stream));
+        waves_set = pick.waves != 0;
+        if (!waves_set) pick.waves = SdemTuning().waves;
         tune = pick;
-        waves_set = true;
         drop_graph();
         if (waves) *waves = pick.waves;
         if (wgs) *wgs = pick.persistent_wgs_per_cu;

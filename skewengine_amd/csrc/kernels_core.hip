@@ -10,11 +10,12 @@ namespace ske {
 
 // ---------------------------------------------------------------------------
 // prepare (src/skewEngine.cuh:962-987).  32x32 tiles through LDS so that the
-// two transposed copies are written coalesced.
+// two transposed copies are written coalesced.  *odd, if not null, becomes 1
+// when a value is not finite or above 1e30.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_prepare(const float* __restrict__ in0, float* __restrict__ in1,
                                                  float* __restrict__ in2, float* __restrict__ in3,
-                                                 int dimx, int dimy) {
+                                                 int dimx, int dimy, int* __restrict__ odd) {
     __shared__ float tile[32][33];
     const int x0 = blockIdx.x * 32, y0 = blockIdx.y * 32;
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
@@ -23,6 +24,7 @@ __global__ __launch_bounds__(256) void k_prepare(const float* __restrict__ in0, 
         if (i < dimy && j < dimx) {
             const float v = in0[(size_t)i * dimx + j];
             tile[k][tx] = v;
+            if (odd && !(fabsf(v) <= 1e30f)) *odd = 1;
             in3[(size_t)i * dimx + (dimx - 1 - j)] = v;  // in3[dimx*i + cj]
         }
     }
@@ -65,10 +67,10 @@ hipError_t launch_fill_f64(double* p, size_t n, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, int dimx, int dimy,
+hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, int dimx, int dimy, int* odd,
                           hipStream_t s) {
     dim3 grid((dimx + 31) / 32, (dimy + 31) / 32);
-    hipLaunchKernelGGL(k_prepare, grid, dim3(256), 0, s, in0, in1, in2, in3, dimx, dimy);
+    hipLaunchKernelGGL(k_prepare, grid, dim3(256), 0, s, in0, in1, in2, in3, dimx, dimy, odd);
     return hipGetLastError();
 }
 

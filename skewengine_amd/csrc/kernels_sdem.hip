@@ -23,6 +23,7 @@
 #include <float.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "device_common.h"
 #include "launch.h"
@@ -135,29 +136,25 @@ __global__ __launch_bounds__(256) void k_op_sdem(const SecDesc* __restrict__ sec
 // ---------------------------------------------------------------------------
 // Guard band on each side of a staged row: the one-chunk scans of a chunk
 // run to its first lane's row end, up to 95 cells past the row (128); with
-// lane compaction a block only runs while some lane's row continues, so
-// every read stays within 32 cells of the row (and of the safe positions).
-// Long rows may also take the per-step scans (kPad).
-template <int kG, bool kLong = false>
-constexpr int pad_bits() { return kLong ? kPad : kG > 1 ? 32 : 128; }
+// pools a block only runs while some lane's row continues, so every read
+// stays within 32 cells of the row (and of the safe positions), and of the
+// per-step scans within kPad.
+template <int kG>
+constexpr int pad_bits() { return kG > 1 ? kPad : 128; }
 // 32-cell chunks of a row of <= 4096 cells, and of the longest (16,000 cells).
 constexpr int kChunksMax = 128, kChunksLong = 512;
-// Chunk-maximum tables of a staged row, each indexed by chunk c in
-// [-kTabLo, kCh + kTabHi): level 0 cm[c] = max row[32c .. 32c+31],
-// level 1..3 the maxima of 2, 4 and 8 consecutive chunks starting at c,
-// then suffix and prefix maxima.  Chunks outside the row hold -inf (the
-// prefix table repeats the row maximum past the end).
-constexpr int kTabLo = 16, kTabHi = 16;
-template <int kCh>
-constexpr int tab_n() { return kTabLo + kCh + kTabHi; }
-enum { kTabL0 = 0, kTabL1 = 1, kTabL2 = 2, kTabL3 = 3, kTabSuf = 4, kTabPre = 5, kTabs = 6 };
-
-// LDS of the bit-block kernels: guard band, row, guard band, chunk tables.
-inline size_t sdem_bits_lds(int maxL, int group = 1) {
-    return sizeof(float) * ((size_t)maxL + 2 * (group > 1 ? pad_bits<4>() : pad_bits<1>()) + kTabs * tab_n<kChunksMax>());
-}
-inline size_t sdem_long_lds(int maxL) {
-    return sizeof(float) * ((size_t)maxL + 2 * pad_bits<4, true>() + kTabs * tab_n<kChunksLong>());
+// Chunk-maximum tables of a staged row: eight words per chunk c in [-kTabLo,
+// nch + kTabHi), nch the row's chunks: level 0 max row[32c .. 32c+31], levels
+// 1..3 the maxima of 2, 4 and 8 consecutive chunks starting at c, then suffix
+// and prefix maxima (two words are free: 32 bytes a chunk, so a position's byte
+// offset is itself rounded down to 32).  Chunks outside the row hold -inf (the
+// prefix maximum repeats the row's past the end).
+constexpr int kTabLo = 16, kTabHi = 16, kTabWords = 8;
+enum { kTabL0 = 0, kTabL1 = 1, kTabL2 = 2, kTabL3 = 3, kTabSuf = 4, kTabPre = 5 };
+__host__ __device__ inline int tab_words(int L) { return kTabWords * (kTabLo + ((L + 31) >> 5) + kTabHi); }
+// The words of the chunk of position p (may lie outside the row).
+__device__ __forceinline__ const float* tab_at(const float* tab, int p) {
+    return tab + kTabLo * kTabWords + ((p & ~31) >> 2);
 }
 
 __device__ __forceinline__ int lshl1_add(int a, int b) {
@@ -242,7 +239,7 @@ __device__ __forceinline__ uint32_t scan_block(const float* rowj, float h, const
 }
 
 // 16 steps d0 + u0 + 1 .. d0 + u0 + 16 of a block (no tail handling),
-// appended to w: the groups' slots run a block as two halves, so only 16
+// appended to w: the pools run a block as two halves, so only 16
 // reciprocal pairs are live in scalar registers at a time.
 template <int kDir>
 __device__ __forceinline__ uint32_t scan_half(const float* rowj, float h, const float2* __restrict__ ytab, int d0,
@@ -285,22 +282,21 @@ __device__ __forceinline__ uint32_t scan_half(const float* rowj, float h, const 
 template <int kDir, bool kClamp = true, int kCh = kChunksMax>
 __device__ __forceinline__ float exit_bound(const float* __restrict__ tab, int jj, int L, float h, int db,
                                             const float2* __restrict__ ytab, float invL) {
-    constexpr int kTabN = tab_n<kCh>();
     const int e = db + 1;
     int p = jj + kDir * e;  // nearest remaining target
     if (kClamp) p = p < 0 ? 0 : (p > L - 1 ? L - 1 : p);
-    const float* t = tab + kTabLo + (p >> 5);
+    const float* t = tab_at(tab, p);
     float s1, s2, s3, s4;
     if (kDir > 0) {  // cells [p, p+32), [p+32, p+96), [p+96, p+224), [p+224, end)
-        s1 = t[kTabL1 * kTabN];
-        s2 = t[kTabL2 * kTabN + 1];
-        s3 = t[kTabL3 * kTabN + 3];
-        s4 = t[kTabSuf * kTabN + 7];
+        s1 = t[kTabL1];
+        s2 = t[kTabL2 + kTabWords];
+        s3 = t[kTabL3 + 3 * kTabWords];
+        s4 = t[kTabSuf + 7 * kTabWords];
     } else {         // cells (p-32, p], (p-96, p-32], (p-224, p-96], [0, p-224]
-        s1 = t[kTabL1 * kTabN - 1];
-        s2 = t[kTabL2 * kTabN - 4];
-        s3 = t[kTabL3 * kTabN - 10];
-        s4 = t[kTabPre * kTabN - 7];
+        s1 = t[kTabL1 - kTabWords];
+        s2 = t[kTabL2 - 4 * kTabWords];
+        s3 = t[kTabL3 - 10 * kTabWords];
+        s4 = t[kTabPre - 7 * kTabWords];
     }
     const float a1 = s1 - h, a2 = s2 - h, a3 = s3 - h, a4 = s4 - h;
     const float amax = fmaxf(fmaxf(a1, a2), fmaxf(a3, a4));
@@ -340,28 +336,33 @@ __device__ __forceinline__ int scan_dir(const float* rowj, float h, const float4
     return myLen > d0 ? A : A - ((d0 + 1) * (d0 + 1) - s * s);
 }
 
-// Build the chunk tables of a staged row of L <= 32 kCh cells (see tab_n).
-// Ends with a barrier.
-template <int kWaves, int kCh>
-__device__ __forceinline__ void row_tables(const float* row, int L, float* tab) {
-    constexpr int kTabN = tab_n<kCh>(), kPer = kCh / 64;
-    const int nch = (L + 31) >> 5;
-    float* t0 = tab + kTabLo;
-    for (int i = threadIdx.x; i < kTabs * kTabN; i += 64 * kWaves) tab[i] = -INFINITY;
+// Build the chunk tables of a staged row of L <= 32 kCh cells.  Ends with a
+// barrier.  kCheck: returns whether every height lies in [-FLT_MAX, 1e30].
+template <int kWaves, int kCh, bool kCheck>
+__device__ __forceinline__ bool row_tables(const float* row, int L, float* tab) {
+    constexpr int kPer = kCh / 64;
+    const int nch = (L + 31) >> 5, total = kTabLo + nch + kTabHi;
+    float* t0 = tab + kTabLo * kTabWords;
+    for (int i = threadIdx.x; i < kTabWords * total; i += 64 * kWaves) tab[i] = -INFINITY;
     __syncthreads();
+    bool plain = true;
     for (int t0i = 0; t0i < nch * 32; t0i += 64 * kWaves) {
         const int t = t0i + (int)threadIdx.x;
         float v = t < L ? row[t] : -INFINITY;
+        if (kCheck) plain &= t >= L || (v >= -FLT_MAX && v <= 1e30f);
 #pragma unroll
         for (int o = 16; o; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-        if ((t & 31) == 0 && t < nch * 32) t0[kTabL0 * kTabN + (t >> 5)] = v;
+        if ((t & 31) == 0 && t < nch * 32) t0[kTabL0 + kTabWords * (t >> 5)] = v;
     }
-    __syncthreads();
+    if (kCheck)
+        plain = __syncthreads_and(plain);
+    else
+        __syncthreads();
     if (threadIdx.x < 64) {  // one wave: suffix and prefix maxima, kPer chunks per lane
         const int l = threadIdx.x;
-        float x[kPer];  // -inf past nch
+        float x[kPer];
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) x[i] = t0[kTabL0 * kTabN + kPer * l + i];
+        for (int i = 0; i < kPer; ++i) x[i] = kPer * l + i < nch ? t0[kTabL0 + kTabWords * (kPer * l + i)] : -INFINITY;
         float vs = x[0];
 #pragma unroll
         for (int i = 1; i < kPer; ++i) vs = fmaxf(vs, x[i]);
@@ -378,279 +379,370 @@ __device__ __forceinline__ void row_tables(const float* row, int L, float* tab) 
 #pragma unroll
         for (int i = kPer - 1; i >= 0; --i) {
             ns = fmaxf(x[i], ns);
-            t0[kTabSuf * kTabN + kPer * l + i] = ns;
+            if (kPer * l + i < nch) t0[kTabSuf + kTabWords * (kPer * l + i)] = ns;
         }
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             np = fmaxf(x[i], np);
-            t0[kTabPre * kTabN + kPer * l + i] = np;
+            if (kPer * l + i < nch) t0[kTabPre + kTabWords * (kPer * l + i)] = np;
         }
-        if (l < kTabHi) t0[kTabPre * kTabN + kCh + l] = __shfl(np, 63);  // whole-row maximum
+        const float top = __shfl(np, 63);  // whole-row maximum
+        if (l < kTabHi) t0[kTabPre + kTabWords * (nch + l)] = top;
     }
     for (int lev = 1; lev <= 3; ++lev) {  // level lev from level lev-1: max of two runs 2^(lev-1) apart
         const int off = 1 << (lev - 1);
-        for (int i = threadIdx.x; i < kTabN - off; i += 64 * kWaves)
-            tab[lev * kTabN + i] = fmaxf(tab[(lev - 1) * kTabN + i], tab[(lev - 1) * kTabN + i + off]);
+        for (int i = threadIdx.x; i < total - off; i += 64 * kWaves)
+            tab[lev + kTabWords * i] = fmaxf(tab[lev - 1 + kTabWords * i], tab[lev - 1 + kTabWords * (i + off)]);
         __syncthreads();
     }
+    return plain;
 }
 
 // ---------------------------------------------------------------------------
-// Lane compaction.  With the early exit a wave still runs until its longest
-// scan stops, while most of its lanes are done.  A wave therefore takes a
-// group of kG chunks (kG x 64 scans of one direction, all starting at d = 1)
-// held in kG register "slots" and steps all of them with the same uniform d.
-// After each 32-step block, lanes whose scan is over retire (write their cv)
-// and, once the live scans fit in fewer slots, they are packed into the
-// lowest slots in (slot, lane) order: the p-th live scan moves to slot p/64,
-// lane p%64.  Per-lane state moves with ds_bpermute; each destination lane
-// finds its source from the slots' live masks (prefix counts, then the n-th
-// set bit), so the packing needs no LDS.  Slots 0..k-1 hold at most 64k live
-// scans, so destination slot k2 draws only from slots >= k2 and the packing
-// can run in place, lowest slot first.
+// Pools.  With the early exit a wave still runs until its longest scan stops,
+// while most of its lanes are done, and most blocks of a scan that goes on hold
+// no visible step: its running maximum bounds them from their chunk maximum
+// alone.  A wave therefore takes a pool of up to kPoolChunks chunks (64 scans
+// of one direction each, all starting at d = 1) and steps them in rounds of one
+// 32-step block with the same uniform d.  A round first tests every live scan:
+//   - over: nothing beyond can be visible (exit_bound, every other round); it
+//     stores its cv and leaves;
+//   - nothing visible in this block: it stays as it is;
+//   - otherwise it goes on the round's list.
+// Then the listed scans run the block, 64 at a time.  State (running maximum,
+// sums) stays at the scan's place in the wave's own LDS; two lists of places
+// are kept in order, the live one rewritten in place (a place is never written
+// past the ones still to be read).
+// A block left out counts as 32 invisible steps: a trailing visible run ends
+// with the last block run, so the sums of the steps with V = 1 and that block's
+// end say everything.
 // A lane's steps past its row end are recorded as visible by or-ing the low
-// bits of its block word; retired and empty lanes read from a position whose
-// remaining steps stay inside the staged row and guard bands.  The
-// right-scan pass stores cv as an integer in the output cell; the left-scan
-// pass of the same group (same wave, later) adds its cv and stores the float
-// (float)(cvR + cvL) * R, the same value as the one-chunk path.
+// bits of its block word; empty lanes read from a position whose remaining
+// steps stay inside the staged row and guard bands.  The right-scan pass stores
+// cv as an integer in the output cell; the left-scan pass of the same pool
+// (same wave, later) adds its cv and stores the float (float)(cvR + cvL) * R,
+// the same value as the one-chunk path.
+//
+// Bound by VALU issue (1.24 wave instructions a clock and CU; the steps' mix
+// reaches 1.5) and LDS gathers of the thinned lists (2.3 clocks a wave and cell
+// in a row, 6 scattered).  Against groups of four chunks packed in registers,
+// every block of a live scan run: all sectors of 1000^2 11.5 -> 9.9 ms, 1501^2
+// 30.2 -> 29.2, 30 of 3000^2 28.6 -> 25.0, 20 of 4000^2 34.5 -> 30.7; 12 of
+// 4600^2 (long rows) 43 -> 36.  Pools of 3 chunks run too many part-filled
+// batches (1000^2 10.4 ms), of 6 leave too few waves per CU (3000^2 27.0).  Two
+// batches at a time hide the LDS latency (one: 34.5 ms at 1501^2); four need
+// 129 registers (45 ms).  One pool for all waves of a row with two barriers a
+// round: 38.7.
 // ---------------------------------------------------------------------------
-// Position of the r-th (0-based) set bit of m; m must have more than r set bits.
-__device__ __forceinline__ int nth_set_bit(uint64_t m, int r) {
-    int pos = 0;
-    uint32_t w = (uint32_t)m;
-    const int c0 = __popc(w);
-    if (r >= c0) {
-        r -= c0;
-        pos = 32;
-        w = (uint32_t)(m >> 32);
-    }
-    int c = __popc(w & 0xFFFFu);
-    if (r >= c) { r -= c; pos += 16; w >>= 16; }
-    c = __popc(w & 0xFFu);
-    if (r >= c) { r -= c; pos += 8; w >>= 8; }
-    c = __popc(w & 0xFu);
-    if (r >= c) { r -= c; pos += 4; w >>= 4; }
-    c = __popc(w & 0x3u);
-    if (r >= c) { r -= c; pos += 2; w >>= 2; }
-    if (r >= (int)(w & 1u)) pos += 1;
-    return pos;
+constexpr int kPoolChunks = 4, kPoolChunksLong = 4;
+// LDS bytes of a pool per scan: M, A | last block run << 24, the trailing run's
+// start s and two places of two bytes; long rows M, cv, d_o^2 with the flag,
+// the last block and the places.
+template <bool kLong>
+__host__ __device__ constexpr int pool_bytes() { return kLong ? 18 : 14; }
+// Chunks of a pool of a row of nchunk chunks: every wave as many pools, of at
+// most `cap` chunks.
+__host__ __device__ inline int pool_chunks(int nchunk, int waves, int cap) {
+    const int turns = (nchunk + waves * cap - 1) / (waves * cap);
+    return (nchunk + waves * turns - 1) / (waves * turns);
+}
+// The cap of a launch: the pools of its longest row.
+template <bool kLong>
+__host__ __device__ inline int pool_cap(int maxL, int waves) {
+    return pool_chunks((maxL + 63) / 64, waves, kLong ? kPoolChunksLong : kPoolChunks);
 }
 
-template <int kDir, int kG, bool kLong>
-__device__ __forceinline__ void scan_group(const float* row, int L, float povh, int c0, int nck,
-                                           const float* __restrict__ tab, const float4* __restrict__ rtab,
-                                           float* __restrict__ so, float R, int& nblk) {
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Chunks [c0, c0 + nck) of a row; st: pool_bytes x stride of this wave's LDS
+// (4-byte aligned), stride >= 64 nck.
+template <int kDir, bool kLong>
+__device__ __forceinline__ void scan_pool(const float* row, int L, float povh, int c0, int nck,
+                                          const float* __restrict__ tab, const float4* __restrict__ rtab,
+                                          float* __restrict__ so, float R, char* st, int stride, int& nblk) {
     const float2* __restrict__ ytab = reinterpret_cast<const float2*>(rtab + kMaxDim + 1);
     constexpr int kCh = kLong ? kChunksLong : kChunksMax;
-    // a scan's first state: A counts the observer's own cell; long rows go on
-    // with the right scan's sum, visible from d = 0
-    constexpr int kA0 = kLong ? 0 : 1, kS0 = kLong ? (int)0x80000000 : 0;
     int* __restrict__ soi = reinterpret_cast<int*>(so);
     const float invL = ytab[L].x;
     const int lane = threadIdx.x & 63;
     const int safe = kDir > 0 ? 0 : L - 1;  // reads row[safe + kDir*d], d <= L + 31: inside the guard bands
-    int jj[kG], A[kG], s[kG];
-    float h[kG], M[kG];
-    uint64_t act[kG];  // live scans of each slot (wave-uniform masks)
-#pragma unroll
-    for (int k = 0; k < kG; ++k) {
-        const int j = 64 * (c0 + k) + lane;
-        const int myLen = kDir > 0 ? L - 1 - j : j;
-        const bool in = k < nck && j < L;
-        if (in && myLen <= 0) {  // no targets in this direction: cv = 0
+    float* const smax = reinterpret_cast<float*>(st);
+    int* const sums = reinterpret_cast<int*>(st + 4 * stride);  // A < 2^24 while steps are left; long rows cv
+    uint32_t* const open = reinterpret_cast<uint32_t*>(st + 8 * stride);  // long rows
+    uint16_t* const tail = reinterpret_cast<uint16_t*>(st + (kLong ? 12 : 8) * stride);  // s; long rows: the last block
+    uint16_t* const live = tail + stride;
+    uint16_t* const todo = live + stride;
+    const int jb = 64 * c0;
+
+    // cv of a scan with steps left, all invisible
+    auto over = [&](int id, int j) {
+        if (kLong) {
+            float cv = __int_as_float(sums[id]);
+            const uint32_t o = open[id];  // its open run closes after the last block run
+            if (o >> 31) cv = add_run(cv, 32 * tail[id] + 1, __uint_as_float(o & 0x7FFFFFFFu));
+            so[j] = kDir > 0 ? cv : cv * R;
+        } else {
+            const int cv = sums[id] & 0xFFFFFF;
             if (kDir > 0)
-                soi[j] = 0;
+                soi[j] = cv;
             else
-                so[j] = (kLong ? so[j] : (float)soi[j]) * R;
+                so[j] = (float)(cv + soi[j]) * R;
         }
-        const bool a = in && myLen > 0;
-        act[k] = __builtin_amdgcn_ballot_w64(a);
-        jj[k] = a ? j : safe;
-        h[k] = row[jj[k]] + povh;
-        M[k] = -2000.0f;
-        A[k] = kLong && kDir < 0 && a ? soi[j] : kA0;
-        s[k] = kS0;
-    }
-    int ns = nck;
-    for (int d0 = 0; ns > 0; d0 += 32) {
-        bool ends = false;  // some lane's row ends in this block (uniform)
-        uint32_t wk[kG];
-#pragma unroll
-        for (int k = 0; k < kG; ++k)
-            if (k < ns) wk[k] = scan_half<kDir>(row + jj[k], h[k], ytab, d0, 0, M[k], 0u);
-#pragma unroll
-        for (int k = 0; k < kG; ++k)
-            if (k < ns) wk[k] = scan_half<kDir>(row + jj[k], h[k], ytab, d0, 16, M[k], wk[k]);
-#pragma unroll
-        for (int k = 0; k < kG; ++k) {
-            if (k < ns) {
-                uint32_t w = wk[k];
-                const int myLen = kDir > 0 ? L - 1 - jj[k] : jj[k];
-                // steps past the row end (the last e of the block) are recorded as
-                // visible; skipped when no lane's row ends in this block (a row
-                // ending at the block's last step adds no steps: e = 0)
-                if (__builtin_amdgcn_ballot_w64(myLen <= d0 + 32) != 0) {
-                    const int e = min(max(d0 + 32 - myLen, 0), 31);
-                    w |= (1u << e) - 1u;
-                    ends = true;
-                }
-                if (kLong)
-                    flush_runs(w, d0, (act[k] >> lane) & 1, A[k], s[k]);
-                else
-                    flush_block(w, d0, A[k], s[k]);
-            }
-        }
+    };
+    // Block d0 of kN batches of scans (places id of the pool, positions j; a:
+    // lane in use).  M, A, s: state before it, s the trailing run's start (long
+    // rows: d_o^2 and flag).  Stores the state, or cv where the row ends; on:
+    // the lanes that go on.
+    auto block = [&](auto kn, const bool* a, const int* id, const int* j, int d0, const float* M0, const int* A0,
+                     const int* s0, bool* on) {
+        constexpr int kN = decltype(kn)::value;
         const int db = d0 + 32;
-        nblk += ns;
-        // The exit bound is tested after every other block (blocks 0, 2, 4,
-        // ...), lanes past their row end retire after every block.  A scan
-        // whose bound holds only runs further invisible steps, which leave A
-        // as it is, so its cv does not change; the bound costs about a
-        // seventh of a block's instructions.
-        const bool tb = ((d0 >> 5) & 1) == 0;
-        if (!tb && !ends) continue;  // no lane can retire: slots and masks stay as they are
-        int T = 0;
+        float h[kN], M[kN];
+        int A[kN], s[kN];
+        uint32_t w[kN];
 #pragma unroll
-        for (int k = 0; k < kG; ++k) {
-            if (k < ns) {
-                const bool a = (act[k] >> lane) & 1;
-                const int myLen = kDir > 0 ? L - 1 - jj[k] : jj[k];
-                bool done = myLen <= db;
-                // active lanes and empty lanes (jj = safe) keep the bound's table reads in range
-                if (tb) done = done | (exit_bound<kDir, false, kCh>(tab, jj[k], L, h[k], db, ytab, invL) <= M[k]);
+        for (int i = 0; i < kN; ++i) {
+            h[i] = row[j[i]] + povh;
+            M[i] = M0[i];
+            A[i] = A0[i];
+            s[i] = s0[i];
+        }
+#pragma unroll
+        for (int i = 0; i < kN; ++i) w[i] = scan_half<kDir>(row + j[i], h[i], ytab, d0, 0, M[i], 0u);
+#pragma unroll
+        for (int i = 0; i < kN; ++i) w[i] = scan_half<kDir>(row + j[i], h[i], ytab, d0, 16, M[i], w[i]);
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            const int myLen = kDir > 0 ? L - 1 - j[i] : j[i];
+            // steps past the row end (the last e of the block) are recorded as
+            // visible; skipped when no lane's row ends in this block
+            if (__builtin_amdgcn_ballot_w64(myLen < db) != 0) {
+                const int e = min(max(db - myLen, 0), 31);
+                w[i] |= (1u << e) - 1u;
+            }
+            if (kLong)
+                flush_runs(w[i], d0, a[i], A[i], s[i]);
+            else
+                flush_block(w[i], d0, A[i], s[i]);
+            on[i] = a[i] && myLen > db;
+            if (on[i]) {
+                smax[id[i]] = M[i];
                 if (kLong) {
-                    if (a && done) {
-                        float cv = __int_as_float(A[k]);
-                        // only invisible steps ahead: a run still open closes at the next one
-                        if (myLen > db && s[k] < 0) cv = add_run(cv, db + 1, __int_as_float(s[k] & 0x7FFFFFFF));
-                        so[jj[k]] = kDir > 0 ? cv : cv * R;
-                    }
-                } else if (a && done) {
-                    const int cv = myLen > db ? A[k] : A[k] - ((db + 1) * (db + 1) - s[k] * s[k]);
+                    sums[id[i]] = A[i];
+                    open[id[i]] = (uint32_t)s[i];
+                    tail[id[i]] = (uint16_t)(db >> 5);
+                } else {
+                    sums[id[i]] = A[i] | (db >> 5) << 24;  // db < L: A <= (db + 1)^2 < 2^24
+                    tail[id[i]] = (uint16_t)s[i];
+                }
+            } else if (a[i]) {
+                if (kLong) {
+                    const float cv = __int_as_float(A[i]);
+                    so[j[i]] = kDir > 0 ? cv : cv * R;
+                } else {
+                    const int cv = A[i] - ((db + 1) * (db + 1) - s[i] * s[i]);
                     if (kDir > 0)
-                        soi[jj[k]] = cv;
+                        soi[j[i]] = cv;
                     else
-                        so[jj[k]] = (float)(cv + soi[jj[k]]) * R;
-                }
-                const bool live = a && !done;
-                act[k] = __builtin_amdgcn_ballot_w64(live);
-                jj[k] = live ? jj[k] : safe;
-                T += (int)__popcll(act[k]);
-            }
-        }
-        T = __builtin_amdgcn_readfirstlane(T);
-        const int nn = (T + 63) >> 6;
-        if (nn < ns) {
-            // live scans before each slot (wave-uniform), from the masks as
-            // they were before any slot is rewritten
-            uint64_t am[kG];
-            int pre[kG];
-            int acc = 0;
-#pragma unroll
-            for (int k = 0; k < kG; ++k) {
-                am[k] = k < ns ? act[k] : 0ull;
-                pre[k] = acc;
-                acc += (int)__popcll(am[k]);
-            }
-#pragma unroll
-            for (int k2 = 0; k2 < kG; ++k2) {
-                if (k2 < nn) {
-                    // the p-th live scan lies in the last slot k with pre[k] <= p
-                    // (k >= k2, since p >= 64 k2 >= pre[k2]) at its (p - pre[k])-th live lane
-                    const int p = 64 * k2 + lane;
-                    uint64_t m = am[k2];
-                    int base = pre[k2], sk = k2;
-#pragma unroll
-                    for (int k = k2 + 1; k < kG; ++k) {
-                        if (k < ns && p >= pre[k]) {
-                            m = am[k];
-                            base = pre[k];
-                            sk = k;
-                        }
-                    }
-                    if (p >= T) sk = -1;  // lane left empty
-                    const int sa = nth_set_bit(m, p >= T ? 0 : p - base) << 2;  // ds_bpermute byte address
-                    int nj = safe, nA = kA0, nS = kS0;
-                    float nh = 0.0f, nM = -2000.0f;
-#pragma unroll
-                    for (int k = k2; k < kG; ++k) {
-                        if (k < ns) {
-                            const int tj = __builtin_amdgcn_ds_bpermute(sa, jj[k]);
-                            const int tA = __builtin_amdgcn_ds_bpermute(sa, A[k]);
-                            const int tS = __builtin_amdgcn_ds_bpermute(sa, s[k]);
-                            const int th = __builtin_amdgcn_ds_bpermute(sa, __float_as_int(h[k]));
-                            const int tM = __builtin_amdgcn_ds_bpermute(sa, __float_as_int(M[k]));
-                            if (sk == k) {
-                                nj = tj;
-                                nA = tA;
-                                nS = tS;
-                                nh = __int_as_float(th);
-                                nM = __int_as_float(tM);
-                            }
-                        }
-                    }
-                    jj[k2] = nj;
-                    A[k2] = nA;
-                    s[k2] = nS;
-                    h[k2] = nh;
-                    M[k2] = nM;
-                    act[k2] = __builtin_amdgcn_ballot_w64(p < T);
+                        so[j[i]] = (float)(cv + soi[j[i]]) * R;
                 }
             }
-            ns = nn;
         }
+        nblk += kN;
+    };
+    // kN batches of the first block: chunks k, k + 1, ..; the live list so far.
+    int n = 0;  // live scans (wave-uniform)
+    auto first = [&](auto kn, int k) {
+        constexpr int kN = decltype(kn)::value;
+        bool a[kN], on[kN];
+        int id[kN], j[kN], A[kN], s[kN];
+        float M[kN];
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            id[i] = 64 * (k + i) + lane;
+            j[i] = jb + id[i];
+            const int myLen = kDir > 0 ? L - 1 - j[i] : j[i];
+            const bool in = j[i] < L;
+            a[i] = in && myLen > 0;
+            if (in && !a[i]) {  // no targets in this direction: cv = 0
+                if (kDir > 0)
+                    soi[j[i]] = 0;
+                else
+                    so[j[i]] = (kLong ? so[j[i]] : (float)soi[j[i]]) * R;
+            }
+            // A counts the observer's own cell; long rows go on with the right
+            // scan's sum, visible from d = 0
+            A[i] = kLong ? (kDir < 0 && a[i] ? __float_as_int(so[j[i]]) : 0) : 1;
+            s[i] = kLong ? (int)0x80000000 : 0;
+            if (!a[i]) j[i] = safe;
+            M[i] = -2000.0f;
+        }
+        block(kn, a, id, j, 0, M, A, s, on);
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64(on[i]);
+            if (on[i]) live[n + lanes_below(m)] = (uint16_t)id[i];
+            n += (int)__popcll(m);
+        }
+    };
+    {
+        int k = 0;
+        for (; k + 2 <= nck; k += 2) first(std::integral_constant<int, 2>{}, k);
+        if (k < nck) first(std::integral_constant<int, 1>{}, k);
+    }
+    for (int d0 = 32; n > 0; d0 += 32) {
+        const int db = d0 + 32, e = d0 + 1;
+        const bool far = ((d0 >> 5) & 1) != 0;  // rounds that test the exit
+        const float y1 = ytab[e].x, y32 = ytab[e + 31].x;
+        int nn = 0, nt = 0;
+        auto test = [&](auto kn, int b) {
+            constexpr int kN = decltype(kn)::value;
+            bool a[kN], need[kN], done[kN];
+            int id[kN], j[kN];
+            float M[kN], h[kN];
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                a[i] = b + 64 * i + lane < n;
+                id[i] = live[b + 64 * i + lane];
+            }
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                id[i] = a[i] ? id[i] : 0;
+                j[i] = a[i] ? jb + id[i] : safe;
+                M[i] = smax[id[i]];
+                h[i] = row[j[i]] + povh;
+                // the block's cells lie in two chunks at most
+                const float a1 = tab_at(tab, j[i] + kDir * e)[kDir > 0 ? kTabL1 : kTabL1 - kTabWords] - h[i];
+                float bnd = fmaxf(a1 * y1, a1 * y32);
+                bnd = __builtin_fmaf(fabsf(bnd), 9.5367431640625e-7f, bnd);
+                need[i] = a[i] && bnd > M[i];
+                done[i] = false;
+            }
+            if (far) {
+#pragma unroll
+                for (int i = 0; i < kN; ++i)
+                    done[i] = exit_bound<kDir, false, kCh>(tab, j[i], L, h[i], d0, ytab, invL) <= M[i];
+            }
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                const int myLen = kDir > 0 ? L - 1 - j[i] : j[i];
+                const bool run = need[i] && !done[i];
+                if (a[i] && !run && (done[i] || myLen <= db)) over(id[i], j[i]);
+                const uint64_t mr = __builtin_amdgcn_ballot_w64(run);
+                if (run) todo[nt + lanes_below(mr)] = (uint16_t)id[i];
+                nt += (int)__popcll(mr);
+                const bool on = a[i] && !done[i] && myLen > db;
+                const uint64_t ml = __builtin_amdgcn_ballot_w64(on);
+                if (on) live[nn + lanes_below(ml)] = (uint16_t)id[i];
+                nn += (int)__popcll(ml);
+            }
+        };
+        auto run = [&](auto kn, int b) {
+            constexpr int kN = decltype(kn)::value;
+            bool a[kN], on[kN];
+            int id[kN], j[kN], A[kN], s[kN];
+            float M[kN];
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                a[i] = b + 64 * i + lane < nt;
+                id[i] = todo[b + 64 * i + lane];
+            }
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                id[i] = a[i] ? id[i] : 0;
+                j[i] = a[i] ? jb + id[i] : safe;
+                M[i] = smax[id[i]];
+                A[i] = sums[id[i]];
+                if (kLong) {
+                    s[i] = (int)open[id[i]];
+                    const int last = 32 * tail[id[i]];
+                    if (a[i] && s[i] < 0 && last != d0) {  // blocks left out since: the open run closed after `last`
+                        A[i] = __float_as_int(
+                            add_run(__int_as_float(A[i]), last + 1, __int_as_float(s[i] & 0x7FFFFFFF)));
+                        s[i] &= 0x7FFFFFFF;
+                    }
+                } else {
+                    s[i] = 32 * (A[i] >> 24) == d0 ? (int)tail[id[i]] : d0 + 1;
+                    A[i] &= 0xFFFFFF;
+                }
+            }
+            block(kn, a, id, j, d0, M, A, s, on);
+        };
+        int b = 0;
+        for (; b + 64 < n; b += 128) test(std::integral_constant<int, 2>{}, b);
+        if (b < n) test(std::integral_constant<int, 1>{}, b);
+        b = 0;
+        for (; b + 64 < nt; b += 128) run(std::integral_constant<int, 2>{}, b);
+        if (b < nt) run(std::integral_constant<int, 1>{}, b);
+        n = __builtin_amdgcn_readfirstlane(nn);
     }
 }
 
+// LDS of the bit-block kernels: the waves' pools, guard band, row, guard band,
+// chunk tables.
+template <bool kLong>
+__host__ __device__ inline int sdem_pools(int maxL, int group, int waves) {
+    return group > 1 ? waves * 64 * pool_cap<kLong>(maxL, waves) * pool_bytes<kLong>() : 0;
+}
+inline size_t sdem_bits_lds(int maxL, int group, int waves) {
+    return sdem_pools<false>(maxL, group, waves) +
+           sizeof(float) * ((size_t)maxL + 2 * (group > 1 ? pad_bits<4>() : pad_bits<1>()) + tab_words(maxL));
+}
+inline size_t sdem_long_lds(int maxL, int waves) {
+    return sdem_pools<true>(maxL, 4, waves) +
+           sizeof(float) * ((size_t)maxL + 2 * pad_bits<4>() + tab_words(maxL));
+}
+
 // One skewed row: stage it, then every wave of the workgroup takes chunks
-// of 64 observers (kG = 1), or groups of kG chunks with lane compaction,
-// handed out by an LDS counter.  Ends with a barrier so the caller may
+// of 64 observers (kG = 1), or pools of chunks, handed out by an LDS counter.  Ends with a barrier so the caller may
 // restage LDS.
-template <int kWaves, int kG, bool kLong = false>
+template <int kWaves, int kG, bool kCheck, bool kLong = false>
 __device__ __forceinline__ void sdem_bits_row(const RowWork w, const SecDesc* __restrict__ secs,
                                               const float* __restrict__ in4, const int* __restrict__ target,
                                               const float* __restrict__ weight, const uint32_t* __restrict__ fl,
                                               const float* __restrict__ Sbuf, const float4* __restrict__ rtab,
-                                              float povh, float* __restrict__ arena, float* row,
+                                              float povh, float* __restrict__ arena, char* pools, int pools_bytes,
                                               unsigned long long* __restrict__ steps, int* gnext) {
+    float* const row = reinterpret_cast<float*>(pools + pools_bytes) + pad_bits<kG>();
     const SecDesc sd = secs[w.sec];
     const int r = w.row;
     const uint32_t v = fl[sd.rows + r];
     const int f = fl_first(v);
     const int L = fl_last(v) - f;
     if (L <= 0) return;  // uniform; the work list holds only rows with L > 0
-    stage_row(row, sd, r, f, L, in4, target, weight, Sbuf, pad_bits<kG, kLong>());
+    stage_row(row, sd, r, f, L, in4, target, weight, Sbuf, pad_bits<kG>());
     if (kG > 1 && threadIdx.x == 0) *gnext = kWaves;
     __syncthreads();
     const int nchunk = (L + 63) >> 6;
     float* so = arena + sd.so + (size_t)r * sd.dim_i + f;
-    if (kLong) {
+    float* tab = row + L + pad_bits<kG>();  // past the right guard band
+    const bool plain = row_tables<kWaves, kLong ? kChunksLong : kChunksMax, kCheck>(row, L, tab);
+    if (kCheck && !(plain && fabsf(povh) <= 1e30f)) {
         // The bit of a step is the sign of M - q, which is not q > M once a
         // difference is infinite or no number.  Heights in [-FLT_MAX, 1e30]
         // keep every one finite (1e30 is below half an ulp of FLT_MAX); a row
         // with any other takes the per-step scans.
-        bool plain = fabsf(povh) <= 1e30f;
-        for (int i = threadIdx.x; i < L; i += 64 * kWaves) plain &= row[i] >= -FLT_MAX && row[i] <= 1e30f;
-        if (!__syncthreads_and(plain)) {
-            for (int c = threadIdx.x >> 6; c < nchunk; c += kWaves)
-                sdem_steps_chunk<0>(row, L, c, povh, rtab, so, sd.R);
-            return;
-        }
+        for (int c = threadIdx.x >> 6; c < nchunk; c += kWaves)
+            sdem_steps_chunk<0>(row, L, c, povh, rtab, so, sd.R);
+        __syncthreads();
+        return;
     }
-    float* tab = row + L + pad_bits<kG, kLong>();  // past the right guard band
-    row_tables<kWaves, kLong ? kChunksLong : kChunksMax>(row, L, tab);
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     int nblk = 0;  // 32-step blocks this wave ran (both directions)
     if (kG > 1) {
-        const int ngroups = (nchunk + kG - 1) / kG;
-        for (int g = wave; g < ngroups;) {
-            const int c0 = g * kG;
-            const int nck = min(kG, nchunk - c0);
-            scan_group<+1, kG, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
-            scan_group<-1, kG, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, nblk);
+        const int cap = pools_bytes / (64 * kWaves * pool_bytes<kLong>());
+        const int per = pool_chunks(nchunk, kWaves, cap), stride = 64 * per;
+        const int npools = (nchunk + per - 1) / per;
+        for (int g = wave; g < npools;) {
+            const int c0 = g * per;
+            const int nck = min(per, nchunk - c0);
+            char* st = pools + wave * pool_bytes<kLong>() * stride;
+            scan_pool<+1, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, st, stride, nblk);
+            scan_pool<-1, kLong>(row, L, povh, c0, nck, tab, rtab, so, sd.R, st, stride, nblk);
             int ng = 0;
             if (lane == 0) ng = atomicAdd(gnext, 1);
             g = __builtin_amdgcn_readfirstlane(ng);
@@ -677,7 +769,7 @@ __device__ __forceinline__ void sdem_bits_row(const RowWork w, const SecDesc* __
 }
 
 // One workgroup per row of the work list.
-template <int kWaves, int kG>
+template <int kWaves, int kG, bool kCheck>
 __global__ __launch_bounds__(64 * kWaves) void k_op_sdem_bits(const SecDesc* __restrict__ secs,
                                                               const RowWork* __restrict__ work,
                                                               const float* __restrict__ in4,
@@ -686,35 +778,35 @@ __global__ __launch_bounds__(64 * kWaves) void k_op_sdem_bits(const SecDesc* __r
                                                               const uint32_t* __restrict__ fl,
                                                               const float* __restrict__ Sbuf,
                                                               const float4* __restrict__ rtab, float povh,
-                                                              float* __restrict__ arena,
+                                                              float* __restrict__ arena, int pools,
                                                               unsigned long long* __restrict__ steps) {
-    extern __shared__ float lds[];
+    extern __shared__ double lds8[];
     __shared__ int gnext;
-    sdem_bits_row<kWaves, kG>(work[blockIdx.x], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
-                              lds + pad_bits<kG>(), steps, &gnext);
+    sdem_bits_row<kWaves, kG, kCheck>(work[blockIdx.x], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
+                              reinterpret_cast<char*>(lds8), pools, steps, &gnext);
 }
 
 // Rows past 4096 cells (see flush_runs), one workgroup per row.  Bound by VALU,
-// like the shorter rows.  Eight waves share a staged row and its tables (64 KB
-// and 13 KB at the longest), so that two workgroups fill a CU.  Twelve sectors
-// of a 4600^2 DEM: 256 ms with every step of every scan (k_op_sdem), 43 ms
+// like the shorter rows.  Eight waves share a staged row and its tables (18 KB
+// and 6 KB at 4600 cells, 64 and 17 KB at the longest).  Twelve sectors
+// of a 4600^2 DEM: 256 ms with every step of every scan (k_op_sdem), 32 ms
 // here.
 constexpr int kLongWaves = 8;
 __global__ __launch_bounds__(64 * kLongWaves) void k_op_sdem_long(
     const SecDesc* __restrict__ secs, const RowWork* __restrict__ work, const float* __restrict__ in4,
     const int* __restrict__ target, const float* __restrict__ weight, const uint32_t* __restrict__ fl,
     const float* __restrict__ Sbuf, const float4* __restrict__ rtab, float povh, float* __restrict__ arena,
-    unsigned long long* __restrict__ steps) {
-    extern __shared__ float lds[];
+    int pools, unsigned long long* __restrict__ steps) {
+    extern __shared__ double lds8[];
     __shared__ int gnext;
-    sdem_bits_row<kLongWaves, 4, true>(work[blockIdx.x], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
-                                       lds + pad_bits<4, true>(), steps, &gnext);
+    sdem_bits_row<kLongWaves, 4, true, true>(work[blockIdx.x], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
+                                       reinterpret_cast<char*>(lds8), pools, steps, &gnext);
 }
 
 static hipError_t launch_op_sdem_long(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
                                       const float4* rtab, float povh, unsigned long long* steps, hipStream_t s) {
-    hipLaunchKernelGGL(k_op_sdem_long, dim3(p.nwork), dim3(64 * kLongWaves), sdem_long_lds(p.maxL), s, p.secs, p.work,
-                       in4, p.target, p.weight, p.fl, Sbuf, rtab, povh, arena, steps);
+    hipLaunchKernelGGL(k_op_sdem_long, dim3(p.nwork), dim3(64 * kLongWaves), sdem_long_lds(p.maxL, kLongWaves), s, p.secs, p.work,
+                       in4, p.target, p.weight, p.fl, Sbuf, rtab, povh, arena, sdem_pools<true>(p.maxL, 4, kLongWaves), steps);
     return hipGetLastError();
 }
 
@@ -728,8 +820,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kOc
     const SecDesc* __restrict__ secs, const RowWork* __restrict__ work, int nwork, int* __restrict__ counter,
     const float* __restrict__ in4, const int* __restrict__ target, const float* __restrict__ weight,
     const uint32_t* __restrict__ fl, const float* __restrict__ Sbuf, const float4* __restrict__ rtab, float povh,
-    float* __restrict__ arena, unsigned long long* __restrict__ steps) {
-    extern __shared__ float lds[];
+    float* __restrict__ arena, int pools, unsigned long long* __restrict__ steps) {
+    extern __shared__ double lds8[];
     __shared__ int item, gnext;
     for (;;) {
         if (threadIdx.x == 0) item = atomicAdd(counter, 1);
@@ -737,8 +829,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kOc
         const int it = __builtin_amdgcn_readfirstlane(item);  // the same value in every lane
         __syncthreads();  // every lane has read `item` before thread 0 overwrites it
         if (it >= nwork) break;
-        sdem_bits_row<kWaves, kG>(work[it], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
-                                  lds + pad_bits<kG>(), steps, &gnext);
+        sdem_bits_row<kWaves, kG, false>(work[it], secs, in4, target, weight, fl, Sbuf, rtab, povh, arena,
+                                  reinterpret_cast<char*>(lds8), pools, steps, &gnext);
     }
 }
 
@@ -753,8 +845,10 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
     if (p.nwork == 0) return hipSuccess;
     if (p.maxL > 32 * kChunksMax) return launch_op_sdem_long(p, in4, Sbuf, arena, rtab, povh, steps, s);
     const int G = t.group > 1 ? 4 : 1;
-    const size_t lds = sdem_bits_lds(p.maxL, G);
-    if (t.persistent_wgs_per_cu > 0 && counter) {
+    const int W = t.waves == 2 || t.waves == 8 ? t.waves : 4;
+    const size_t lds = sdem_bits_lds(p.maxL, G, W);
+    const int pools = sdem_pools<false>(p.maxL, G, W);
+    if (t.persistent_wgs_per_cu > 0 && counter && !t.check) {
         int dev = 0, ncu = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return e;
@@ -764,7 +858,7 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
         const int grid = std::min(p.nwork, ncu * t.persistent_wgs_per_cu);
 #define SKE_PERS(W, O, G)                                                                                        \
     hipLaunchKernelGGL((k_op_sdem_bits_persistent<W, O, G>), dim3(grid), dim3(64 * W), lds, s, p.secs, p.work,    \
-                       p.nwork, counter, in4, p.target, p.weight, p.fl, Sbuf, rtab, povh, arena, steps)
+                       p.nwork, counter, in4, p.target, p.weight, p.fl, Sbuf, rtab, povh, arena, pools, steps)
 #define SKE_PERS_W(O, G)                                                                                         \
     if (t.waves == 2) SKE_PERS(2, O, G); else if (t.waves == 8) SKE_PERS(8, O, G); else SKE_PERS(4, O, G)
 #define SKE_PERS_G(O)                                                                                            \
@@ -781,13 +875,15 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
 #undef SKE_PERS
         return hipGetLastError();
     }
-#define SKE_GRID(W, G)                                                                                            \
-    hipLaunchKernelGGL((k_op_sdem_bits<W, G>), dim3(p.nwork), dim3(64 * W), lds, s, p.secs, p.work, in4, p.target, \
-                       p.weight, p.fl, Sbuf, rtab, povh, arena, steps)
-    if (G == 4) {
-        if (t.waves == 2) SKE_GRID(2, 4); else if (t.waves == 8) SKE_GRID(8, 4); else SKE_GRID(4, 4);
+#define SKE_GRID(W, G, C)                                                                                         \
+    hipLaunchKernelGGL((k_op_sdem_bits<W, G, C>), dim3(p.nwork), dim3(64 * W), lds, s, p.secs, p.work, in4, p.target, \
+                       p.weight, p.fl, Sbuf, rtab, povh, arena, pools, steps)
+    if (G == 4 && t.check) {
+        if (t.waves == 2) SKE_GRID(2, 4, true); else if (t.waves == 8) SKE_GRID(8, 4, true); else SKE_GRID(4, 4, true);
+    } else if (G == 4) {
+        if (t.waves == 2) SKE_GRID(2, 4, false); else if (t.waves == 8) SKE_GRID(8, 4, false); else SKE_GRID(4, 4, false);
     } else {
-        if (t.waves == 2) SKE_GRID(2, 1); else if (t.waves == 8) SKE_GRID(8, 1); else SKE_GRID(4, 1);
+        if (t.waves == 2) SKE_GRID(2, 1, false); else if (t.waves == 8) SKE_GRID(8, 1, false); else SKE_GRID(4, 1, false);
     }
 #undef SKE_GRID
     return hipGetLastError();
@@ -798,9 +894,9 @@ hipError_t launch_op_sdem(const DevPlan& p, const float* in4, const float* Sbuf,
     if (p.nwork == 0) return hipSuccess;
     if (variant == 0) {
         if (p.maxL > 32 * kChunksMax) return launch_op_sdem_long(p, in4, Sbuf, arena, rtab, povh, nullptr, s);
-        const size_t lds = sdem_bits_lds(p.maxL);
-        hipLaunchKernelGGL((k_op_sdem_bits<4, 1>), dim3(p.nwork), dim3(256), lds, s, p.secs, p.work, in4, p.target,
-                           p.weight, p.fl, Sbuf, rtab, povh, arena, nullptr);
+        const size_t lds = sdem_bits_lds(p.maxL, 1, 4);
+        hipLaunchKernelGGL((k_op_sdem_bits<4, 1, false>), dim3(p.nwork), dim3(256), lds, s, p.secs, p.work, in4, p.target,
+                           p.weight, p.fl, Sbuf, rtab, povh, arena, 0, nullptr);
         return hipGetLastError();
     }
     const size_t lds = sizeof(float) * (size_t)(p.maxL + 2 * kPad);

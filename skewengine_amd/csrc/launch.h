@@ -28,7 +28,8 @@ struct SdemTuning {
     int waves = 4;                 // waves per workgroup (observer chunks of one row in parallel): 2, 4 or 8
     int persistent_wgs_per_cu = 0; // 0: one workgroup per row; >0: persistent grid of this many per CU
     int occupancy = 0;             // persistent grid: 8 = compile for 8 waves per SIMD (fewer VGPRs)
-    int group = 4;                 // 1: one 64-observer chunk per wave; 4: groups of 4 chunks, lane compaction
+    int group = 4;                 // 1: one 64-observer chunk per wave; 4: pools of up to 4 chunks
+    bool check = false;            // rows may hold heights that are not finite or above 1e30 (pools, grid launch)
 };
 
 // Graph-safe clears (kernels, not hipMemsetAsync).
@@ -36,7 +37,8 @@ hipError_t launch_fill_f32(float* p, size_t n, float v, hipStream_t s);
 hipError_t launch_fill_f64(double* p, size_t n, hipStream_t s);
 
 // prepare(): the three mirrored/transposed copies (src/skewEngine.cuh:962-987).
-hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, int dimx, int dimy,
+// odd (may be null): set to 1 when a value is not finite or above 1e30.
+hipError_t launch_prepare(const float* in0, float* in1, float* in2, float* in3, int dimx, int dimy, int* odd,
                           hipStream_t s);
 
 // Materialise the skewInput rows (H*dim_i) of one sector; cells without a

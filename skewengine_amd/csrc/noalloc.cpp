@@ -233,7 +233,7 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
 
     // Oriented copies of the caller's grid (prepare) and cleared accumulators.
     SKE_HIP(hipMemcpyAsync(in4, d_input, N * sizeof(float), hipMemcpyDeviceToDevice, stream));
-    SKE_HIP(launch_prepare(in4, in4 + N, in4 + 2 * N, in4 + 3 * N, n, n, stream));
+    SKE_HIP(launch_prepare(in4, in4 + N, in4 + 2 * N, in4 + 3 * N, n, n, nullptr, stream));
     SKE_HIP(launch_fill_f32(acc, 4 * N, 0.0f, stream));
     SKE_HIP(launch_fill_f32(reinterpret_cast<float*>(counter), 16, 0.0f, stream));  // zero bits
     for (NaChunk& ch : chunks) {
@@ -262,12 +262,16 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
         v.maxI = ch.ip.maxI;
         switch (kernel_id) {
         case SKE_KERNEL_SDEM: {
-            // the engine's default launch shape (two waves for short rows)
-            SdemTuning t;
-            const int nchunks = (v.maxL + 63) / 64;
-            const int units = (nchunks + t.group - 1) / t.group;
-            t.waves = units < 4 ? 2 : 4;
-            SKE_HIP(launch_op_sdem_tuned(v, in4, nullptr, arena, rtab, povh, t, counter, nullptr, stream));
+            for (const SdemRun& r : sdem_runs(ch.ip)) {  // the engine's default launches
+                DevPlan p = v;
+                p.work += r.first;
+                p.nwork = r.count;
+                p.maxL = r.maxL;
+                SdemTuning t;
+                t.waves = r.waves;
+                t.check = true;  // the input has not been looked at on the host
+                SKE_HIP(launch_op_sdem_tuned(p, in4, nullptr, arena, rtab, povh, t, counter, nullptr, stream));
+            }
             break;
         }
         case SKE_KERNEL_CEPSTRUM:

@@ -178,6 +178,31 @@ void plan_one(int dimx, int dimy, const SectorPlan& sp, ImagePlan& ip) {
     });
 }
 
+std::vector<SdemRun> sdem_runs(const ImagePlan& ip) {
+    constexpr int kLong = 4096, kRows = 2048;
+    const int bounds[] = {kLong, 3328, 2048, 1024, 0};
+    std::vector<SdemRun> runs;
+    int cls = -1;
+    for (int i = 0; i < (int)ip.work.size(); i++) {
+        const RowWork& w = ip.work[i];
+        const uint32_t v = ip.fl[ip.secs[w.sec].rows + w.row];
+        const int L = (int)(v >> 16) - (int)(v & 0xffffu);
+        int c = 0;
+        while (L <= bounds[c] && bounds[c] > 0) c++;
+        if (runs.empty() || (c != cls && (runs.back().count >= kRows || runs.back().maxL > kLong)))
+            runs.push_back(SdemRun{i, 0, L, 0});
+        cls = c;
+        runs.back().count++;
+        runs.back().maxL = std::max(runs.back().maxL, L);
+    }
+    if (runs.size() > 1 && runs.back().count < kRows && runs[runs.size() - 2].maxL <= kLong) {
+        runs[runs.size() - 2].count += runs.back().count;
+        runs.pop_back();
+    }
+    for (SdemRun& r : runs) r.waves = r.maxL <= 1024 ? 2 : r.maxL <= 3328 ? 4 : 8;
+    return runs;
+}
+
 void recip_table(int n, std::vector<float>& tab4) {
     tab4.assign(4 * (size_t)n + 2 * ((size_t)n + 32), 0.0f);
     float* tab2 = tab4.data() + 4 * (size_t)n;

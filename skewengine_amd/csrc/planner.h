@@ -65,6 +65,21 @@ void plan_one(int dimx, int dimy, const SectorPlan& sp, ImagePlan& ip);
 void plan_append(int dimx, int dimy, int s0, int s1, long long img, ImagePlan& ip, int range8[8]);
 void plan_finish(ImagePlan& ip, int order);
 
+// A run of the viewshed's row list (rows by descending length) that one launch
+// takes: its LDS is sized to the run's longest row, and more waves share a
+// longer row while fewer keep the pools of a short row large (kernels_sdem.hip).
+// Measured with one launch: all sectors of 500^2 2 waves 1.74 ms, 4 waves 2.34;
+// 1000^2 9.9, 10.5; 1501^2 29.3, 29.2 (8 waves 33.8); 30 of 3000^2 4 waves 25,
+// 8 waves 27.7; 20 of 4000^2 33.1, 30.7.  Cut into runs (default waves):
+// 1000^2 10.2 ms, 1501^2 28.6, 3000^2 24.5, 4000^2 31.2 (whole list 30.7 to 33),
+// a batch of 1000^2 .. 4000^2 556 -> 545, 12 of 4600^2 36 -> 32.
+struct SdemRun {
+    int first, count, maxL, waves;
+};
+// Runs end where the length passes 4096 (rows with other sums), 3328, 2048 or
+// 1024 cells, and hold at least 2048 rows (eight per CU) if there are as many.
+std::vector<SdemRun> sdem_runs(const ImagePlan& ip);
+
 // {RN(1/d), RN(1/d - RN(1/d)), d, d*d} for d = 0..n-1, followed by the
 // pairs {RN(1/d), RN(1/d - RN(1/d))} for d = 0..n+31 (the viewshed's
 // block-preloaded table).

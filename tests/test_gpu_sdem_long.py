@@ -51,3 +51,35 @@ def test_long_rows_with_special_heights(value):
             out = e.run(ske.KERNEL_SDEM, s0, s0 + 1)
             e.set_option(_lib.OPT_SDEM_VARIANT, 2)
             assert np.array_equal(out, e.run(ske.KERNEL_SDEM, s0, s0 + 1), equal_nan=True), (value, s0)
+
+
+@pytest.mark.parametrize("n,s0,s1", [(1100, 0, 180), (2100, 40, 60), (3400, 44, 48), (4300, 44, 46)])
+def test_runs_by_row_length_match_per_step_kernel(n, s0, s1):
+    """Row lists that cross 1024, 2048, 3328 and 4096 cells, one launch each."""
+    g = _terrain("fbm", n)
+    with ske.SkewEngine(g) as e:
+        out = e.run(ske.KERNEL_SDEM, s0, s1)
+        e.set_option(_lib.OPT_SDEM_VARIANT, 2)
+        assert np.array_equal(out, e.run(ske.KERNEL_SDEM, s0, s1))
+
+
+def test_runs_of_an_uneven_batch():
+    gs = [_terrain("fbm", n) for n in (150, 1100, 2500, 90)]
+    with ske.SkewBatch(gs) as b:
+        b.run(ske.KERNEL_SDEM, 30, 60)
+        outs = b.outputs()
+    for g, out in zip(gs, outs):
+        with ske.SkewEngine(g) as e:
+            e.set_option(_lib.OPT_SDEM_VARIANT, 2)
+            assert np.array_equal(out, e.run(ske.KERNEL_SDEM, 30, 60)), g.shape
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, -3.4028235e38])
+def test_rows_with_special_heights_take_the_per_step_scans(value):
+    g = synth.dem(128, 0.8, 3, 1500.0)[:100, :100].copy()
+    at = np.random.default_rng(1).integers(0, 100, (40, 2))
+    g[at[:, 0], at[:, 1]] = value
+    with ske.SkewEngine(g) as e:
+        out = e.run(ske.KERNEL_SDEM)
+        e.set_option(_lib.OPT_SDEM_VARIANT, 2)
+        assert np.array_equal(out, e.run(ske.KERNEL_SDEM), equal_nan=True)
