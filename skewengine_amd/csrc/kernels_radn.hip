@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void k_radn_rowsum(const SecDesc* __restrict__
     if (lane == 0) P[sd.q + w.row] = acc;
 }
 
-// The fused row sums (no materialised skewInput): one wave per 64
-// consecutive skewed rows of one sector, lane = row.  Each lane adds
+// The fused row sums (no materialised skewInput): one wave per 63
+// consecutive skewed rows of one sector, lane = row (lane 0 the row before).  Each lane adds
 // S(r, j) over its own [first, last) in ascending j in double -- the
 // reference's own order (kernelRADN.h:227-232), so P is the reference's sum
 // bit for bit -- with S(r, j) computed as skew_cell does.  The two taps of
@@ -80,38 +80,40 @@ __global__ __launch_bounds__(256) void k_radn_rowsum(const SecDesc* __restrict__
 //   type 0: in0[a][j] = in2[j][dimy-1-a]        type 1: in1[a][j] = in3[dimy-1-j][a]
 //   type 2: in2[a][j] = in0[dimy-1-j][a]        type 3: in3[a][j] = in2[dimx-1-j][dimy-1-a]
 // so at every j the 64 lanes' taps are 64 consecutive floats of one row and
-// t_j, w_j are wave-uniform (scalar loads).  The byte offset of the lane's
-// lower-addressed tap is A + B j + C t_j + D: three sector constants and a
+// t_j, w_j are wave-uniform (scalar loads).  A lane loads the tap of row r - t_j
+// and takes that of row r - t_j - 1 from the lane before, whose row is r - 1.
+// The tap's byte offset is A + B j + C t_j + D: three sector constants and a
 // per-lane term.  The wave walks the union of its rows' ranges; cells
 // outside a lane's own range are read but add zero (acc + 0 = acc: acc is
 // never -0).
 constexpr int kColsUnroll = 8;
-// Columns [j0, j1) of the walk, adding to acc.  kMask: test the lane's own
-// [f, l) (columns where some lane of the wave is outside its range).  The
+// Columns [j0, j1) of the walk, adding to acc.  Unless kInner (every lane inside
+// its range and both taps inside the image) the lane's own [f, l) and the taps'
+// rows are tested.  The
 // first tap's value is w * x1 without the reference's 0 + (it differs only
 // in the sign of a zero, which no later sum can see: acc is never -0).
-template <bool kRev, bool kMask>
+template <bool kInner>
 __device__ __forceinline__ void rowsum_cols_span(const int* __restrict__ tt, const float* __restrict__ ww,
                                                  __amdgpu_buffer_rsrc_t src, int A, int B, int C, int D, int r,
                                                  int dim_o, int f, int l, int j0, int j1, double& acc) {
-    auto cell = [&](int j, int t, float w, uint2 pr) -> float {
-        // kRev: the tap of row r - t at the lower address
-        const float x1 = __uint_as_float(kRev ? pr.y : pr.x), x0 = __uint_as_float(kRev ? pr.x : pr.y);
+    auto cell = [&](int j, int t, float w, unsigned tap) -> float {
+        // row r - t, and from the lane before row r - 1 - t
+        const float x0 = __uint_as_float(tap);
+        const float x1 = __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)tap, 0x138, 0xf, 0xf, true));
+        if (kInner) return w * x1 + (1.0f - w) * x0;
         const int i0 = r - t;
         const float s = ((unsigned)(i0 - 1) < (unsigned)dim_o) ? w * x1 : 0.0f;
         const float v = ((unsigned)i0 < (unsigned)dim_o) ? s + (1.0f - w) * x0 : s;
-        return (!kMask || (unsigned)(j - f) < (unsigned)(l - f)) ? v : 0.0f;
+        return (unsigned)(j - f) < (unsigned)(l - f) ? v : 0.0f;
     };
-    auto load = [&](int j, int t) -> uint2 {
-        const int o = A + B * j + C * t + D;
-        return make_uint2(__builtin_amdgcn_raw_buffer_load_b32(src, o, 0, 0),
-                          __builtin_amdgcn_raw_buffer_load_b32(src, o + 4, 0, 0));
+    auto load = [&](int j, int t) -> unsigned {
+        return __builtin_amdgcn_raw_buffer_load_b32(src, A + B * j + C * t + D, 0, 0);
     };
     int j = j0;
     for (; j + kColsUnroll <= j1; j += kColsUnroll) {
         int t[kColsUnroll];
         float w[kColsUnroll];
-        uint2 pr[kColsUnroll];
+        unsigned pr[kColsUnroll];
 #pragma unroll
         for (int u = 0; u < kColsUnroll; ++u) {
             t[u] = tt[j + u];
@@ -128,34 +130,35 @@ __device__ __forceinline__ void rowsum_cols_span(const int* __restrict__ tt, con
     }
 }
 
-// The walk over [lo, hi): columns [fmax, lmin), inside every lane's range,
-// without the range test.
-template <bool kRev>
+// The walk over [lo, hi): columns [ia, ib) without tests.
 __device__ __forceinline__ double rowsum_cols_walk(const int* __restrict__ tt, const float* __restrict__ ww,
                                                    __amdgpu_buffer_rsrc_t src, int A, int B, int C, int D, int r,
-                                                   int dim_o, int f, int l, int lo, int hi, int fmax, int lmin) {
+                                                   int dim_o, int f, int l, int lo, int hi, int ia, int ib) {
     double acc = 0.0;
-    if (fmax < lmin) {
-        rowsum_cols_span<kRev, true>(tt, ww, src, A, B, C, D, r, dim_o, f, l, lo, fmax, acc);
-        rowsum_cols_span<kRev, false>(tt, ww, src, A, B, C, D, r, dim_o, f, l, fmax, lmin, acc);
-        rowsum_cols_span<kRev, true>(tt, ww, src, A, B, C, D, r, dim_o, f, l, lmin, hi, acc);
+    if (ia < ib) {
+        rowsum_cols_span<false>(tt, ww, src, A, B, C, D, r, dim_o, f, l, lo, ia, acc);
+        rowsum_cols_span<true>(tt, ww, src, A, B, C, D, r, dim_o, f, l, ia, ib, acc);
+        rowsum_cols_span<false>(tt, ww, src, A, B, C, D, r, dim_o, f, l, ib, hi, acc);
     } else {
-        rowsum_cols_span<kRev, true>(tt, ww, src, A, B, C, D, r, dim_o, f, l, lo, hi, acc);
+        rowsum_cols_span<false>(tt, ww, src, A, B, C, D, r, dim_o, f, l, lo, hi, acc);
     }
     return acc;
 }
 
 //
-// Bound by latency: the 64 lanes' taps are one partner row, and an L2 miss in
-// any of a pass's eight rows stalls the wave.  Workgroups go to the eight XCDs
+// Bound by VALU (about 18 operations a column with the tests, 9 without) and by
+// L2 misses: the 64 lanes' taps are one partner row, and a miss in any of a
+// pass's eight rows stalls the wave.  Workgroups go to the eight XCDs
 // in turn, so runs of 23 sectors (an image's 180 over all eight; nearly always
 // one partner copy) are laid on one XCD, whose L2 then serves them: 8 x 955^2
 // passes 1,498 -> 855 us.  A workgroup is one wave: rows of a sector differ in
 // length by up to 8 times, and waves that share a workgroup leave their slots
-// to the next one only together.  16 x 512^2: 500 -> 387 us for both.  Not
+// to the next one only together.  16 x 512^2: 500 -> 387 us for both; columns
+// without tests and one load a tap: 387 -> 323 (one 512^2 image 53 -> 43).  Not
 // faster: scalar offsets with two or three taps per load (unaligned wide
-// loads), passes in flight from tables held in lanes (540 to 670 us).
-constexpr int kXcdSectors = 23, kRowsumWaves = 1;
+// loads), passes in flight from tables held in lanes (540 to 670 us), 32
+// columns a pass for a single image (59).
+constexpr int kXcdSectors = 23, kRowsumWaves = 1, kRowsumRows = 63;
 __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const SecDesc* __restrict__ secs,
                                                           const float* __restrict__ in4,
                                                           const int* __restrict__ target,
@@ -166,11 +169,11 @@ __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const Se
     const int si = (k / kXcdSectors * 8 + (blockIdx.x & 7)) * kXcdSectors + k % kXcdSectors;
     if (si >= nsec) return;
     const SecDesc sd = secs[si];
-    const int r0 = ((at - k * nblk) * kRowsumWaves + (threadIdx.x >> 6)) * 64;
+    const int r0 = ((at - k * nblk) * kRowsumWaves + (threadIdx.x >> 6)) * kRowsumRows;
     if (r0 >= sd.H) return;  // wave-uniform
     const int lane = threadIdx.x & 63;
-    const int r = r0 + lane;
-    const bool live = r < sd.H;
+    const int r = r0 + lane - 1;  // lane 0 only loads its tap for lane 1
+    const bool live = lane > 0 && r < sd.H;
     int f = 0, l = 0;
     if (live) {
         const uint32_t v = fl[sd.rows + r];
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const Se
     if (!(live && l > f)) f = l = 0;  // no cell of this lane is added
     int lo = l > f ? f : INT_MAX, hi = l > f ? l : INT_MIN;
     // [fmax, lmin): inside every lane's range (empty when some lane has none)
-    int fmax = l > f ? f : INT_MAX, lmin = l > f ? l : INT_MIN;
+    int fmax = l > f ? f : lane == 0 ? INT_MIN : INT_MAX, lmin = l > f ? l : lane == 0 ? INT_MAX : INT_MIN;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
         lo = min(lo, __shfl_xor(lo, off, 64));
@@ -192,6 +195,14 @@ __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const Se
     hi = __builtin_amdgcn_readfirstlane(hi);
     fmax = __builtin_amdgcn_readfirstlane(fmax);
     lmin = __builtin_amdgcn_readfirstlane(lmin);
+    // Both taps of a row r in the image: r - dim_o < t_j < r.  Column j is in the
+    // range of row x only if x - dim_o <= t_j <= x, so the columns from the row
+    // after the wave's last on, and up to the row before its first, have that.
+    int ia = hi, ib = hi;
+    if (r0 > 0 && r0 + kRowsumRows < sd.H && lo < hi) {
+        ia = max(fmax, __builtin_amdgcn_readfirstlane((int)fl_first(fl[sd.rows + r0 + kRowsumRows])));
+        ib = min(lmin, __builtin_amdgcn_readfirstlane((int)fl_last(fl[sd.rows + r0 - 1])));
+    }
     const int dim_o = sd.dim_o, dim_i = sd.dim_i, type = sd.type;
     const int partner = type == 0 ? 2 : type == 1 ? 3 : type == 2 ? 0 : 2;
     // the partner copy as a raw buffer of N floats: a tap outside it (a row
@@ -200,23 +211,20 @@ __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const Se
         (void*)(in4 + sd.img + (size_t)partner * sd.N), 0, sd.N * 4, kBufferRsrcWord3);
     const int* const tt = target + sd.tab;
     const float* const ww = weight + sd.tab;
-    double acc;
-    if (type == 0)  // partner row j, position dim_o-1-a: tap r-t at 4 (j dim_o + dim_o-1 + t - r)
-        acc = rowsum_cols_walk<true>(tt, ww, src, 4 * (dim_o - 1), 4 * dim_o, 4, -4 * r, r, dim_o, f, l, lo, hi, fmax,
-                                     lmin);
-    else if (type == 3)  // partner row dim_i-1-j, position dim_o-1-a
-        acc = rowsum_cols_walk<true>(tt, ww, src, 4 * ((dim_i - 1) * dim_o + dim_o - 1), -4 * dim_o, 4, -4 * r, r,
-                                     dim_o, f, l, lo, hi, fmax, lmin);
-    else  // types 1, 2: partner row dim_i-1-j, position a: tap r-t-1 at 4 ((dim_i-1-j) dim_o + r - t - 1)
-        acc = rowsum_cols_walk<false>(tt, ww, src, 4 * ((dim_i - 1) * dim_o - 1), -4 * dim_o, -4, 4 * r, r, dim_o,
-                                      f, l, lo, hi, fmax, lmin);
+    // byte offset of tap r - t of column j, row r: A + B j + C t + D r
+    //   type 0: partner row j, position dim_o-1-(r-t)     type 3: partner row dim_i-1-j, the same position
+    //   types 1, 2: partner row dim_i-1-j, position r-t
+    const int D = type == 0 || type == 3 ? -4 : 4;
+    const int A = 4 * ((type == 0 ? 0 : (dim_i - 1) * dim_o) + (D < 0 ? dim_o - 1 : 0));
+    const double acc = rowsum_cols_walk(tt, ww, src, A, type == 0 ? 4 * dim_o : -4 * dim_o, -D, D * r, r, dim_o, f, l,
+                                        lo, hi, ia, ib);
     if (live) P[sd.q + r] = acc;
 }
 
 hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* Sbuf, double* P, hipStream_t s) {
     if (!Sbuf) {  // writes every row r < H of every sector (rows without cells: 0)
         if (p.nsec == 0 || p.maxH <= 0) return hipSuccess;
-        const int nblk = (p.maxH + 64 * kRowsumWaves - 1) / (64 * kRowsumWaves);
+        const int nblk = (p.maxH + kRowsumRows * kRowsumWaves - 1) / (kRowsumRows * kRowsumWaves);
         const unsigned units = (unsigned)(p.nsec + 8 * kXcdSectors - 1) / (8 * kXcdSectors);
         hipLaunchKernelGGL(k_radn_rowsum_cols, dim3(8 * kXcdSectors * units * nblk), dim3(64 * kRowsumWaves), 0, s, p.secs,
                            in4, p.target, p.weight, p.fl, P, p.nsec, nblk);

@@ -35,10 +35,11 @@ def test_few_sectors_match_oracle(s0, s1):
     assert np.array_equal(out, oracle.execute(oracle.SDEM, g, nthreads=1, s0=s0, s1=s1)[0])
 
 
-@pytest.mark.parametrize("n", [2, 7, 50, 131])
+@pytest.mark.parametrize("n", [2, 7, 50, 62, 63, 64, 131, 190])
 @pytest.mark.parametrize("s0,s1", [(0, 180), (0, 1), (45, 46), (3, 25), (3, 26), (80, 104), (1, 180), (0, 8)])
 def test_radon_sector_ranges_match_oracle(n, s0, s1):
-    """Row sums of sector counts around the runs of 23 that share an XCD; filters of 2 to 256 points."""
+    """Row sums around 63 rows a wave, sector counts around the runs of 23 that share an XCD; filters of 2 to 512
+    points."""
     img = np.random.default_rng(n).uniform(0.1, 1.0, (n, n)).astype(np.float32)
     with ske.SkewEngine(img) as e:
         out = e.run(ske.KERNEL_RADON, s0, s1)
