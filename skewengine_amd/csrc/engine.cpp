@@ -12,10 +12,10 @@
 //  * ske_batch: many grids of uneven sizes in one call.
 // All-sector path: every (grid, sector) is planned once; a chunk of them that
 // fits the arena budget gets one operator launch over all its rows (rows are
-// gathered straight from the oriented inputs; the viewshed uses a persistent
-// grid pulling cost-sorted rows off an atomic counter), then one deskew per
-// grid in ascending sector order, and finally one reduce per grid.  The whole
-// sequence can be captured once in a hipGraph and replayed.
+// gathered straight from the oriented inputs; the viewshed gets one launch per
+// run of rows of similar length, longest first, or a persistent grid pulling
+// cost-sorted rows off an atomic counter), then one deskew per grid in
+// ascending sector order, and finally one reduce launch per 64 grids.  The whole sequence can be captured once in a hipGraph and replayed.
 // Results are bit-identical to a one-thread run of the reference CPU path for
 // the viewshed and identity operators, and equal to it up to FP64 rounding
 // for Radon and cepstrum.
@@ -1024,6 +1024,10 @@ int ske_set_kernel(ske_engine* e, int kernel_id, float povh) {
 
 int ske_set_device_operator(ske_engine* e, ske_device_operator op, void* user) {
     if (!e) return fail(SKE_EINVAL, "engine is NULL");
+    if (op && e->have_sector) {  // the current sector's S may be read on any stream from now on
+        SKE_HIP(hipSetDevice(e->core.device));
+        SKE_HIP(hipStreamSynchronize(e->core.stream));
+    }
     e->custom = op;
     e->custom_user = user;
     return SKE_OK;

@@ -79,8 +79,10 @@ int ske_fbp_create(int n, int n_angles, int n_det, const float* angles, int max_
     // not to be had
     const size_t part1 = proj_part_floats(n, n_angles, max_batch, 1);
     const size_t part4 = max_batch > 1 ? proj_part_floats(n, n_angles, std::min(max_batch, 8), 4) : 0;
-    if (part4 <= part1 || part4 * sizeof(float) > (8ull << 30) || f->part.ensure(part4) != SKE_OK)
+    if (part4 <= part1 || part4 * sizeof(float) > (8ull << 30) || f->part.ensure(part4) != SKE_OK) {
+        (void)hipGetLastError();  // of the refused allocation: the next launch would report it
         SKE_TRY(f->part.ensure(part1));
+    }
     SKE_TRY(f->timer.sync(f->stream));
     *out = f.release();
     return SKE_OK;

@@ -1,9 +1,11 @@
 // kernels_sdem.hip -- total-viewshed operator (src/kernelSDEM.h:168-222) on
 // gfx950.
 //
-// Layout: one workgroup (4 waves) per skewed row.  The row is staged once in
-// LDS; each wave takes 64 consecutive observers and runs their right scans
-// then their left scans with a wave-uniform step d = 1, 2, ...  Because d is
+// Layout: one workgroup (2 to 8 waves) per skewed row.  The row is staged once
+// in LDS.  Per-step and one-chunk kernels: each wave takes 64 consecutive
+// observers and runs their right scans then their left scans with a
+// wave-uniform step d = 1, 2, ... (the default kernels take pools of up to four
+// such chunks and skip blocks of steps that cannot be visible: below).  As d is
 // uniform, 1/d and d*d come from a scalar table and every lane reads
 // row[j +/- d] from consecutive LDS words (no bank conflicts).  Each lane
 // keeps the reference's per-observer state (max angle, visible flag, opening

@@ -1,11 +1,15 @@
 """The per-sector calls' table ring: more sectors than slots without a wait
 between them, sides whose ring has 16 and 2 slots, and several engines in turn;
 each sector's result against the all-sector run of that sector alone."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 import skewengine_amd as ske
 from skewengine_amd import synth
+from skewengine_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +46,23 @@ def test_tables_of_the_last_sector():
         for r in range(S.shape[0]):
             j = np.arange(f[r], l[r])
             assert np.array_equal(SO[r, j], S[r, j]) and not SO[r, :f[r]].any() and not SO[r, l[r]:].any()
+
+
+@pytest.mark.parametrize("before", [True, False])
+def test_device_operator_finds_the_sector_ready(before):
+    """An operator may read skewInput on a stream of its own: the engine's is
+    idle when it is called, whether it was set before or after skew()."""
+    form = ctypes.CFUNCTYPE(None, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                            ctypes.c_void_p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p)
+    idle = []
+    op = form(lambda so, s, dim_i, h, last, first, val, angle, stream, user:
+              idle.append(torch.cuda.ExternalStream(stream).query()))
+    with ske.SkewEngine(synth.dem(1024, 0.8, 3, 1500.0)) as e:
+        if before:
+            check(lib().ske_set_device_operator(e._h, ctypes.cast(op, ctypes.c_void_p), None))
+        for a in range(12):
+            e.skew(a)
+        if not before:
+            check(lib().ske_set_device_operator(e._h, ctypes.cast(op, ctypes.c_void_p), None))
+        e.kernel()
+    assert idle == [True]
