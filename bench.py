@@ -34,12 +34,12 @@ sys.path.insert(0, ROOT)
 PEAK_FP32_PUBLISHED = 157.3
 PEAK_VALU_TOPS = PEAK_FP32_PUBLISHED / 2
 OPS_PER_STEP = 4  # sub, divide, compare, max per ray step (src/kernelSDEM.h:191-196)
-# VALU wave instructions per 64 executed lane-steps of the viewshed kernel,
+# VALU wave instructions per 64 executed lane-steps of the viewshed kernels,
 # measured with rocprofv3 --pmc SQ_INSTS_VALU over the bench's timed step
 # (6 per step in the scan, then per 32-step block of a slot the popcount
-# flush, the end-of-row mask, the early-exit bound and the retire/compaction
-# bookkeeping, plus row staging and chunk tables).
-VALU_PER_LANE_STEP = 8.26
+# flush, the end-of-row mask, the early-exit bound, the pools' tests of the
+# next blocks and their packing, plus row staging and chunk tables).
+VALU_PER_LANE_STEP = 10.82
 HBM_PEAK_GBS = 8000.0
 
 
