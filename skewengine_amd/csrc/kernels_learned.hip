@@ -1019,9 +1019,9 @@ __global__ __launch_bounds__(256) void k_conv_mid_bwd_mfma(const float* __restri
 
 // Weight gradient of a conv C -> C layer:
 //   dW[co][t][ci] += sum_p dz[p][co] x[p + off(t)][ci],  db[co] += sum_p dz[p][co].
-// One workgroup per 16 x 16 tile, summed over the slices b = blockIdx.z,
-// blockIdx.z + gridDim.z, ... in registers, then added into grad[] with
-// atomics once.  K = pixels: A[co][p] = dz, split into bf16 hi and lo parts
+// A workgroup goes through 16 x 16 tiles blockIdx.x, blockIdx.x + gridDim.x,
+// ... of all slices, sums in registers, and adds into grad[] with atomics
+// once.  K = pixels: A[co][p] = dz, split into bf16 hi and lo parts
 // (split_bf16) and transposed in LDS ([co][16 rows][16 columns], co stride
 // 272 elements); B[p][ci] = x (bf16, exact), transposed with a one-pixel
 // halo ([ci][18 rows][pitch 24]).  A K block is two tile rows: lane block kb
@@ -1030,9 +1030,66 @@ __global__ __launch_bounds__(256) void k_conv_mid_bwd_mfma(const float* __restri
 // the next 4 bytes and v_alignbyte.  The co stride of A and the ci stride of
 // B keep each 16-byte read cycle on distinct banks.  Wave w takes the taps
 // w, w + 4 and (w = 0) 8.
+// Bound by memory (402 MB of dz and x for 16 x 512^2 at C = 16: 83 us at the
+// rate of a copy) now that loads are 16 bytes wide, two pixels of a few
+// channels a thread, in flight during the previous tile's products, with
+// offsets made once, and the workgroups are as many as stay resident (2,048
+// with loads of one channel took two rounds): 220 -> 105 us.
+
+// The next tile's share of a thread, in registers.
 template <int C>
-__global__ __launch_bounds__(256) void k_wgrad_mfma(const float* __restrict__ dz, const uint16_t* __restrict__ x,
-                                                    float* __restrict__ grad, int woff, int boff, int n, int batch) {
+struct WgradTile {
+    static constexpr int kA = C / 8, kB = (18 * 9 * C / 8 + 255) / 256;  // items of a thread
+    float4 a[kA][2];
+    uint4 x[kB][2];
+
+    int off_a[kA], off_b[kB], edge[kB];
+
+    // A item: columns 2p, 2p + 1 of a row, channels 4g .. +3.  B item: columns 2p - 1, 2p of a halo row,
+    // channels 8g .. +7; edge: the image borders that the item lies beyond if its tile touches them.
+    __device__ __forceinline__ void init(int n) {
+#pragma unroll
+        for (int k = 0; k < kA; k++) {
+            const int t = threadIdx.x + 256 * k;
+            off_a[k] = ((t / (2 * C)) * n + 2 * ((t / (C / 4)) & 7)) * C + 4 * (t % (C / 4));
+        }
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            const int t = threadIdx.x + 256 * k;
+            const int q = t / (C / 8), row = q / 9, p = q - 9 * row;
+            off_b[k] = (row * n + 2 * p) * C + 8 * (t % (C / 8));
+            edge[k] = (row == 0 ? 1 : 0) | (row == 17 ? 2 : 0) | (p == 0 ? 4 : 0) | (p == 8 ? 8 : 0) |
+                      (row > 17 ? 16 : 0);
+        }
+    }
+    __device__ __forceinline__ void load(const float* __restrict__ dz, const uint16_t* __restrict__ xin, int item,
+                                         int nt, int n) {
+        const int b = item / (nt * nt), r = item - b * (nt * nt);
+        const int ti = r / nt, tj = r % nt;
+        const long long at = (((long long)b * n + ti * kFT) * n + tj * kFT) * C;
+        const float* const da = dz + at;
+        const uint16_t* const xb = xin + (at - (long long)(n + 1) * C);
+        const int rows = 16 | (ti == 0 ? 1 : 0) | (ti == nt - 1 ? 2 : 0);
+        const int m0 = rows | (tj == 0 ? 4 : 0), m1 = rows | (tj == nt - 1 ? 8 : 0);
+#pragma unroll
+        for (int k = 0; k < kA; k++) {
+            a[k][0] = *(const float4*)(da + off_a[k]);
+            a[k][1] = *(const float4*)(da + off_a[k] + C);
+        }
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            x[k][0] = x[k][1] = make_uint4(0, 0, 0, 0);
+            if (!(edge[k] & m0)) x[k][0] = *(const uint4*)(xb + off_b[k]);
+            if (!(edge[k] & m1)) x[k][1] = *(const uint4*)(xb + off_b[k] + C);
+        }
+    }
+};
+
+template <int C>
+__global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float* __restrict__ dz,
+                                                                     const uint16_t* __restrict__ x,
+                                                                     float* __restrict__ grad, int woff, int boff,
+                                                                     int n, int batch) {
     constexpr int H = C / 16;
     constexpr int kAS = 272;         // A: co stride (elements)
     constexpr int kXP = 24;          // B: row pitch (elements)
@@ -1041,7 +1098,6 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(const float* __restrict__ dz
     __shared__ __align__(16) uint16_t al[C * kAS];
     __shared__ __align__(16) uint16_t xs[C * kXS];
     __shared__ float bsum[C];
-    const int i0 = blockIdx.y * kFT, j0 = blockIdx.x * kFT;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j16 = lane & 15, kb = lane >> 4;
@@ -1053,46 +1109,65 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(const float* __restrict__ dz
         for (int a = 0; a < H; a++)
 #pragma unroll
             for (int c = 0; c < H; c++) acc[k][a][c] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
-    for (int b = blockIdx.z; b < batch; b += gridDim.z) {
+    const int nt = n / kFT, items = nt * nt * batch;
+    const int g4 = threadIdx.x % (C / 4);  // the channel group of the thread's A items
+    float4 bs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    WgradTile<C> T;
+    T.init(n);
+    int item = blockIdx.x;
+    if (item < items) T.load(dz, x, item, nt, n);
+    for (; item < items; item += gridDim.x) {
         __syncthreads();
-        // A: item (co, 8 pixels of a row)
-        for (int t = threadIdx.x; t < C * 32; t += 64 * kFWaves) {
-            const int co = t % C, pg = t / C;
-            const int row = pg >> 1, c0 = 8 * (pg & 1);
-            const float* src = dz + (((size_t)b * n + i0 + row) * n + j0 + c0) * C + co;
-            float v[8];
+        // A: word (co, row, column pair); the threads of a wave's four groups store their four channels in
+        // turned order, which puts them on distinct banks (4 co are 544 words, a multiple of the banks)
+        uint32_t* const wh = (uint32_t*)ah;
+        uint32_t* const wl = (uint32_t*)al;
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = src[(size_t)e * C];
-            uint32_t hi[4], lo[4];
+        for (int k = 0; k < T.kA; k++) {
+            const int t = threadIdx.x + 256 * k;
+            const int p = (t / (C / 4)) & 7, row = t / (2 * C);
+            const float4 u = T.a[k][0], v = T.a[k][1];
+            bs.x += u.x + v.x;
+            bs.y += u.y + v.y;
+            bs.z += u.z + v.z;
+            bs.w += u.w + v.w;
+            uint32_t hi[4], lo[4], h1[4], l1[4];
+            split_bf16(u.x, v.x, hi[0], lo[0]);
+            split_bf16(u.y, v.y, hi[1], lo[1]);
+            split_bf16(u.z, v.z, hi[2], lo[2]);
+            split_bf16(u.w, v.w, hi[3], lo[3]);
 #pragma unroll
-            for (int e = 0; e < 4; e++) split_bf16(v[2 * e], v[2 * e + 1], hi[e], lo[e]);
-            *(u32x4*)(ah + co * kAS + row * 16 + c0) = (u32x4){hi[0], hi[1], hi[2], hi[3]};
-            *(u32x4*)(al + co * kAS + row * 16 + c0) = (u32x4){lo[0], lo[1], lo[2], lo[3]};
-            atomicAdd(&bsum[co], ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
-        }
-        // B: item (ci, halo row, 8 columns); columns 18..23 are zeros
-        for (int t = threadIdx.x; t < C * 18 * 3; t += 64 * kFWaves) {
-            const int ci = t % C, rg = t / C;
-            const int row = rg / 3, g = rg % 3;
-            const int ii = i0 - 1 + row;
-            uint32_t v[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                uint32_t pr = 0;
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    const int col = 8 * g + 2 * e + u, jj = j0 - 1 + col;
-                    uint32_t h = 0;
-                    if (col < 18 && ii >= 0 && ii < n && jj >= 0 && jj < n)
-                        h = x[(((size_t)b * n + ii) * n + jj) * C + ci];
-                    pr |= h << (16 * u);
-                }
-                v[e] = pr;
+            for (int c = 0; c < 4; c++) {
+                h1[c] = g4 & 1 ? hi[(c + 1) & 3] : hi[c];
+                l1[c] = g4 & 1 ? lo[(c + 1) & 3] : lo[c];
             }
-            *(u32x4*)(xs + ci * kXS + row * kXP + 8 * g) = (u32x4){v[0], v[1], v[2], v[3]};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int w = (4 * g4 + ((c + g4) & 3)) * (kAS / 2) + row * 8 + p;
+                wh[w] = g4 & 2 ? h1[(c + 2) & 3] : h1[c];
+                wl[w] = g4 & 2 ? l1[(c + 2) & 3] : l1[c];
+            }
+        }
+        // B: word (ci, halo row, column pair); columns 18 .. 23 of a row are not read
+#pragma unroll
+        for (int k = 0; k < T.kB; k++) {
+            const int t = threadIdx.x + 256 * k;
+            const int g = t % (C / 8), q = t / (C / 8);
+            const int row = q / 9, p = q - 9 * row;
+            if (row < 18) {
+                uint32_t* const w = (uint32_t*)xs + 8 * g * (kXS / 2) + row * (kXP / 2) + p;
+                const uint32_t a[4] = {T.x[k][0].x, T.x[k][0].y, T.x[k][0].z, T.x[k][0].w};
+                const uint32_t b[4] = {T.x[k][1].x, T.x[k][1].y, T.x[k][1].z, T.x[k][1].w};
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    w[2 * c * (kXS / 2)] = __builtin_amdgcn_perm(b[c], a[c], 0x05040100u);
+                    w[(2 * c + 1) * (kXS / 2)] = __builtin_amdgcn_perm(b[c], a[c], 0x07060302u);
+                }
+            }
         }
         __syncthreads();
-#pragma unroll 2
+        if (item + (int)gridDim.x < items) T.load(dz, x, item + gridDim.x, nt, n);
+#pragma unroll 1
         for (int kblk = 0; kblk < 8; kblk++) {
             const int prow = 2 * kblk + (kb >> 1), pc = 8 * (kb & 1);
             bf16x8 a_h[H], a_l[H];
@@ -1143,6 +1218,10 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(const float* __restrict__ dz
                 for (int r = 0; r < 4; r++)
                     atomicAdd(grad + woff + ((16 * a + 4 * kb + r) * 9 + tap) * C + 16 * c + j16, acc[k][a][c][r]);
     }
+    atomicAdd(&bsum[4 * g4 + 0], bs.x);
+    atomicAdd(&bsum[4 * g4 + 1], bs.y);
+    atomicAdd(&bsum[4 * g4 + 2], bs.z);
+    atomicAdd(&bsum[4 * g4 + 3], bs.w);
     __syncthreads();
     if ((int)threadIdx.x < C) atomicAdd(grad + boff + threadIdx.x, bsum[threadIdx.x]);
 }
@@ -1454,17 +1533,15 @@ hipError_t backward_t(const LearnedBufs& B, const float* prm, const float* dout,
                       hipStream_t s) {
     constexpr LearnedLayout L = learned_layout(C);
     const dim3 g16(n / kFT, n / kFT, batch);
-    // weight gradients sum over a share of the slices: about 2048 workgroups
     const int tiles16 = (n / kFT) * (n / kFT);
-    const dim3 gm(n / kFT, n / kFT, (unsigned)std::max(1, std::min(batch, 2048 / tiles16)));
-    // workgroups the card holds: four (out), four or two (in, by its LDS) per CU of 256
+    // workgroups the card holds: four (out), four or two (the others, by their LDS) per CU of 256
     const unsigned items = (unsigned)tiles16 * (unsigned)batch;
     const unsigned out_wgs = std::min(items, 1024u), in_wgs = std::min(items, C == 16 ? 1024u : 512u);
     hipLaunchKernelGGL(k_conv_out_bwd<C>, dim3(out_wgs), dim3(256), 0, s, dout, B.a3, prm, B.dz3, grad, n, batch);
     hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, B.wt3, B.dz2, n);
     hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, B.wt2, B.dz1, n);
-    hipLaunchKernelGGL(k_wgrad_mfma<C>, gm, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, grad, L.W3, L.B3, n, batch);
-    hipLaunchKernelGGL(k_wgrad_mfma<C>, gm, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, grad, L.W2, L.B2, n, batch);
+    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz3, B.a2, grad, L.W3, L.B3, n, batch);
+    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz2, B.a1, grad, L.W2, L.B2, n, batch);
     hipLaunchKernelGGL(k_conv_in_bwd<C>, dim3(in_wgs), dim3(256), 0, s, B.dz1, dout, B.r0, prm, B.dr0, grad, n, batch);
     return hipGetLastError();
 }

@@ -39,3 +39,22 @@ def test_gradients_at_split_edges(n, nang, ndet, batch, channels):
     assert _rel(dq, ref_dq) <= 1e-4
     dfull = sum(L.filter_grad(ref_dq[b], sino[b]) for b in range(batch))
     assert _rel(grad[taps_off:], L.fold_taps(dfull)) <= 1e-4
+
+
+@pytest.mark.parametrize("n,channels", [(544, 16), (384, 32)])
+def test_weight_gradients_past_one_tile_a_workgroup(n, channels):
+    """34^2 and 24^2 tiles: a few more than the workgroups that go through
+    them, so some take a second tile and most none."""
+    with FBP(n, 3, n, max_batch=1) as f, lm.LearnedFBP(f, channels=channels) as m:
+        prm = _random_params(m, n, n, seed=11)
+        m.set_params(prm)
+        m.make_batch(1, seed=3, i0=1e4, mu=1.0)
+        target = f.download(IMAGE, 1)
+        _, grad = m.gradient(1)
+        out, r0 = f.download(RECON, 1), m.download(lm.R0, 1)
+        acts = [_bf(m.download(w, 1)) for w in (lm.A1, lm.A2, lm.A3)]
+    dout = 2.0 * (out.astype(np.float64) - target) / target.size
+    cache = {"x0": L.bf16(r0)[..., None], "a1": acts[0], "a2": acts[1], "a3": acts[2]}
+    ref, _ = L.cnn_backward(prm.astype(np.float64), cache, dout, C=channels)
+    for name, (o, s) in L.layout(channels)[0].items():
+        assert _rel(grad[o:o + s], np.asarray(ref[name]).reshape(-1)) <= 2e-4, name
