@@ -660,10 +660,10 @@ __global__ __launch_bounds__(64 * FwdSplit<C>::kWaves, C == 16 ? 5 : 2) void k_c
 // lane i + 16k, B[k][j] at lane j + 16k, D[i][j] at lane j + 16(i/4), register
 // i%4).  As many workgroups as the card holds at once (a second, part-filled
 // round doubled the time) walk the 16 x 16 tiles of all slices, the next tile's
-// loads in flight, and add their weight sums into grad[] once.  Both are bound
-// by memory: 402 MB (out) and 285 MB (in) at 16 x 512^2, C = 16.  Each was two
-// kernels, the weight sums on the VALU with two LDS reads a product: out 106 +
-// 310 -> 131 us, in 271 + 310 -> 140 us.
+// loads in flight, and store their weight sums once, a row of part[] each
+// (k_sum_parts).  Both are bound by memory: 402 MB (out) and 285 MB (in) at
+// 16 x 512^2, C = 16.  Each was two kernels, the weight sums on the VALU with
+// two LDS reads a product: out 106 + 310 -> 100 us, in 271 + 310 -> 113 us.
 
 // out[p] = r0[p] + b4 + sum_t W4[t] . a3[p + off(t)]:
 //   dz3[q][ci]  = (a3[q][ci] > 0) sum_t W4[t][ci] dout[q - off(t)]   A = W4^T (K = 9 of 12), B = shifted dout
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(64 * FwdSplit<C>::kWaves, C == 16 ? 5 : 2) void k_c
 template <int C>
 __global__ __launch_bounds__(256) void k_conv_out_bwd(const float* __restrict__ dout, const uint16_t* __restrict__ a3,
                                                       const float* __restrict__ prm, float* __restrict__ dz3,
-                                                      float* __restrict__ grad, int n, int batch) {
+                                                      float* __restrict__ part, int n, int batch) {
     constexpr LearnedLayout L = learned_layout(C);
     constexpr int H = C / 16, kW = T + 2;
     __shared__ float ds[kW * kW];
@@ -764,7 +764,8 @@ __global__ __launch_bounds__(256) void k_conv_out_bwd(const float* __restrict__ 
             }
         }
     }
-    // lane (j16, kb) holds dW4[4kb + r][16h + j16]: the four waves' sums, then grad[]
+    // lane (j16, kb) holds dW4[4kb + r][16h + j16]: the four waves' sums, then the workgroup's row of part[]
+    part += (size_t)blockIdx.x * L.Taps;
 #pragma unroll
     for (int h = 0; h < H; h++)
 #pragma unroll
@@ -776,11 +777,14 @@ __global__ __launch_bounds__(256) void k_conv_out_bwd(const float* __restrict__ 
         float v = 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; q++) v += red[(q * H + h) * 256 + threadIdx.x];
-        if (t < 9) atomicAdd(grad + L.W4 + t * C + 16 * h + c, v);
+        if (t < 9) part[L.W4 + t * C + 16 * h + c] = v;
     }
+    __shared__ float wsum[4];
 #pragma unroll
     for (int o = 32; o; o >>= 1) bsum += __shfl_xor(bsum, o);
-    if (lane == 0) atomicAdd(grad + L.B4, bsum);
+    if (lane == 0) wsum[wave] = bsum;
+    __syncthreads();
+    if (threadIdx.x == 0) part[L.B4] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
 }
 
 // a1 = relu(b1 + sum_t W1[.][t] r0[p + off(t)]), out = r0 + ...:
@@ -790,7 +794,7 @@ __global__ __launch_bounds__(256) void k_conv_out_bwd(const float* __restrict__ 
 template <int C>
 __global__ __launch_bounds__(256) void k_conv_in_bwd(const float* __restrict__ dz1, const float* __restrict__ dout,
                                                      const float* __restrict__ r0, const float* __restrict__ prm,
-                                                     float* __restrict__ dr0, float* __restrict__ grad, int n,
+                                                     float* __restrict__ dr0, float* __restrict__ part, int n,
                                                      int batch) {
     constexpr LearnedLayout L = learned_layout(C);
     constexpr int H = C / 16, kW = T + 2, kN = kW * kW;
@@ -880,6 +884,7 @@ __global__ __launch_bounds__(256) void k_conv_in_bwd(const float* __restrict__ d
         }
     }
     // lane (j16, kb) holds dW1[16h + 4kb + r][j16] (j16 < 9) and db1 (j16 == 9)
+    part += (size_t)blockIdx.x * L.Taps;
     __syncthreads();
     float* red = zs;  // 4 waves x H x 256 floats
     static_assert(4 * H * 256 <= kN * kPz, "the reduction fits the tile buffer");
@@ -895,9 +900,9 @@ __global__ __launch_bounds__(256) void k_conv_in_bwd(const float* __restrict__ d
 #pragma unroll
         for (int q = 0; q < 4; q++) v += red[(q * H + h) * 256 + threadIdx.x];
         if (t < 9)
-            atomicAdd(grad + L.W1 + co * 9 + t, v);
+            part[L.W1 + co * 9 + t] = v;
         else if (t == 9)
-            atomicAdd(grad + L.B1 + co, v);
+            part[L.B1 + co] = v;
     }
 }
 
@@ -1020,8 +1025,8 @@ __global__ __launch_bounds__(256) void k_conv_mid_bwd_mfma(const float* __restri
 // Weight gradient of a conv C -> C layer:
 //   dW[co][t][ci] += sum_p dz[p][co] x[p + off(t)][ci],  db[co] += sum_p dz[p][co].
 // A workgroup goes through 16 x 16 tiles blockIdx.x, blockIdx.x + gridDim.x,
-// ... of all slices, sums in registers, and adds into grad[] with atomics
-// once.  K = pixels: A[co][p] = dz, split into bf16 hi and lo parts
+// ... of all slices, sums in registers, and stores its row of part[] once.
+// K = pixels: A[co][p] = dz, split into bf16 hi and lo parts
 // (split_bf16) and transposed in LDS ([co][16 rows][16 columns], co stride
 // 272 elements); B[p][ci] = x (bf16, exact), transposed with a one-pixel
 // halo ([ci][18 rows][pitch 24]).  A K block is two tile rows: lane block kb
@@ -1088,7 +1093,7 @@ struct WgradTile {
 template <int C>
 __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float* __restrict__ dz,
                                                                      const uint16_t* __restrict__ x,
-                                                                     float* __restrict__ grad, int woff, int boff,
+                                                                     float* __restrict__ part, int woff, int boff,
                                                                      int n, int batch) {
     constexpr int H = C / 16;
     constexpr int kAS = 272;         // A: co stride (elements)
@@ -1206,6 +1211,7 @@ __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float
         }
     }
     // lane (j16, kb) holds D[co = 16a + 4kb + r][ci = 16c + j16]
+    part += (size_t)blockIdx.x * learned_layout(C).Taps;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         const int tap = wave + 4 * k;
@@ -1216,14 +1222,42 @@ __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float
             for (int c = 0; c < H; c++)
 #pragma unroll
                 for (int r = 0; r < 4; r++)
-                    atomicAdd(grad + woff + ((16 * a + 4 * kb + r) * 9 + tap) * C + 16 * c + j16, acc[k][a][c][r]);
+                    part[woff + ((16 * a + 4 * kb + r) * 9 + tap) * C + 16 * c + j16] = acc[k][a][c][r];
     }
     atomicAdd(&bsum[4 * g4 + 0], bs.x);
     atomicAdd(&bsum[4 * g4 + 1], bs.y);
     atomicAdd(&bsum[4 * g4 + 2], bs.z);
     atomicAdd(&bsum[4 * g4 + 3], bs.w);
     __syncthreads();
-    if ((int)threadIdx.x < C) atomicAdd(grad + boff + threadIdx.x, bsum[threadIdx.x]);
+    if ((int)threadIdx.x < C) part[boff + threadIdx.x] = bsum[threadIdx.x];
+}
+
+// grad[i] += the sum of column i of part[rows][m]; rows: those of the kernel
+// that wrote the column (out_rows in [out0, m), the output layer's, else
+// in_rows).  A workgroup takes 32 columns, each 32 strided shares of rows.
+// Instead of atomics on grad[], which up to 1,024 workgroups hit at the same
+// few lines at their end: the output layer's kernel 133 -> 100 us, the input
+// layer's 149 -> 113 (16 x 512^2, 16 channels), for 8 us here, and the sums are
+// the same on every run.
+__global__ __launch_bounds__(1024) void k_sum_parts(const float* __restrict__ part, float* __restrict__ grad, int m,
+                                                    int out0, int out_rows, int in_rows) {
+    __shared__ float red[32][33];
+    const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + c;
+    float v = 0.0f;
+    if (i < m) {
+        const int rows = i >= out0 ? out_rows : in_rows;
+#pragma unroll 8
+        for (int r = g; r < rows; r += 32) v += part[(size_t)r * m + i];
+    }
+    red[g][c] = v;
+    __syncthreads();
+    if (g == 0 && i < m) {
+        float t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 32; k++) t += red[k][c];
+        grad[i] += t;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1536,13 +1570,15 @@ hipError_t backward_t(const LearnedBufs& B, const float* prm, const float* dout,
     const int tiles16 = (n / kFT) * (n / kFT);
     // workgroups the card holds: four (out), four or two (the others, by their LDS) per CU of 256
     const unsigned items = (unsigned)tiles16 * (unsigned)batch;
-    const unsigned out_wgs = std::min(items, 1024u), in_wgs = std::min(items, C == 16 ? 1024u : 512u);
-    hipLaunchKernelGGL(k_conv_out_bwd<C>, dim3(out_wgs), dim3(256), 0, s, dout, B.a3, prm, B.dz3, grad, n, batch);
+    const unsigned out_wgs = std::min(items, (unsigned)kPartRows), in_wgs = std::min(items, C == 16 ? (unsigned)kPartRows : 512u);
+    hipLaunchKernelGGL(k_conv_out_bwd<C>, dim3(out_wgs), dim3(256), 0, s, dout, B.a3, prm, B.dz3, B.part, n, batch);
     hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz3, B.a2, B.wt3, B.dz2, n);
     hipLaunchKernelGGL(k_conv_mid_bwd_mfma<C>, g16, dim3(64 * kFWaves), 0, s, B.dz2, B.a1, B.wt2, B.dz1, n);
-    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz3, B.a2, grad, L.W3, L.B3, n, batch);
-    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz2, B.a1, grad, L.W2, L.B2, n, batch);
-    hipLaunchKernelGGL(k_conv_in_bwd<C>, dim3(in_wgs), dim3(256), 0, s, B.dz1, dout, B.r0, prm, B.dr0, grad, n, batch);
+    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz3, B.a2, B.part, L.W3, L.B3, n, batch);
+    hipLaunchKernelGGL(k_wgrad_mfma<C>, dim3(in_wgs), dim3(64 * kFWaves), 0, s, B.dz2, B.a1, B.part, L.W2, L.B2, n, batch);
+    hipLaunchKernelGGL(k_conv_in_bwd<C>, dim3(in_wgs), dim3(256), 0, s, B.dz1, dout, B.r0, prm, B.dr0, B.part, n, batch);
+    hipLaunchKernelGGL(k_sum_parts, dim3((L.Taps + 31) / 32), dim3(1024), 0, s, B.part, grad, L.Taps, L.W4,
+                       (int)out_wgs, (int)in_wgs);
     return hipGetLastError();
 }
 

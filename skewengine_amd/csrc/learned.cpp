@@ -27,6 +27,7 @@ struct ske_learned {
     bool derived = false;          // full taps and bf16 weights match prm (cleared whenever prm changes)
     DevBuf<float> prm, grad, m1, m2, full, dq, dfull, dout;
     DevBuf<double> loss;
+    DevBuf<float> part;  // the backward's weight sums by workgroup
     DevBuf<float> r0, dz, dr0, drL, dqp;  // dz: three layers back to back; drL, dqp: the adjoint's lines and partial sums
     DevBuf<uint16_t> act, wb;      // act: a1, a2, a3 back to back; wb: bf16 weights (learned_wb_size)
     DevBuf<float> ell;
@@ -45,6 +46,7 @@ struct ske_learned {
             B.dz2 = dz.p + a;
             B.dz3 = dz.p + 2 * a;
             B.dr0 = dr0.p;
+            B.part = part.p;
         }
         B.wb2 = wb.p;
         B.wb3 = wb.p + 9 * C * C;
@@ -130,6 +132,7 @@ int ensure_train(ske_learned* l) {
     const FbpGeom& g = l->f->g;
     SKE_TRY(l->dz.ensure(3 * l->pix(mb) * l->C));
     SKE_TRY(l->dr0.ensure(l->pix(mb)));
+    SKE_TRY(l->part.ensure(learned_part_floats(l->C, g.n, mb)));
     SKE_TRY(l->drL.ensure(adjoint_lines_floats(g.n, mb)));
     if (adjoint_chunks(g.n) > 1) SKE_TRY(l->dqp.ensure((size_t)adjoint_chunks(g.n) * mb * g.nang * g.ndet));
     SKE_TRY(l->dout.ensure(l->pix(mb)));

@@ -46,8 +46,17 @@ struct LearnedBufs {
     const uint16_t* wt2; // bf16 W2, W3 transposed ([ci][t][co]): the backward's operands
     const uint16_t* wt3;
     const uint16_t* w1b; // bf16 W1 as [co][16] (9 taps, 7 zeros)
+    float* part;         // a row of CNN gradients per workgroup of the backward (learned_part_floats)
     int C;               // hidden channels (16 or 32)
 };
+
+// The backward's weight sums: a row of the CNN's parameters for each of at
+// most kPartRows workgroups, one 16 x 16 tile each at least.
+constexpr int kPartRows = 1024;
+inline size_t learned_part_floats(int C, int n, int batch) {
+    const size_t tiles = (size_t)(n / 16) * (n / 16) * batch;
+    return (tiles < kPartRows ? tiles : kPartRows) * learned_layout(C).Taps;
+}
 
 // wb: bf16 W2, W3 ([co][t][ci]), W1 as [co][16], then W2, W3 transposed
 // ([ci][t][co]); learned_wb_size(C) elements.
