@@ -120,10 +120,7 @@ int forward(ske_learned* l, int batch, bool train) {
     }));
     return f->timer.launch(s, "cnn_forward", [&] {
         if (!train) return launch_cnn_infer(B, l->prm.p, g.n, batch, s);
-        hipError_t e = launch_fill_f64(l->loss.p, 1, s);
-        if (e != hipSuccess) return e;
-        return launch_cnn_forward(B, l->prm.p, g.n, batch, train ? f->buf[SKE_FBP_IMAGE].p : nullptr,
-                                  train ? l->dout.p : nullptr, train ? l->loss.p : nullptr, s);
+        return launch_cnn_forward(B, l->prm.p, g.n, batch, f->buf[SKE_FBP_IMAGE].p, l->dout.p, l->loss.p, s);
     });
 }
 
@@ -139,7 +136,7 @@ int ensure_train(ske_learned* l) {
     SKE_TRY(l->dq.ensure((size_t)mb * g.nang * g.ndet));
     SKE_TRY(l->dfull.ensure(2 * (size_t)g.ndet - 1));
     SKE_TRY(l->grad.ensure(l->nparam));
-    SKE_TRY(l->loss.ensure(1));
+    SKE_TRY(l->loss.ensure(1 + (size_t)(g.n / 16) * (g.n / 16) * mb));  // the sum and each tile's share
     return SKE_OK;
 }
 

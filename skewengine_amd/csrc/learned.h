@@ -62,7 +62,8 @@ inline size_t learned_part_floats(int C, int n, int batch) {
 // ([ci][t][co]); learned_wb_size(C) elements.
 constexpr size_t learned_wb_size(int C) { return 4 * 9 * (size_t)C * C + 16 * (size_t)C; }
 hipError_t launch_pack_weights(const float* prm, int C, uint16_t* wb, hipStream_t s);
-// Training forward: a1..a3 stored (n a multiple of 16).
+// Training forward: a1..a3 stored (n a multiple of 16).  loss: the sum, then
+// room for one value per 16 x 16 tile of the batch.
 hipError_t launch_cnn_forward(const LearnedBufs& B, const float* prm, int n, int batch, const float* target,
                               float* dout, double* loss, hipStream_t s);
 // Inference forward, fused in LDS (no activations stored; n a multiple of 16).
