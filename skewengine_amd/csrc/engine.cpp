@@ -546,17 +546,21 @@ struct Core {
         return SKE_OK;
     }
 
+    // Whether the viewshed must look at its rows' heights: the bit of a step is
+    // the sign of a difference, which is right for heights of at most 1e30.
+    bool check_heights(float povh) const { return odd || !(std::fabs(povh) <= 1e30f); }
+
     // The viewshed over a planned row list.  Without a caller's or the
     // autotuner's choice (`own`) the waves of a grid workgroup follow the run's
     // rows; with one chunk per wave, rows of fewer than four chunks run 2
     // instead of 4, so that no wave of it idles.
     hipError_t launch_sdem(const DevPlan& v, const std::vector<SdemRun>& runs, SdemTuning t, bool own, float* dst,
                            float povh, unsigned long long* steps) {
-        if (t.group == 1 || (t.persistent_wgs_per_cu > 0 && !odd)) {
+        t.check = check_heights(povh);
+        if (t.group == 1 || (t.persistent_wgs_per_cu > 0 && !t.check)) {
             if (own && t.persistent_wgs_per_cu == 0) t.waves = (v.maxL + 63) / 64 < 4 ? 2 : 4;
             return launch_op_sdem_tuned(v, in4.p, nullptr, dst, rtab.p, povh, t, counter.p, steps, stream);
         }
-        t.check = odd || !(std::fabs(povh) <= 1e30f);
         for (const SdemRun& r : runs) {
             DevPlan p = v;
             p.work += r.first;
@@ -593,7 +597,7 @@ struct Core {
                     }));
                 } else {
                     SKE_TRY(launch("op_sdem", [&] {
-                        return launch_op_sdem(v, in4.p, nullptr, arena.p, rtab.p, povh, sdem_variant, stream);
+                        return launch_op_sdem(v, in4.p, nullptr, arena.p, rtab.p, povh, sdem_variant, false, stream);
                     }));
                 }
                 break;
@@ -844,6 +848,7 @@ struct ske_engine {
     ImagePlan one;        // the current sector as a plan, its tables on the device
     SectorTables tables;
     bool exposed = false;  // ske_device_pointers handed out: skew() returns after the device is done
+    bool foreign = false;  // a caller holds skewInput's address and may have written any height there
     DevBuf<float> S, SO;  // 2N + dim_l each, like skewAlloc (src/skewEngine.cuh:425-426)
     DevBuf<double> P1;
     DevBuf<float> q1;
@@ -907,6 +912,7 @@ int sector_kernel(ske_engine* e) {
     const DevPlan v = e->tables.view(e->one);
     const SectorPlan& sp = e->cur;
     if (e->custom) {
+        e->foreign = true;
         e->custom(e->SO.p, e->S.p, sp.dim_i, sp.H, e->tables.last(), e->tables.first(), e->povh, sp.newAngle, (void*)c.stream,
                   e->custom_user);
         SKE_HIP(hipGetLastError());
@@ -915,7 +921,8 @@ int sector_kernel(ske_engine* e) {
     switch (e->kernel_id) {
     case SKE_KERNEL_SDEM:
         SKE_TRY(c.launch("op_sdem", [&] {
-            return launch_op_sdem(v, c.in4.p, e->S.p, e->SO.p, c.rtab.p, e->povh, c.sdem_variant, c.stream);
+            return launch_op_sdem(v, c.in4.p, e->S.p, e->SO.p, c.rtab.p, e->povh, c.sdem_variant,
+                                  e->foreign || c.check_heights(e->povh), c.stream);
         }));
         break;
     case SKE_KERNEL_CEPSTRUM:
@@ -1114,7 +1121,7 @@ int ske_device_pointers(ske_engine* e, float** d_skewInput, float** d_skewOutput
     if (!e->have_sector) return fail(SKE_ESTATE, "no sector skewed yet");
     SKE_HIP(hipSetDevice(e->core.device));
     SKE_HIP(hipStreamSynchronize(e->core.stream));
-    e->exposed = true;
+    e->exposed = e->foreign = true;
     if (d_skewInput) *d_skewInput = e->S.p;
     if (d_skewOutput) *d_skewOutput = e->SO.p;
     if (d_first) *d_first = e->tables.first();

@@ -880,27 +880,27 @@ hipError_t launch_op_sdem_tuned(const DevPlan& p, const float* in4, const float*
 #define SKE_GRID(W, G, C)                                                                                         \
     hipLaunchKernelGGL((k_op_sdem_bits<W, G, C>), dim3(p.nwork), dim3(64 * W), lds, s, p.secs, p.work, in4, p.target, \
                        p.weight, p.fl, Sbuf, rtab, povh, arena, pools, steps)
-    if (G == 4 && t.check) {
-        if (t.waves == 2) SKE_GRID(2, 4, true); else if (t.waves == 8) SKE_GRID(8, 4, true); else SKE_GRID(4, 4, true);
-    } else if (G == 4) {
-        if (t.waves == 2) SKE_GRID(2, 4, false); else if (t.waves == 8) SKE_GRID(8, 4, false); else SKE_GRID(4, 4, false);
+#define SKE_GRID_W(G, C)                                                                                          \
+    if (t.waves == 2) SKE_GRID(2, G, C); else if (t.waves == 8) SKE_GRID(8, G, C); else SKE_GRID(4, G, C)
+    if (G == 4) {
+        if (t.check) { SKE_GRID_W(4, true); } else { SKE_GRID_W(4, false); }
     } else {
-        if (t.waves == 2) SKE_GRID(2, 1, false); else if (t.waves == 8) SKE_GRID(8, 1, false); else SKE_GRID(4, 1, false);
+        if (t.check) { SKE_GRID_W(1, true); } else { SKE_GRID_W(1, false); }
     }
+#undef SKE_GRID_W
 #undef SKE_GRID
     return hipGetLastError();
 }
 
 hipError_t launch_op_sdem(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
-                          const float4* rtab, float povh, int variant, hipStream_t s) {
-    if (p.nwork == 0) return hipSuccess;
+                          const float4* rtab, float povh, int variant, bool check, hipStream_t s) {
     if (variant == 0) {
-        if (p.maxL > 32 * kChunksMax) return launch_op_sdem_long(p, in4, Sbuf, arena, rtab, povh, nullptr, s);
-        const size_t lds = sdem_bits_lds(p.maxL, 1, 4);
-        hipLaunchKernelGGL((k_op_sdem_bits<4, 1, false>), dim3(p.nwork), dim3(256), lds, s, p.secs, p.work, in4, p.target,
-                           p.weight, p.fl, Sbuf, rtab, povh, arena, 0, nullptr);
-        return hipGetLastError();
+        SdemTuning t;
+        t.group = 1;
+        t.check = check;
+        return launch_op_sdem_tuned(p, in4, Sbuf, arena, rtab, povh, t, nullptr, nullptr, s);
     }
+    if (p.nwork == 0) return hipSuccess;
     const size_t lds = sizeof(float) * (size_t)(p.maxL + 2 * kPad);
     if (variant == 1)
         hipLaunchKernelGGL(k_op_sdem<1>, dim3(p.nwork), dim3(256), lds, s, p.secs, p.work, in4, p.target,

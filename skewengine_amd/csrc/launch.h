@@ -29,7 +29,7 @@ struct SdemTuning {
     int persistent_wgs_per_cu = 0; // 0: one workgroup per row; >0: persistent grid of this many per CU
     int occupancy = 0;             // persistent grid: 8 = compile for 8 waves per SIMD (fewer VGPRs)
     int group = 4;                 // 1: one 64-observer chunk per wave; 4: pools of up to 4 chunks
-    bool check = false;            // rows may hold heights that are not finite or above 1e30 (pools, grid launch)
+    bool check = false;            // rows or povh may hold heights that are not finite or above 1e30 (grid launch)
 };
 
 // Graph-safe clears (kernels, not hipMemsetAsync).
@@ -52,8 +52,9 @@ hipError_t launch_copy16(void* dst, const void* src, int n, hipStream_t s);
 // (fused path); otherwise rows come from a materialised skewInput.
 hipError_t launch_op_unit(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
                           hipStream_t s);
+// variant 0: one chunk per wave, `check` as in SdemTuning.
 hipError_t launch_op_sdem(const DevPlan& p, const float* in4, const float* Sbuf, float* arena,
-                          const float4* rtab, float povh, int variant, hipStream_t s);
+                          const float4* rtab, float povh, int variant, bool check, hipStream_t s);
 // Bit-block viewshed with an explicit launch shape; `counter` (one int of
 // device memory) feeds the persistent grid.
 // `steps`, when not null, receives += the lane-steps the scans executed
