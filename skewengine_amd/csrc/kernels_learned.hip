@@ -1270,7 +1270,12 @@ __global__ __launch_bounds__(1024) void k_sum_parts(const float* __restrict__ pa
 // it walks the rows (the columns when |c| < |sn|); along a line kf is linear
 // with a slope of magnitude as >= 0.7, so the pixels within one bin of k are
 // at most three, from t = ceil(tc - 1/as), tc the position where kf = k, with
-// weights 1 - |t - tc| as.  Their positions and weights serve the four slices,
+// weights 1 - |t - tc| as.  tc moves by the same step from line to line: both
+// are found in FP64 and kept in 32.32 fixed point, so that its error (2^-33 a
+// line, 2^-25 from the fraction in FP32) does not grow with tc; tc = tc0 + u dt
+// in FP32 is off by the same amount along a whole ray (512^2 noise: dq off by
+// 6e-5 of its largest value, 2e-5 with each pixel's kf in FP32, now 5e-7).
+// Their positions and weights serve the four slices,
 // which k_adjoint_lines interleaves (float4 per pixel, four zero pixels at
 // each end of a line, so t needs one clamp and no test).  The lines are cut in
 // `nchunk` shares, one workgroup each, whose sums k_adjoint_sum adds in order.
@@ -1316,11 +1321,10 @@ __global__ __launch_bounds__(256) void k_bp_adjoint(const float4* __restrict__ r
     const bool walk_rows = fabsf(c) >= fabsf(sn);
     const float4* const im = (walk_rows ? rows : cols) + (size_t)grp * n * pitch + kAdjPad;
     // kf of line u, position t: A + u B + t slope
-    const float m = 0.5f * (float)n - 0.5f;
     const float slope = walk_rows ? c : -sn, B = walk_rows ? -sn : c;
-    const float A = g.det_c + m * (sn - c);
-    const float rsl = 1.0f / slope, as = fabsf(slope), half = fabsf(rsl);
-    const float tc0 = ((float)k - A) * rsl, dt = -B * rsl;
+    const double A = (double)g.det_c + (0.5 * n - 0.5) * ((double)sn - (double)c);
+    const double t0 = ((double)k - A) / (double)slope, dt64 = -(double)B / (double)slope;
+    const float tc0 = (float)t0, dt = (float)dt64;
     const int per = (n + nchunk - 1) / nchunk;
     int u0 = ch * per, u1 = min(u0 + per, n);
     {   // lines whose pixels a lane of this wave can reach: -2 < tc < n + 1 (two lines of margin)
@@ -1338,17 +1342,21 @@ __global__ __launch_bounds__(256) void k_bp_adjoint(const float4* __restrict__ r
         u0 = __builtin_amdgcn_readfirstlane((int)lo);
         u1 = __builtin_amdgcn_readfirstlane((int)hi);
     }
-    const float tmax = (float)n;
+    // q: tc - 1/as + 1, whose integer part is the first pixel (|tc| < 2^15); with its fraction f the pixels'
+    // distances from tc, times as, are as - 1, 2 as - 1 and 3 as - 1 less f as
+    constexpr double kOne = 4294967296.0;
+    const float as = fabsf(slope), unit = as * (float)(1.0 / kOne);
+    const float c1 = 2.0f * as - 1.0f, c2 = (float)(2.0 - 3.0 * (double)as);
+    long long q = (long long)rint((t0 + u0 * dt64 + (1.0 - 1.0 / (double)as)) * kOne);
+    const long long dq = (long long)rint(dt64 * kOne);
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 2
-    for (int u = u0; u < u1; u++) {
-        const float tc = __builtin_fmaf((float)u, dt, tc0);
-        const float tf = ceilf(tc - half);
-        const float d = (tf - tc) * as;
-        const float w0 = fmaxf(1.0f - fabsf(d), 0.0f), w1 = fmaxf(1.0f - fabsf(d + as), 0.0f),
-                    w2 = fmaxf(1.0f - fabsf(__builtin_fmaf(2.0f, as, d)), 0.0f);
+    for (int u = u0; u < u1; u++, q += dq) {
+        const float fr = (float)(uint32_t)q;
+        const float w0 = __builtin_fmaf(fr, -unit, as), w1 = 1.0f - fabsf(__builtin_fmaf(fr, -unit, c1)),
+                    w2 = fmaxf(__builtin_fmaf(fr, unit, c2), 0.0f);
         // clamped, the three pixels are padding
-        const int t = (int)__builtin_amdgcn_fmed3f(tf, -3.0f, tmax);
+        const int t = min(max((int)(q >> 32), -3), n);
         const float4* p = im + (size_t)u * pitch + t;
         const float4 v0 = p[0], v1 = p[1], v2 = p[2];
         acc[0] = __builtin_fmaf(w2, v2.x, __builtin_fmaf(w1, v1.x, __builtin_fmaf(w0, v0.x, acc[0])));
