@@ -149,9 +149,11 @@ __device__ __forceinline__ double rowsum_cols_walk(const int* __restrict__ tt, c
 // Bound by VALU (about 18 operations a column with the tests, 9 without) and by
 // L2 misses: the 64 lanes' taps are one partner row, and a miss in any of a
 // pass's eight rows stalls the wave.  Workgroups go to the eight XCDs
-// in turn, so runs of 23 sectors (an image's 180 over all eight; nearly always
-// one partner copy) are laid on one XCD, whose L2 then serves them: 8 x 955^2
-// passes 1,498 -> 855 us.  A workgroup is one wave: rows of a sector differ in
+// in turn, so runs of up to 23 sectors (an image's 180 over all eight; nearly
+// always one partner copy) are laid on one XCD, whose L2 then serves them: 8 x
+// 955^2 passes 1,498 -> 855 us.  A run is as long as gives every XCD one: with 23
+// always, a share of 23 sectors ran on one XCD (1600^2: 199 us, now 114; 46
+// sectors 208 and 126; without runs 130 and 128).  A workgroup is one wave: rows of a sector differ in
 // length by up to 8 times, and waves that share a workgroup leave their slots
 // to the next one only together.  16 x 512^2: 500 -> 387 us for both; columns
 // without tests and one load a tap: 387 -> 323 (one 512^2 image 53 -> 43).  Not
@@ -164,9 +166,9 @@ __global__ __launch_bounds__(64 * kRowsumWaves) void k_radn_rowsum_cols(const Se
                                                           const int* __restrict__ target,
                                                           const float* __restrict__ weight,
                                                           const uint32_t* __restrict__ fl, double* __restrict__ P,
-                                                          int nsec, int nblk) {
+                                                          int nsec, int nblk, int run) {
     const int at = blockIdx.x >> 3, k = at / nblk;
-    const int si = (k / kXcdSectors * 8 + (blockIdx.x & 7)) * kXcdSectors + k % kXcdSectors;
+    const int si = (k / run * 8 + (int)(blockIdx.x & 7)) * run + k % run;
     if (si >= nsec) return;
     const SecDesc sd = secs[si];
     const int r0 = ((at - k * nblk) * kRowsumWaves + (threadIdx.x >> 6)) * kRowsumRows;
@@ -225,9 +227,9 @@ hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* S
     if (!Sbuf) {  // writes every row r < H of every sector (rows without cells: 0)
         if (p.nsec == 0 || p.maxH <= 0) return hipSuccess;
         const int nblk = (p.maxH + kRowsumRows * kRowsumWaves - 1) / (kRowsumRows * kRowsumWaves);
-        const unsigned units = (unsigned)(p.nsec + 8 * kXcdSectors - 1) / (8 * kXcdSectors);
-        hipLaunchKernelGGL(k_radn_rowsum_cols, dim3(8 * kXcdSectors * units * nblk), dim3(64 * kRowsumWaves), 0, s, p.secs,
-                           in4, p.target, p.weight, p.fl, P, p.nsec, nblk);
+        const int rounds = (p.nsec + 8 * kXcdSectors - 1) / (8 * kXcdSectors), run = (p.nsec + 8 * rounds - 1) / (8 * rounds);
+        hipLaunchKernelGGL(k_radn_rowsum_cols, dim3(8u * run * rounds * nblk), dim3(64 * kRowsumWaves), 0, s, p.secs,
+                           in4, p.target, p.weight, p.fl, P, p.nsec, nblk, run);
         return hipGetLastError();
     }
     if (p.nwork == 0) return hipSuccess;  // writes the rows of the work list only: P zeroed by the caller
