@@ -466,7 +466,6 @@ __device__ __forceinline__ void scan_pool(const float* row, int L, float povh, i
                                           float* __restrict__ so, float R, char* st, int stride, int& nblk) {
     const float2* __restrict__ ytab = reinterpret_cast<const float2*>(rtab + kMaxDim + 1);
     constexpr int kCh = kLong ? kChunksLong : kChunksMax;
-    int* __restrict__ soi = reinterpret_cast<int*>(so);
     const float invL = ytab[L].x;
     const int lane = threadIdx.x & 63;
     const int safe = kDir > 0 ? 0 : L - 1;  // reads row[safe + kDir*d], d <= L + 31: inside the guard bands
@@ -477,6 +476,9 @@ __device__ __forceinline__ void scan_pool(const float* row, int L, float povh, i
     uint16_t* const live = tail + stride;
     uint16_t* const todo = live + stride;
     const int jb = 64 * c0;
+    // the right scan's cv as an integer in the output cell (a float's bits: every access is of the one type)
+    auto put = [&](int j, int cv) { so[j] = __int_as_float(cv); };
+    auto right = [&](int j) { return __float_as_int(so[j]); };
 
     // cv of a scan with steps left, all invisible
     auto over = [&](int id, int j) {
@@ -488,9 +490,9 @@ __device__ __forceinline__ void scan_pool(const float* row, int L, float povh, i
         } else {
             const int cv = sums[id] & 0xFFFFFF;
             if (kDir > 0)
-                soi[j] = cv;
+                put(j, cv);
             else
-                so[j] = (float)(cv + soi[j]) * R;
+                so[j] = (float)(cv + right(j)) * R;
         }
     };
     // Block d0 of kN batches of scans (places id of the pool, positions j; a:
@@ -546,9 +548,9 @@ __device__ __forceinline__ void scan_pool(const float* row, int L, float povh, i
                 } else {
                     const int cv = A[i] - ((db + 1) * (db + 1) - s[i] * s[i]);
                     if (kDir > 0)
-                        soi[j[i]] = cv;
+                        put(j[i], cv);
                     else
-                        so[j[i]] = (float)(cv + soi[j[i]]) * R;
+                        so[j[i]] = (float)(cv + right(j[i])) * R;
                 }
             }
         }
@@ -570,9 +572,9 @@ __device__ __forceinline__ void scan_pool(const float* row, int L, float povh, i
             a[i] = in && myLen > 0;
             if (in && !a[i]) {  // no targets in this direction: cv = 0
                 if (kDir > 0)
-                    soi[j[i]] = 0;
+                    put(j[i], 0);  // long rows: +0
                 else
-                    so[j[i]] = (kLong ? so[j[i]] : (float)soi[j[i]]) * R;
+                    so[j[i]] = (kLong ? so[j[i]] : (float)right(j[i])) * R;
             }
             // A counts the observer's own cell; long rows go on with the right
             // scan's sum, visible from d = 0
