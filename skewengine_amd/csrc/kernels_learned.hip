@@ -1102,11 +1102,10 @@ __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float
     __shared__ __align__(16) uint16_t ah[C * kAS];
     __shared__ __align__(16) uint16_t al[C * kAS];
     __shared__ __align__(16) uint16_t xs[C * kXS];
-    __shared__ float bsum[C];
+    __shared__ __align__(16) float bsum[kFWaves][C];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j16 = lane & 15, kb = lane >> 4;
-    if ((int)threadIdx.x < C) bsum[threadIdx.x] = 0.0f;
     f32x4 acc[3][H][H];
 #pragma unroll
     for (int k = 0; k < 3; k++)
@@ -1224,12 +1223,19 @@ __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float
                 for (int r = 0; r < 4; r++)
                     part[woff + ((16 * a + 4 * kb + r) * 9 + tap) * C + 16 * c + j16] = acc[k][a][c][r];
     }
-    atomicAdd(&bsum[4 * g4 + 0], bs.x);
-    atomicAdd(&bsum[4 * g4 + 1], bs.y);
-    atomicAdd(&bsum[4 * g4 + 2], bs.z);
-    atomicAdd(&bsum[4 * g4 + 3], bs.w);
+    // the bias: the lanes of a channel group, then the waves, in a fixed order
+#pragma unroll
+    for (int o = C / 4; o < 64; o <<= 1) {
+        bs.x += __shfl_xor(bs.x, o);
+        bs.y += __shfl_xor(bs.y, o);
+        bs.z += __shfl_xor(bs.z, o);
+        bs.w += __shfl_xor(bs.w, o);
+    }
+    if (lane < C / 4) *(float4*)&bsum[wave][4 * lane] = bs;
     __syncthreads();
-    if ((int)threadIdx.x < C) part[boff + threadIdx.x] = bsum[threadIdx.x];
+    if ((int)threadIdx.x < C)
+        part[boff + threadIdx.x] =
+            (bsum[0][threadIdx.x] + bsum[1][threadIdx.x]) + (bsum[2][threadIdx.x] + bsum[3][threadIdx.x]);
 }
 
 // grad[i] += the sum of column i of part[rows][m]; rows: those of the kernel
@@ -1237,8 +1243,8 @@ __global__ __launch_bounds__(256, C == 16 ? 4 : 2) void k_wgrad_mfma(const float
 // in_rows).  A workgroup takes 32 columns, each 32 strided shares of rows.
 // Instead of atomics on grad[], which up to 1,024 workgroups hit at the same
 // few lines at their end: the output layer's kernel 133 -> 100 us, the input
-// layer's 149 -> 113 (16 x 512^2, 16 channels), for 8 us here, and the sums are
-// the same on every run.
+// layer's 149 -> 113 (16 x 512^2, 16 channels), for 8 us here, and the CNN's sums
+// are the same on every run (the filter taps are still added by atomics).
 __global__ __launch_bounds__(1024) void k_sum_parts(const float* __restrict__ part, float* __restrict__ grad, int m,
                                                     int out0, int out_rows, int in_rows) {
     __shared__ float red[32][33];
