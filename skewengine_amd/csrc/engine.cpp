@@ -480,6 +480,9 @@ struct Core {
                     have += need;
                     b++;
                 }
+                // The deskew of a sector of folded angle 0 reads a row of the sector before
+                // it: the two stay together, past the budget if a chunk holds no more.
+                if (a < b && b < s1 && sp.newAngle == 0) b += b - 1 > a || !cur->parts.empty() ? -1 : 1;
                 if (b == a) {  // nothing fits next to what the chunk holds: start a new chunk
                     SKE_TRY(flush());
                     continue;

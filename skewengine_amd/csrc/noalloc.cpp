@@ -192,6 +192,8 @@ int execute_noalloc(int kernel_id, int n, const float* d_input, float* d_output,
             have += need;
             b++;
         }
+        // a sector of folded angle 0 and the one before it, whose row its deskew reads, stay together
+        if (a + 1 < b && b < s1 && sp.newAngle == 0) b--;
         if (b == a) return fail(SKE_EINVAL, "ske_execute_noalloc: one sector does not fit the scratch array");
         chunks.emplace_back();
         NaChunk& ch = chunks.back();
