@@ -47,7 +47,7 @@ __device__ __forceinline__ double fast_log(double x, const double* lt) {
 }
 
 // tab layout (double): [0,128): cos/sin(2 pi t/64) interleaved; [128,160): cos(2 pi t/32);
-// from kLogTab the log table of fast_log; from kBlurD the window DFT by rows.
+// from kLogTab the log table of fast_log.
 __global__ __launch_bounds__(64) void k_op_blur(const SecDesc* __restrict__ secs, const RowWork* __restrict__ work,
                                                 const float* __restrict__ in4, const int* __restrict__ target,
                                                 const float* __restrict__ weight, const uint32_t* __restrict__ fl,

@@ -17,8 +17,7 @@ constexpr int kLogTab = 192;    // offset of the log table in the cepstrum const
 constexpr int kLrtC = 720;
 // second DFT: cos, sin of 2 pi (q m mod 64)/64 at [kLrtY + 64 m + 2 i (+1)], q the i-th of 0, 4, .., 24, 2, 6, .., 22, 1, 3, .., 25
 constexpr int kLrtY = kLrtC + 360;
-constexpr int kBlurD = kLrtY + 2048;  // cepstrum window DFT: cos, sin of 2 pi (k m mod 64)/64 at [kBlurD + 64 m + 2 k (+1)]
-constexpr int kCtabSize = kBlurD + 4096;
+constexpr int kCtabSize = kLrtY + 2048;
 constexpr int kNumSectors = 180; // maxSector, src/global.cpp:69
 
 // One sector of one image, as the device sees it.  Mirrors the public fields
