@@ -2,7 +2,7 @@
 // the global transform (LRT=false) and the local one (LRT=true, pointRadon
 // :114-182).
 //
-//   rowsum : one wave per skewed row, P_r = sum_j S(r,j) in double (the
+//   rowsum : P_r = sum_j S(r,j) of every skewed row in double (the
 //            reference sums in double too, kernelRADN.h:227-232).
 //   filter : one workgroup per sector.  P is zero-padded to H2 = 2^ceil(log2 H)
 //            in LDS and filtered with the reference's own transform: the
@@ -21,11 +21,9 @@
 
 namespace ske {
 
+// The rows of a materialised skewInput (the per-sector calls).
 __global__ __launch_bounds__(256) void k_radn_rowsum(const SecDesc* __restrict__ secs,
                                                      const RowWork* __restrict__ work, int nwork,
-                                                     const float* __restrict__ in4,
-                                                     const int* __restrict__ target,
-                                                     const float* __restrict__ weight,
                                                      const uint32_t* __restrict__ fl,
                                                      const float* __restrict__ Sbuf, double* __restrict__ P) {
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -35,35 +33,8 @@ __global__ __launch_bounds__(256) void k_radn_rowsum(const SecDesc* __restrict__
     const SecDesc sd = secs[w.sec];
     const uint32_t v = fl[sd.rows + w.row];
     const int f = fl_first(v), l = fl_last(v);
-    const float* src = in4 + sd.img + (size_t)sd.type * sd.N;
     double acc = 0.0;
-    int j = f + lane;
-    if (!Sbuf) {
-        // four cells per lane and pass: table reads, then gathers, in flight
-        // together; the lane's sum still runs over j in ascending order
-        for (; j + 192 < l; j += 256) {
-            int t[4];
-            float wt[4], x[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                t[u] = target[sd.tab + j + 64 * u];
-                wt[u] = weight[sd.tab + j + 64 * u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                x[u] = skew_cell_sel(src, t[u], wt[u], w.row, j + 64 * u, sd.dim_i, sd.dim_o);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc += (double)x[u];
-        }
-    }
-    for (; j < l; j += 64) {
-        float x;
-        if (Sbuf)
-            x = Sbuf[(size_t)w.row * sd.dim_i + j];
-        else
-            x = skew_cell(src, target[sd.tab + j], weight[sd.tab + j], w.row, j, sd.dim_i, sd.dim_o);
-        acc += (double)x;
-    }
+    for (int j = f + lane; j < l; j += 64) acc += (double)Sbuf[(size_t)w.row * sd.dim_i + j];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
     if (lane == 0) P[sd.q + w.row] = acc;
@@ -233,8 +204,7 @@ hipError_t launch_radn_rowsum(const DevPlan& p, const float* in4, const float* S
         return hipGetLastError();
     }
     if (p.nwork == 0) return hipSuccess;  // writes the rows of the work list only: P zeroed by the caller
-    hipLaunchKernelGGL(k_radn_rowsum, dim3((p.nwork + 3) / 4), dim3(256), 0, s, p.secs, p.work, p.nwork, in4,
-                       p.target, p.weight, p.fl, Sbuf, P);
+    hipLaunchKernelGGL(k_radn_rowsum, dim3((p.nwork + 3) / 4), dim3(256), 0, s, p.secs, p.work, p.nwork, p.fl, Sbuf, P);
     return hipGetLastError();
 }
 

@@ -32,9 +32,8 @@ struct SdemTuning {
     bool check = false;            // rows or povh may hold heights that are not finite or above 1e30 (grid launch)
 };
 
-// Graph-safe clears (kernels, not hipMemsetAsync).
+// Graph-safe clear (a kernel, not hipMemsetAsync).
 hipError_t launch_fill_f32(float* p, size_t n, float v, hipStream_t s);
-hipError_t launch_fill_f64(double* p, size_t n, hipStream_t s);
 
 // prepare(): the three mirrored/transposed copies (src/skewEngine.cuh:962-987).
 // odd (may be null): set to 1 when a value is not finite or above 1e30.
