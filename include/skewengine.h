@@ -108,7 +108,10 @@ int ske_set_kernel(ske_engine *e, int kernel_id, float povh);
 int ske_set_device_operator(ske_engine *e, ske_device_operator op, void *user);
 
 /* skew(angle) (src/skewEngine.cuh:605-682): computeParams, skewShape,
- * resetSkew and the skewed copy of the oriented input. */
+ * resetSkew and the skewed copy of the oriented input.  Returns before the
+ * device is done, like ske_kernel and ske_deskew (all on the engine's stream;
+ * ske_synchronize, or a call that returns data, waits); with an operator of
+ * the caller's set, or after ske_device_pointers, when skewInput is complete. */
 int ske_skew(ske_engine *e, int angle);
 /* kernel() (src/skewEngine.cuh:694-746): run the operator on the skewed rows. */
 int ske_kernel(ske_engine *e);
@@ -255,14 +258,19 @@ typedef struct ske_fbp ske_fbp;
 #define SKE_FBP_RECON 3    /* batch x n x n */
 /* angles: n_angles radians, or NULL for a*pi/n_angles, a = 0..n_angles-1.
  * Device memory: the four buffers above for max_batch slices, plus the
- * projector's zero-bordered image copy, max_batch x (n+8)^2 floats. */
+ * projector's partial ray sums per image tile. */
 int ske_fbp_create(int n, int n_angles, int n_det, const float *angles, int max_batch, int device_id,
                    ske_fbp **out);
 int ske_fbp_destroy(ske_fbp *f);
 int ske_fbp_upload(ske_fbp *f, int buffer, int batch, const float *host);
 int ske_fbp_download(ske_fbp *f, int buffer, int batch, float *host);
 int ske_fbp_buffer(ske_fbp *f, int buffer, float **d_ptr);
-int ske_fbp_project(ske_fbp *f, int batch);     /* IMAGE -> SINO */
+/* IMAGE -> SINO.  Slices are projected four at a time, a single one (and often
+ * the last of 4k + 1) by itself with larger tiles: the same samples summed in
+ * another order, so a slice's sinogram may differ in the last bits between
+ * batches.  The filter and the back-projection give a slice the same bits in
+ * any batch. */
+int ske_fbp_project(ske_fbp *f, int batch);
 int ske_fbp_filter(ske_fbp *f, int batch);      /* SINO -> FILTERED with the current taps */
 int ske_fbp_backproject(ske_fbp *f, int batch); /* FILTERED -> RECON */
 int ske_fbp_reconstruct(ske_fbp *f, int batch); /* filter + backproject */

@@ -59,7 +59,7 @@ __device__ __forceinline__ RayCoord ray_coord(const FbpGeom& g, float s, float c
 // The kernel is bound by VALU issue (23 of a sample's 30 instructions found
 // its position and weights) and then by LDS: with S = 4 slices these serve
 // four slices, and a slice adds four products and a quarter of four 16-byte
-// reads.  16 x 512^2, 180 angles: 643 us with one slice per workgroup, 361 with
+// reads.  16 x 512^2, 180 angles: 624 us with one slice per workgroup, 371 with
 // four.  A single slice keeps larger tiles (fewer samples lost at tile
 // edges: 79% of a pass are inside, 65% at the four-slice size); both fit LDS
 // twice per CU, so that one workgroup stages while the other sums.
@@ -331,7 +331,7 @@ constexpr int kFiltPitch = kFiltKC + 2;
 // Bound by the matrix cores at two to four workgroups per CU (27 KB of LDS,
 // five fit): 192 columns a workgroup, so that 2,880 rows of 725 bins give 720
 // workgroups for 256 CUs.  256 columns, five LDS reads for four MFMAs and a
-// division per staged value: 59 us; now 37 (20 at the FP32 matrix rate);
+// division per staged value: 58 us; now 36 (20 at the FP32 matrix rate);
 // 3,840 rows 61 -> 48 us.
 __global__ __launch_bounds__(256) void k_fbp_filter_mfma(const float* __restrict__ sino, float* __restrict__ filt,
                                                          const float* __restrict__ taps, int ndet, int rows) {
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256) void k_fbp_backproject(const float* __restrict
 // Angles go in chunks of CH, a wave staging every fourth angle; with kAhead
 // the next chunk's windows are loaded into registers meanwhile.  Bound by LDS
 // latency and VALU issue at four waves per SIMD.  16 slices of 512^2, 180
-// angles: 199 -> 114 us; 64 slices, 60 angles: 279 -> 148 us.
+// angles: 192 -> 109 us; 64 slices, 60 angles: 279 -> 147 us.
 template <int PX>
 struct BpCfg {
     // >= 2 (half diagonal + 2): 15.5 and 4 PX - 0.5 pixels from the centre

@@ -270,7 +270,7 @@ __device__ void lds_fft(double* re, double* im, int N, const double2* __restrict
 // places, into registers (16 values a thread at most: H2 <= 4096), and writes
 // it in order for the second transform; the result is read bit-reversed too.
 // Bound by LDS passes and their barriers (two radix-2 stages a pass, no
-// permutation passes: 2,880 sectors of 512^2 slices 69 -> FFTIME us).
+// permutation passes: 2,880 sectors of 512^2 slices 68 -> 36 us).
 template <bool kPad>
 __global__ __launch_bounds__(256) void k_radn_filter(const SecDesc* __restrict__ secs, const double* __restrict__ P,
                                                      float* __restrict__ q, const double2* __restrict__ tw,
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void k_lrt_rowsum(const SecDesc* __restrict__ 
 // peak rule and leaves the search for the first rise at once; otherwise 97% of
 // cells stop at m <= 9.
 // Bound by FP64 VALU issue: 64 columns x 32 rows a workgroup, a wave per row
-// at a time, five window-sum reads of 8 B per cell from memory and 64 from LDS
+// at a time, three window-sum reads of 8 B per cell from memory and 64 from LDS
 // (conflict-free).  512^2, 180 sectors: 5.28 -> 1.42 ms.
 constexpr int kLrtRows = 32, kLrtWin = kLrtRows + 63;
 __global__ __launch_bounds__(512) void k_op_lrt(const SecDesc* __restrict__ secs, int nsec, int coltiles,
