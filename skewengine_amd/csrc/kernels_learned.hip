@@ -1039,7 +1039,7 @@ __global__ __launch_bounds__(256) void k_conv_mid_bwd_mfma(const float* __restri
 // rate of a copy) now that loads are 16 bytes wide, two pixels of a few
 // channels a thread, in flight during the previous tile's products, with
 // offsets made once, and the workgroups are as many as stay resident (2,048
-// with loads of one channel took two rounds): 220 -> 105 us.
+// with loads of one channel took two rounds): 220 -> 96 us.
 
 // The next tile's share of a thread, in registers.
 template <int C>
