@@ -178,9 +178,8 @@ int ske_synchronize(ske_engine *e);
 
 /* Options (no reference counterpart). */
 #define SKE_OPT_SDEM_VARIANT 1  /* viewshed inner loop: 0 bit-block (default), 1 IEEE divide per step, 2 exact fma division
-                                   per step.  All three give identical results for heights (and povh)
-                                   of at most 1e30 in magnitude; with others, or ones that are not
-                                   finite, 0 gives what 2 gives in every launch shape and call. */
+                                   per step.  All three give identical results, also with heights or
+                                   a povh that are not finite. */
 #define SKE_OPT_ARENA_BYTES 2   /* device budget for one chunk of skewOutput rows */
 #define SKE_OPT_PROFILE 3       /* 1: time every launch with HIP events on the engine stream */
 #define SKE_OPT_GRAPH 4         /* 1: capture the all-sector run once in a hipGraph and replay it */

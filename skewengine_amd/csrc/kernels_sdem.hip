@@ -37,12 +37,14 @@ __device__ __forceinline__ void sdem_step(float sk, float h, const float4 t, flo
                                           float& cv) {
     const float a = sk - h;
     float q;
-    if (kVariant == 0)
+    if (kVariant == 0) {
         q = __builtin_fmaf(a, t.x, a * t.y);
-    else
+        q = __builtin_isinf(a) ? a : q;  // the products would give inf * 0
+    } else {
         q = a / t.z;
+    }
     const bool above = q > M;
-    M = above ? q : M;  // std::max(cAngle, max_angle)
+    M = q < M ? M : q;  // std::max(cAngle, max_angle): a quotient that is no number stays
     const bool opening = above && !vis;
     const bool closing = !above && vis;
     vis = above;
@@ -727,7 +729,8 @@ __device__ __forceinline__ void sdem_bits_row(const RowWork w, const SecDesc* __
         // The bit of a step is the sign of M - q, which is not q > M once a
         // difference is infinite or no number.  Heights in [-FLT_MAX, 1e30]
         // keep every one finite (1e30 is below half an ulp of FLT_MAX); a row
-        // with any other takes the per-step scans.
+        // with any other takes the per-step scans, which compare as the
+        // reference does.
         for (int c = threadIdx.x >> 6; c < nchunk; c += kWaves)
             sdem_steps_chunk<0>(row, L, c, povh, rtab, so, sd.R);
         __syncthreads();

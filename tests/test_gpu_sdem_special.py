@@ -1,10 +1,13 @@
 """Viewshed of grids with heights (or an observer height) that are not finite or
 are huge, through every launch shape of the bit-block kernels and call by call:
 the sign of a difference is not its comparison there, so such rows take the
-per-step scans and equal OPT_SDEM_VARIANT = 2 bit for bit."""
+per-step scans and equal OPT_SDEM_VARIANT = 2, and with it the one-thread oracle
+(quotients of infinite differences, the running maximum with a quotient that is
+no number), bit for bit."""
 import numpy as np
 import pytest
 
+import oracle
 import skewengine_amd as ske
 from skewengine_amd import _lib, synth
 
@@ -61,3 +64,24 @@ def test_launch_shapes_equal_the_per_step_scans(value, povh, shape):
 def test_calls_equal_the_per_step_scans(value, povh):
     g = _grid(value, 60)
     assert np.array_equal(_by_calls(g, povh, 0), _by_calls(g, povh, 2), equal_nan=True)
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2])
+@pytest.mark.parametrize("value,povh", CASES)
+def test_variants_equal_the_oracle(value, povh, variant):
+    g = _grid(value)
+    with ske.SkewEngine(g) as e:
+        e.set_option(_lib.OPT_SDEM_VARIANT, variant)
+        out = e.run(ske.KERNEL_SDEM, povh=povh)
+    assert np.array_equal(out, oracle.execute(oracle.SDEM, g, nthreads=1, povh=povh)[0], equal_nan=True)
+
+
+@pytest.mark.parametrize("value,povh", CASES)
+def test_scratch_array_equals_the_oracle(value, povh):
+    torch = pytest.importorskip("torch")
+    g = _grid(value)
+    d_in, d_out = torch.from_numpy(g).cuda(), torch.empty(g.shape, device="cuda")
+    torch.cuda.synchronize()
+    _lib.check(_lib.lib().ske_execute_noalloc(ske.KERNEL_SDEM, g.shape[0], d_in.data_ptr(), d_out.data_ptr(), povh, 0,
+                                              180, 0, None))
+    assert np.array_equal(d_out.cpu().numpy(), oracle.execute(oracle.SDEM, g, nthreads=1, povh=povh)[0], equal_nan=True)
